@@ -53,29 +53,53 @@ __device__ __forceinline__ void tm_dma16_buf(tm_rsrc_t rsrc, uint32_t voff, uint
 // tm_dma16_buf with a scalar byte offset added to every lane's (soff: one
 // SGPR, so a loop can step through a matrix's K dimension without touching
 // the per-lane offsets) and the LDS base already in an SGPR.
+// ONCE: for data that is read once, a non-temporal load (the L2 does not keep
+// it in front of lines that are read again).
+template <bool ONCE = false>
 __device__ __forceinline__ void tm_dma16_buf_so(tm_rsrc_t rsrc, uint32_t voff, uint32_t soff, uint32_t lds_base) {
   uint32_t saved;
-  asm volatile(
-      "s_mov_b32 %0, m0\n\t"
-      "s_mov_b32 m0, %4\n\t"
-      "buffer_load_dwordx4 %1, %2, %3 offen lds\n\t"
-      "s_mov_b32 m0, %0"
-      : "=&s"(saved)
-      : "v"(voff), "s"(rsrc), "s"(soff), "s"(lds_base)
-      : "memory");
+  if constexpr (ONCE)
+    asm volatile(
+        "s_mov_b32 %0, m0\n\t"
+        "s_mov_b32 m0, %4\n\t"
+        "buffer_load_dwordx4 %1, %2, %3 offen nt lds\n\t"
+        "s_mov_b32 m0, %0"
+        : "=&s"(saved)
+        : "v"(voff), "s"(rsrc), "s"(soff), "s"(lds_base)
+        : "memory");
+  else
+    asm volatile(
+        "s_mov_b32 %0, m0\n\t"
+        "s_mov_b32 m0, %4\n\t"
+        "buffer_load_dwordx4 %1, %2, %3 offen lds\n\t"
+        "s_mov_b32 m0, %0"
+        : "=&s"(saved)
+        : "v"(voff), "s"(rsrc), "s"(soff), "s"(lds_base)
+        : "memory");
 }
 
 // tm_dma16 with the LDS base already in an SGPR (no readfirstlane).
+template <bool ONCE = false>
 __device__ __forceinline__ void tm_dma16_s(const void *gaddr, uint32_t lds_base) {
   uint32_t saved;
-  asm volatile(
-      "s_mov_b32 %0, m0\n\t"
-      "s_mov_b32 m0, %2\n\t"
-      "global_load_lds_dwordx4 %1, off\n\t"
-      "s_mov_b32 m0, %0"
-      : "=&s"(saved)
-      : "v"(gaddr), "s"(lds_base)
-      : "memory");
+  if constexpr (ONCE)
+    asm volatile(
+        "s_mov_b32 %0, m0\n\t"
+        "s_mov_b32 m0, %2\n\t"
+        "global_load_lds_dwordx4 %1, off nt\n\t"
+        "s_mov_b32 m0, %0"
+        : "=&s"(saved)
+        : "v"(gaddr), "s"(lds_base)
+        : "memory");
+  else
+    asm volatile(
+        "s_mov_b32 %0, m0\n\t"
+        "s_mov_b32 m0, %2\n\t"
+        "global_load_lds_dwordx4 %1, off\n\t"
+        "s_mov_b32 m0, %0"
+        : "=&s"(saved)
+        : "v"(gaddr), "s"(lds_base)
+        : "memory");
 }
 
 template <int N>
@@ -83,4 +107,12 @@ __device__ __forceinline__ void tm_wait_vm_lgkm0() {
   // s_waitcnt vmcnt(N) lgkmcnt(0), expcnt left at its maximum
   static_assert(N >= 0 && N < 64, "vmcnt range");
   __builtin_amdgcn_s_waitcnt((N & 0xF) | ((N >> 4) << 14) | (0x7 << 4));
+}
+
+// The same wait as an asm block with a memory clobber: LDS reads written
+// after it stay after it (the builtin alone does not order them).
+template <int N>
+__device__ __forceinline__ void tm_wait_vm_lgkm0_mem() {
+  static_assert(N >= 0 && N < 64, "vmcnt range");
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(N) : "memory");
 }

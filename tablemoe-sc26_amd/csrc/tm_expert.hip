@@ -17,15 +17,13 @@
 // of LDS atomics; every output row is computed the same way wherever its row
 // sits in a tile, so results do not depend on it.
 //
-// grouped_gemm_kernel computes one BM x BN tile C = A B^T of one expert:
-// A rows gathered (token rows of x, or the grouped rows of the intermediate),
-// B rows k-contiguous (nn.Linear weights [out, in]), K in BK-wide stages
-// moved global -> LDS by direct loads (16-byte chunks XOR-swizzled by row, so
-// the operand reads of 32 rows spread over the banks), three in flight.
-// Four waves, one per SIMD, each software-pipelined so that the operand reads
-// of one k-step run under the MFMAs of the previous one.  Up mode multiplies
-// W1 and W3 against the same A fragments and applies the SiLU-mul epilogue;
-// down mode writes each row to its slot of the output.
+// The two GEMMs of a tile run in one of two kernels, with the same bits:
+// skinny_gemm_kernel (few rows: one wave per column group, bound by the stream
+// of weights) and tile_gemm_kernel (eight waves per 256-row tile).  Both move K
+// in BK-wide stages global -> LDS by direct loads (16-byte chunks XOR-swizzled
+// by row, so the operand reads of 32 rows spread over the banks).  The up GEMM
+// multiplies W1 and W3 against the same activation operands and applies the
+// SiLU-mul; the down GEMM writes each row to its slot of the output.
 //
 // Packed path (tm_expert_pack_weights, tm_grouped_swiglu_packed,
 // tm_expert_swiglu_packed): each weight tile is stored stage by stage in the
@@ -42,12 +40,6 @@ namespace {
 constexpr int BM = 256, BK = 32, kThreads = 256;
 constexpr int kMinBN = 128;                  // column tile of the up GEMM (and of narrow down GEMMs)
 constexpr int kCPR = BK / 8;                 // 16-byte chunks per tile row and stage
-constexpr int kAStage = BM * kCPR;           // A slots (16 bytes) per stage
-constexpr int kADma = kAStage / kThreads;    // A loads per thread per stage (4)
-constexpr int kMI = 4;                       // 32-row blocks per wave: 128 rows
-constexpr int kStageCols = 128;              // epilogue staging width (columns per pass)
-constexpr int kStageLd = kStageCols + 8;     // staging row stride in floats
-constexpr int kEpiFloats = BM * kStageLd;    // staging tile size in floats (139,264 bytes)
 
 enum { kModeUp = 0, kModeDown = 1 };
 
@@ -67,56 +59,148 @@ struct TileSrc {
   int32_t rows;
 };
 
-// One BM x BN tile C = A B^T of one expert (NB = 2: two B matrices against
-// the same A, the gate and up projections).  Four waves in a 2 x 2 grid of
-// 128 x BN/2 quadrants, one wave per SIMD, 16 accumulator blocks of
-// v_mfma_f32_32x32x16 per wave (all 256 AGPRs): 4 x 2 per B for the up GEMM
-// (BN = 128), 4 x 4 for the down GEMM (BN = 256), so every k-step reads 8
-// operand fragments from LDS for 16 MFMAs (a hidden size that is not a
-// multiple of 256 takes 128-column down tiles: 6 reads, 8 MFMAs).
+// Few rows per expert (a decode batch, a short prompt, one token through one
+// expert): the MLP is a stream of the experts' weights, and 256-row tiles put
+// it on few workgroups (6 for one expert of 768 intermediate columns) that
+// each wait for a stage at every barrier.  Here one wave is a workgroup: it
+// owns CW output columns of one expert's tile and streams their weight rows
+// and up to RBMAX activation rows through an LDS ring of its own (direct
+// global -> LDS loads, no barrier anywhere), LDS bytes deep, so a CU's waves
+// keep it filled and even a single expert spreads over one wave per CW
+// columns.  16 KiB rings (10 waves per CU) measured 30 + 17 us (up + down) on
+// a decode batch of 28 experts, 40 KiB ones 36 + 20 (the last round of waves
+// is then less even).  Where waves are few, stages of two sub-stages halve the
+// LDS round trips per column (one expert, one row: up 8.5 -> 6.9 us).
 //
-// K moves in BK-wide stages through a 4-slot LDS ring filled by direct
-// global -> LDS loads (A rows gathered by 64-bit per-lane addresses, B rows
-// through a buffer resource whose scalar offset walks K), three stages in
-// flight.  Each wave is software-pipelined over half-stages (k-steps): while
-// the matrix core runs the 16 MFMAs of one k-step, the wave reads the next
-// k-step's 8 fragments into the other register set (sched_group_barrier
-// interleaves one read per two MFMAs).  The stage boundary sits between a
-// stage's two k-steps: wait for this wave's loads of the next stage, barrier
-// (every wave's loads of it are then visible and every wave has finished its
-// reads of the current stage's slot), and refill that slot with the stage
-// four ahead.  Stages past the last re-read the last one (never multiplied),
-// so the wait counts are the same in every iteration.
-template <int DT, int NB, int MODE, int BN, bool PB>
-__global__ __launch_bounds__(kThreads, 1) void grouped_gemm_kernel(
+// A = weight rows (up: the gate and up rows of the same columns, so a lane
+// ends with both and the SiLU-mul needs no exchange), B = the activation rows.
+// Each result is the same chain of 32x32x16 products over K as in the tile
+// kernel, so the rows are the same bit for bit, whichever kernel runs a tile.
+//
+// Bound by HBM: at 2 rows per expert (128 experts, hidden 2048, inter 768) the
+// up GEMM streams its 0.8 GB at 6.9 TB/s.  us per call before (256-row tiles
+// of 4 waves) -> now: one expert and one row 56 -> 11 (device), 32 slots of 28
+// experts 74 -> 47, 256 slots of 110 experts 233 -> 138.
+//
+// A ring stage is SUB sub-stages of BK columns.
+template <int MODE_, int CW_, int SUB_, int LDS_, int RBMAX_>
+struct SkinnyCfg {
+  static constexpr int MODE = MODE_, CW = CW_, SUB = SUB_, LDS = LDS_, RBMAX = RBMAX_;
+  static constexpr int kWRows = MODE == kModeUp ? 2 * CW : CW;  // weight rows per stage
+  static constexpr int kWDma = kWRows / 16;                     // loads of 16 rows x 64 bytes
+  static constexpr int kNA = kWRows > 32 ? kWRows / 32 : 1;     // 32-row A operands (16 rows: read twice)
+};
+
+template <class Cfg, int RB>
+struct SkinnyShape {
+  static constexpr int kXDma = RB / 16;
+  static constexpr int kNB = RB > 32 ? RB / 32 : 1;
+  static constexpr int kDma = Cfg::SUB * (Cfg::kWDma + kXDma);
+  static constexpr int kSubBytes = (Cfg::kWDma + kXDma) * 1024;
+  static constexpr int kStageBytes = Cfg::SUB * kSubBytes;
+  static constexpr int kFit = Cfg::LDS / kStageBytes;
+  static constexpr int kDeep = (kFit * kDma < 62 ? kFit : 62 / kDma) & ~1;  // stages in flight (even; vmcnt holds 63)
+  static constexpr int kShallow = Cfg::SUB == 1 && kDeep >= 4 ? 4 : 2;      // for K of 128 columns
+};
+
+template <int DT, class Cfg, int RB, int D, bool ONCE>
+__device__ __forceinline__ void skinny_block(const typename Elem<DT>::T *const (&w_src)[4], int64_t w_step,
+                                             const typename Elem<DT>::T *const (&x_src)[4], int64_t x_step, int KT,
+                                             const uint32_t (&a_off)[2], uint32_t lds0, const char *lds,
+                                             tm_f32x16 (&acc)[Cfg::kNA][Cfg::RBMAX > 32 ? Cfg::RBMAX / 32 : 1]) {
+  using S = SkinnyShape<Cfg, RB>;
+  constexpr int SUB = Cfg::SUB, NA = Cfg::kNA, NB = S::kNB, kWDma = Cfg::kWDma;
+  static_assert(D >= 2 && D % 2 == 0 && D * S::kStageBytes <= Cfg::LDS && D * S::kDma < 63, "ring shape");
+  const int lane = threadIdx.x & 63;
+  const int tr = lane & (RB < 32 ? RB - 1 : 31);
+  uint32_t b_off[2];
+#pragma unroll
+  for (int ks = 0; ks < 2; ++ks)
+    b_off[ks] = (uint32_t)(kWDma * 1024 + tr * 64 + swz_chunk(tr, 2 * ks + (lane >> 5)) * 16);
+  auto issue = [&](int st, uint32_t slot) {
+    tm_static_for<SUB>([&](auto u_c) {
+      constexpr int u = decltype(u_c)::value;
+      const int64_t kt = (int64_t)st * SUB + u;
+      const uint32_t dst = lds0 + slot + u * S::kSubBytes;
+      tm_static_for<kWDma>([&](auto j_c) {
+        constexpr int j = decltype(j_c)::value;
+        tm_dma16_s<ONCE>(w_src[j] + kt * w_step, dst + j * 1024);
+      });
+      tm_static_for<S::kXDma>([&](auto j_c) {
+        constexpr int j = decltype(j_c)::value;
+        tm_dma16_s(x_src[j] + kt * x_step, dst + (kWDma + j) * 1024);
+      });
+    });
+  };
+  uint4 fa[2][2 * SUB][NA], fb[2][2 * SUB][NB];  // [stage parity][k-step]
+  auto read = [&](auto p_c, uint32_t slot) {
+    constexpr int p = decltype(p_c)::value;
+#pragma unroll
+    for (int ks = 0; ks < 2 * SUB; ++ks) {
+      const char *const sub = lds + slot + (ks >> 1) * S::kSubBytes;
+#pragma unroll
+      for (int a = 0; a < NA; ++a) fa[p][ks][a] = *reinterpret_cast<const uint4 *>(sub + a_off[ks & 1] + a * 2048);
+#pragma unroll
+      for (int b = 0; b < NB; ++b) fb[p][ks][b] = *reinterpret_cast<const uint4 *>(sub + b_off[ks & 1] + b * 2048);
+    }
+  };
+  auto mul = [&](auto p_c) {
+    constexpr int p = decltype(p_c)::value;
+#pragma unroll
+    for (int ks = 0; ks < 2 * SUB; ++ks)
+#pragma unroll
+      for (int a = 0; a < NA; ++a)
+#pragma unroll
+        for (int b = 0; b < NB; ++b) acc[a][b] = tm_mfma32x32x16<DT>(fa[p][ks][a], fb[p][ks][b], acc[a][b]);
+  };
+  constexpr uint32_t kRing = (uint32_t)(D * S::kStageBytes);
+  for (int i = 0; i < D; ++i) issue(i, (uint32_t)(i * S::kStageBytes));
+  tm_wait_vm_lgkm0_mem<(D - 1) * S::kDma>();
+  uint32_t slot = 0;
+  read(std::integral_constant<int, 0>{}, slot);
+  // stage i is in registers (parity p) or on its way there; its slot takes
+  // stage i + D, then stage i + 1 is read while stage i is multiplied
+  auto step = [&](auto p_c, int i) {
+    constexpr int p = decltype(p_c)::value;
+    tm_wait_vm_lgkm0_mem<63>();  // stage i is read: its slot is free
+    issue(i + D, slot);
+    slot = slot + S::kStageBytes == kRing ? 0u : slot + S::kStageBytes;
+    tm_wait_vm_lgkm0_mem<(D - 1) * S::kDma>();  // stage i + 1 landed
+    read(std::integral_constant<int, 1 - p>{}, slot);
+    mul(p_c);
+  };
+  for (int i = 0; i < KT / SUB - D; i += 2) {  // KT is a multiple of 4; KT / SUB and D are even
+    step(std::integral_constant<int, 0>{}, i);
+    step(std::integral_constant<int, 1>{}, i + 1);
+  }
+  tm_static_for<D>([&](auto t_c) {
+    constexpr int t = decltype(t_c)::value;
+    if constexpr (t < D - 1) {
+      slot = slot + S::kStageBytes == kRing ? 0u : slot + S::kStageBytes;
+      tm_wait_vm_lgkm0_mem<(D - 2 - t) * S::kDma>();
+      read(std::integral_constant<int, (t + 1) & 1>{}, slot);
+    }
+    mul(std::integral_constant<int, t & 1>{});
+  });
+  tm_wait_vm_lgkm0_mem<0>();  // every read is done before the next block's loads
+}
+
+// split > 0 (dense rows): a workgroup takes one RBMAX-row block of a tile
+// (split blocks per tile); split == 0: all of the tile's, one after the other.
+// ONCE: no other workgroup reads these weights (grouped rows), so they are
+// loaded non-temporally and leave the L2 to the activation rows.
+template <int DT, class Cfg, bool PB, bool ONCE>
+__global__ __launch_bounds__(64) void skinny_gemm_kernel(
     const typename Elem<DT>::T *__restrict__ A, int64_t lda, const int32_t *__restrict__ a_rows,
     const typename Elem<DT>::T *__restrict__ B0, const typename Elem<DT>::T *__restrict__ B1, int64_t b_expert,
-    int K, int n_tiles, TileSrc ts, typename Elem<DT>::T *__restrict__ C, int64_t ldc,
+    int K, int n_groups, int pack_bn, int split, TileSrc ts, typename Elem<DT>::T *__restrict__ C, int64_t ldc,
     const int64_t *__restrict__ c_rows, const typename Elem<DT>::T *__restrict__ addend, int64_t ld_add) {
   using T = typename Elem<DT>::T;
-  constexpr int kNI = BN / 64;                   // 32-column blocks per wave and B
-  constexpr int kBStage = BN * kCPR;             // slots of each B per stage
-  constexpr int kBDma = kBStage / kThreads;      // loads of each B per thread per stage
-  constexpr int kStage = kAStage + NB * kBStage;
-  constexpr int kDma = kADma + NB * kBDma;       // loads per wave per stage
-  constexpr int kFrag = kMI + NB * kNI;          // operand fragments per k-step
-  constexpr int kMfma = NB * kMI * kNI;          // MFMAs per k-step (16; 8 for a 128-column down GEMM)
-  static_assert(kMfma <= 16, "accumulators fit the AGPRs");
-  static_assert(kBStage % kThreads == 0 && 3 * kDma < 64, "stage shape");
-  // One LDS array: the 4-slot ring during the K loop, then the fp32 staging
-  // tile of the epilogue (kStageCols columns, rows padded to kStageLd floats).
-  constexpr int kLdsSlots = 4 * kStage > kEpiFloats / 4 ? 4 * kStage : kEpiFloats / 4;
-  __shared__ uint4 lds_all[kLdsSlots];
-  uint4 *const ring0 = lds_all, *const ring1 = lds_all + kStage, *const ring2 = lds_all + 2 * kStage,
-               *const ring3 = lds_all + 3 * kStage;
-
-  // Block b runs on XCD b % 8 (the dispatcher's round robin): the n_tiles
-  // column tiles of row tile y get ids 8 apart, so they share one XCD and its
-  // L2 copy of the tile's A rows.
-  const int64_t b = blockIdx.x;
-  const int64_t slot = b >> 3;
-  const int64_t y = (slot / n_tiles) * 8 + (b & 7);
-  const int n0 = (int)(slot % n_tiles) * BN;
+  constexpr int MODE = Cfg::MODE, CW = Cfg::CW, SUB = Cfg::SUB;
+  __shared__ uint4 ring[Cfg::LDS / 16];
+  const int64_t blk = blockIdx.x / n_groups;
+  const int64_t y = split > 0 ? blk / split : blk;
+  const int n0 = (int)(blockIdx.x % n_groups) * CW;
   int e, r0, r_end;
   if (ts.tiles != nullptr) {
     if (y >= ts.t_max || y >= ts.tiles[1]) return;  // uniform: past the last tile
@@ -129,198 +213,412 @@ __global__ __launch_bounds__(kThreads, 1) void grouped_gemm_kernel(
     if (r0 >= ts.rows) return;
     r_end = ts.rows;
   }
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wm = wave >> 1, wn = wave & 1;
+  r_end = r_end < r0 + BM ? r_end : r0 + BM;  // this tile's rows
+  const int rb0 = split > 0 ? (int)(blk % split) * Cfg::RBMAX : 0;
+  const int rb1 = split > 0 && rb0 + Cfg::RBMAX < r_end - r0 ? rb0 + Cfg::RBMAX : r_end - r0;
+  const int lane = threadIdx.x & 63;
+  const int KT = K / BK;
+  const uint32_t lds0 = (uint32_t)(uintptr_t)ring;
+  const char *const lds = reinterpret_cast<const char *>(ring);
 
-  // Loads: thread t fills slots t + 256 j of the A part and of each B part;
-  // slot p holds row p / kCPR, chunk swz_chunk(row, p % kCPR) (the swizzle is
-  // its own inverse).  A: 64-bit address of stage 0 (stage s adds s * BK).
-  // The packed down GEMM reads the intermediate tile y as the up GEMM wrote
-  // it, stage by stage in slot order: stage s of the tile is the contiguous
-  // block s * BM * BK (rows past the expert hold whatever was there; their
-  // results are dropped).
+  // Weight loads: lane l fills 16-byte slot l % 4 of LDS row 16 j + l / 4;
+  // row r holds chunk swz_chunk(r in its 128- or 256-row tile, slot), the
+  // order of the packed layout, so the packed loads are contiguous.
+  const T *w_src[4] = {nullptr, nullptr, nullptr, nullptr};
+  const int64_t w_step = PB ? (int64_t)pack_bn * BK : BK;
+  auto w_addr = [&](const T *B, int col) {  // column `col` (a weight row), slot lane % 4
+    const T *we = B + (int64_t)e * b_expert;
+    if constexpr (PB)
+      return we + (int64_t)(col / pack_bn) * pack_bn * K + (col % pack_bn) * BK + (lane & 3) * 8;
+    else
+      return we + (int64_t)col * K + swz_chunk(col, lane & 3) * 8;
+  };
+  const int lr = lane >> 2;
+  uint32_t a_off[2];
+  const int ar = lane & 31;  // operand row of this lane
+  int a_lds, a_col;          // its LDS row and weight row (for the swizzle)
+  if constexpr (MODE == kModeUp && CW == 32) {  // operands: 32 gate rows, 32 up rows
+    w_src[0] = w_addr(B0, n0 + lr);
+    w_src[1] = w_addr(B0, n0 + 16 + lr);
+    w_src[2] = w_addr(B1, n0 + lr);
+    w_src[3] = w_addr(B1, n0 + 16 + lr);
+    a_lds = ar;
+    a_col = n0 + ar;
+  } else if constexpr (MODE == kModeUp && CW == 16) {  // one operand: 16 gate rows, 16 up rows
+    w_src[0] = w_addr(B0, n0 + lr);
+    w_src[1] = w_addr(B1, n0 + lr);
+    a_lds = ar;
+    a_col = n0 + (ar & 15);
+  } else if constexpr (MODE == kModeUp) {  // CW == 8: gate rows 0-7, up rows 8-15 of one load, read twice
+    static_assert(CW == 8, "column counts");
+    w_src[0] = w_addr(lr < 8 ? B0 : B1, n0 + (lr & 7));
+    a_lds = ar & 15;
+    a_col = n0 + (ar & 7);
+  } else {
+#pragma unroll
+    for (int j = 0; j < Cfg::kWDma; ++j) w_src[j] = w_addr(B0, n0 + 16 * j + lr);
+    a_lds = CW < 32 ? ar & (CW - 1) : ar;
+    a_col = n0 + a_lds;
+  }
+#pragma unroll
+  for (int ks = 0; ks < 2; ++ks)
+    a_off[ks] = (uint32_t)(a_lds * 64 + swz_chunk(a_col, 2 * ks + (lane >> 5)) * 16);
+
   constexpr bool kTiledA = PB && MODE == kModeDown;
-  constexpr int64_t kAStep = kTiledA ? BM * BK : BK;  // elements from one stage to the next
-  const T *a_src[kADma];
+  constexpr int kNBMax = Cfg::RBMAX > 32 ? Cfg::RBMAX / 32 : 1;
+  const int64_t x_step = kTiledA ? (int64_t)BM * BK : BK;
+  for (int rb = rb0; rb < rb1; rb += Cfg::RBMAX) {
+    const int rows = rb1 - rb;
+    const T *x_src[4] = {};
 #pragma unroll
-  for (int j = 0; j < kADma; ++j) {
-    const int p = tid + kThreads * j;
-    const int row = p / kCPR, kc = swz_chunk(row, p % kCPR);
-    if constexpr (kTiledA) {
-      a_src[j] = A + y * (int64_t)BM * lda + (int64_t)p * 8;
-    } else {
-      int gr = r0 + row;
-      gr = gr < r_end ? gr : r_end - 1;  // rows past the expert re-read its last row; their results are dropped
-      const int64_t ar = a_rows ? (int64_t)a_rows[gr] : (int64_t)gr;
-      a_src[j] = A + ar * lda + kc * 8;
+    for (int j = 0; j < Cfg::RBMAX / 16; ++j) {
+      const int tr = 16 * j + lr;
+      if constexpr (kTiledA) {
+        x_src[j] = A + y * (int64_t)BM * lda + (int64_t)(rb + tr) * BK + (lane & 3) * 8;
+      } else {
+        int gr = r0 + rb + tr;
+        gr = gr < r_end ? gr : r_end - 1;  // rows past the expert re-read its last row; their results are dropped
+        const int64_t xr = a_rows ? (int64_t)a_rows[gr] : (int64_t)gr;
+        x_src[j] = A + xr * lda + swz_chunk(tr, lane & 3) * 8;
+      }
     }
-  }
-  // B: the expert's BN rows from n0 on, through a buffer; lane offsets fixed,
-  // the stage's K offset in the scalar offset.  Packed weights (PB) hold each
-  // stage of the tile as one contiguous block in slot order, so slot p is at
-  // byte 16 p of the stage's block.
-  tm_rsrc_t b_rs[NB];
-  b_rs[0] = tm_make_rsrc(B0 + (int64_t)e * b_expert + (int64_t)n0 * K, (uint64_t)BN * K * sizeof(T));
-  if constexpr (NB > 1) b_rs[1] = tm_make_rsrc(B1 + (int64_t)e * b_expert + (int64_t)n0 * K, (uint64_t)BN * K * sizeof(T));
-  uint32_t b_off[kBDma];
+    tm_f32x16 acc[Cfg::kNA][kNBMax];
 #pragma unroll
-  for (int j = 0; j < kBDma; ++j) {
-    const int p = tid + kThreads * j;
-    const int row = p / kCPR, kc = swz_chunk(row, p % kCPR);
-    b_off[j] = PB ? (uint32_t)p * 16u : (uint32_t)row * (uint32_t)K * (uint32_t)sizeof(T) + (uint32_t)kc * 16u;
-  }
-  const int KT = K / BK;  // a multiple of 4 (the host checks)
-  // Load j (0 .. kDma-1) of stage `stage` into `ring`: A loads first, then
-  // each B's.  Stages past the last re-read the last one.
-  auto issue_one = [&](auto j_c, uint4 *ring, int stage) {
-    constexpr int j = decltype(j_c)::value;
-    const int kt = stage < KT ? stage : KT - 1;
-    const uint32_t lds = (uint32_t)(uintptr_t)ring + (uint32_t)wave * 1024u;  // wave's 64 slots of load 0
-    if constexpr (j < kADma) {
-      tm_dma16_s(a_src[j] + (int64_t)kt * kAStep, lds + (uint32_t)(j * kThreads * 16));
-    } else {
-      constexpr int bb = (j - kADma) / kBDma, jb = (j - kADma) % kBDma;
-      tm_dma16_buf_so(b_rs[bb], b_off[jb], (uint32_t)kt * (uint32_t)(PB ? kBStage * 16 : BK * sizeof(T)),
-                      lds + (uint32_t)((kAStage + bb * kBStage + jb * kThreads) * 16));
-    }
-  };
-  auto issue = [&](uint4 *ring, int stage) { tm_static_for<kDma>([&](auto j_c) { issue_one(j_c, ring, stage); }); };
-
-  // Fragment byte offsets within a slot: row R + (lane % 32) (R a multiple of
-  // 32) at chunk 2 ks + lane / 32 sits at R * 64 + off[ks], the same for every
-  // block, part and slot; opaque, so the rest stays an immediate offset.
-  uint32_t f_off[2];
+    for (int a = 0; a < Cfg::kNA; ++a)
 #pragma unroll
-  for (int ks = 0; ks < 2; ++ks) {
-    const int r = lane & 31;
-    f_off[ks] = (uint32_t)(r * kCPR + swz_chunk(r, 2 * ks + (lane >> 5))) * 16u;
-    asm volatile("" : "+v"(f_off[ks]));
-  }
-  uint4 fr[2][kFrag];  // two k-steps' operands: [0..kMI) A blocks, then B blocks
-  auto read_one = [&](auto g_c, uint4 (&f)[kFrag], const uint4 *ring, int ks) {
-    constexpr int g = decltype(g_c)::value;
-    const char *base = reinterpret_cast<const char *>(ring) + f_off[ks];
-    if constexpr (g < kMI) {
-      f[g] = *reinterpret_cast<const uint4 *>(base + (wm * 128 + g * 32) * 64);
-    } else {
-      constexpr int bb = (g - kMI) / kNI, ni = (g - kMI) % kNI;
-      f[g] = *reinterpret_cast<const uint4 *>(base + (kAStage + bb * kBStage) * 16 + (wn * (BN / 2) + ni * 32) * 64);
-    }
-  };
-
-  tm_f32x16 acc[NB][kMI][kNI];
+      for (int b = 0; b < kNBMax; ++b) acc[a][b] = tm_f32x16{};
+    auto run = [&](auto rb_c) {
+      constexpr int RB = decltype(rb_c)::value;
+      using S = SkinnyShape<Cfg, RB>;
+      if (KT / SUB >= S::kDeep)
+        skinny_block<DT, Cfg, RB, S::kDeep, ONCE>(w_src, w_step, x_src, x_step, KT, a_off, lds0, lds, acc);
+      else
+        skinny_block<DT, Cfg, RB, S::kShallow, ONCE>(w_src, w_step, x_src, x_step, KT, a_off, lds0, lds, acc);
+    };
+    if (rows <= 16) run(std::integral_constant<int, 16>{});
+    else if (Cfg::RBMAX == 32 || rows <= 32) run(std::integral_constant<int, 32>{});
+    else run(std::integral_constant<int, Cfg::RBMAX>{});
+    // lane: activation row lane % 32 of each B operand, weight rows 8 (i / 4)
+    // + 4 (lane / 32) + i % 4 of each A operand: runs of 4 consecutive columns
 #pragma unroll
-  for (int bb = 0; bb < NB; ++bb)
+    for (int b = 0; b < kNBMax; ++b) {
+      const int tr = 32 * b + (lane & 31);
+      if (tr < rows && (rows > 16 || tr < 16)) {
+        const int gr = r0 + rb + tr;
 #pragma unroll
-    for (int mi = 0; mi < kMI; ++mi)
+        for (int u = 0; u < CW / 8; ++u) {
+          const int col = n0 + 8 * u + 4 * (lane >> 5);
+          float v[4];
 #pragma unroll
-      for (int ni = 0; ni < kNI; ++ni) acc[bb][mi][ni] = tm_f32x16{};
-  auto mfma_one = [&](auto m_c, const uint4 (&f)[kFrag]) {
-    constexpr int m = decltype(m_c)::value;
-    constexpr int bb = m / (kMI * kNI), mi = (m / kNI) % kMI, ni = m % kNI;
-    acc[bb][mi][ni] = tm_mfma32x32x16<DT>(f[mi], f[kMI + bb * kNI + ni], acc[bb][mi][ni]);
-  };
-  // One k-step: its MFMAs on `f`, and between them (in fixed groups, so the
-  // waits of neither sit in front of the matrix core) the reads of `next`
-  // from `rd` at k-step ks and, with DMA, the kDma loads of stage `st` into
-  // `dst` (kDma == kFrag for every shape here).
-  static_assert(kDma == kFrag, "one load per operand read");
-  constexpr int kPer = kMfma / kFrag;
-  auto kstep = [&](auto dma_c, const uint4 (&f)[kFrag], uint4 (&next)[kFrag], const uint4 *rd, int ks, uint4 *dst,
-                   int st) {
-    tm_static_for<kFrag>([&](auto g_c) {
-      constexpr int g = decltype(g_c)::value;
-      tm_static_for<kPer>([&](auto q_c) { mfma_one(std::integral_constant<int, g * kPer + decltype(q_c)::value>{}, f); });
-      read_one(g_c, next, rd, ks);
-      if constexpr (decltype(dma_c)::value) issue_one(g_c, dst, st);
-      __builtin_amdgcn_sched_barrier(0);
-    });
-    tm_static_for<kMfma - kFrag * kPer>(
-        [&](auto q_c) { mfma_one(std::integral_constant<int, kFrag * kPer + decltype(q_c)::value>{}, f); });
-  };
-
-  issue(ring0, 0);
-  issue(ring1, 1);
-  issue(ring2, 2);
-  issue(ring3, 3);
-  tm_wait_vm_lgkm0<3 * kDma>();  // stage 0 of this wave landed
-  __builtin_amdgcn_s_barrier();
-  tm_static_for<kFrag>([&](auto g_c) { read_one(g_c, fr[0], ring0, 0); });
-
-  // stage i in ring slot `cur`, stage i + 1 in `nxt`
-  auto step = [&](uint4 *cur, const uint4 *nxt, int i) {
-    kstep(std::false_type{}, fr[0], fr[1], cur, 1, cur, 0);
-    tm_wait_vm_lgkm0<2 * kDma>();  // stage i + 1 of this wave landed (i + 2, i + 3 may fly); reads done
-    __builtin_amdgcn_s_barrier();  // ... in every wave; no wave reads slot `cur` any more
-    kstep(std::true_type{}, fr[1], fr[0], nxt, 0, cur, i + 4);
-  };
-  for (int i = 0; i < KT; i += 4) {
-    step(ring0, ring1, i);
-    step(ring1, ring2, i + 1);
-    step(ring2, ring3, i + 2);
-    step(ring3, ring0, i + 3);
-  }
-  tm_wait_vm_lgkm0<0>();  // no load may still target this workgroup's LDS when it exits
-  __syncthreads();         // ... and every wave is done with the ring
-
-  // Epilogue through LDS, kStageCols columns at a time.  Each wave writes its
-  // fp32 results (up mode: silu(dtype(g)) * u, unrounded) to the staging tile
-  // [BM][kStageLd]: lane owns column (lane % 32) of each block and its 16 rows
-  // 8 (i / 4) + 4 (lane / 32) + i % 4 (the +8 float row padding puts the two
-  // row groups of one write on disjoint banks).  Then each thread rounds and
-  // stores 8-column chunks: 16 threads per 128-column row, so every store of a
-  // wave writes 4 whole rows (down mode adds the addend row chunk first, in
-  // fp32, one rounding).
-  float *const stage = reinterpret_cast<float *>(lds_all);
-  const int lrow = wm * 128 + 4 * (lane >> 5), lcol = wn * (BN / 2) + (lane & 31);
-#pragma unroll
-  for (int pass = 0; pass < BN / kStageCols; ++pass) {
-    if (pass > 0) __syncthreads();  // the previous pass's chunks are read
-    if (lcol - (lane & 31) >= pass * kStageCols && lcol - (lane & 31) < (pass + 1) * kStageCols) {  // uniform
-      float *w = stage + lrow * kStageLd + (lcol - pass * kStageCols);
-#pragma unroll
-      for (int mi = 0; mi < kMI; ++mi)
-#pragma unroll
-        for (int ni = 0; ni < kNI; ++ni)
-#pragma unroll
-          for (int i = 0; i < 16; ++i) {
-            float v;
+          for (int i = 0; i < 4; ++i) {
             if constexpr (MODE == kModeUp) {
-              const float g = tm_round<DT>(acc[0][mi][ni][i]);
-              v = g * __builtin_amdgcn_rcpf(1.f + __expf(-g)) * acc[NB - 1][mi][ni][i];
+              const float g = tm_round<DT>(acc[0][b][4 * u + i]);
+              const float up = CW == 32 ? acc[Cfg::kNA - 1][b][4 * u + i] : acc[0][b][(CW / 2 + 4 * u + i) & 15];
+              v[i] = g * __builtin_amdgcn_rcpf(1.f + __expf(-g)) * up;
             } else {
-              v = acc[0][mi][ni][i];
+              v[i] = acc[u / 4][b][(4 * u + i) & 15];
             }
-            w[(mi * 32 + 8 * (i >> 2) + (i & 3)) * kStageLd + ni * 32] = v;
           }
-    }
-    __syncthreads();
-#pragma unroll 4
-    for (int k = 0; k < BM * kStageCols / 8 / kThreads; ++k) {
-      const int c = tid + k * kThreads;
-      const int row = c / (kStageCols / 8), col8 = (c % (kStageCols / 8)) * 8;
-      const int gr = r0 + row;
-      if (gr >= r_end) break;  // rows only grow with k
-      const int col = n0 + pass * kStageCols + col8;
-      float v[8];
-      const float4 *src = reinterpret_cast<const float4 *>(stage + row * kStageLd + col8);
-      const float4 lo = src[0], hi = src[1];
-      v[0] = lo.x; v[1] = lo.y; v[2] = lo.z; v[3] = lo.w; v[4] = hi.x; v[5] = hi.y; v[6] = hi.z; v[7] = hi.w;
-      if constexpr (MODE == kModeDown) {
-        if (addend != nullptr) {  // dense rows only
-          float a[8];
-          tm_load8<DT>(addend + (int64_t)gr * ld_add + col, a);
+          if constexpr (MODE == kModeDown) {
+            if (addend != nullptr) {  // dense rows only
+              const uint2 a = *reinterpret_cast<const uint2 *>(addend + (int64_t)gr * ld_add + col);
+              const T *ae = reinterpret_cast<const T *>(&a);
 #pragma unroll
-          for (int j = 0; j < 8; ++j) v[j] += a[j];
+              for (int i = 0; i < 4; ++i) v[i] += Elem<DT>::to_f(ae[i]);
+            }
+          }
+          uint2 r;
+          T *re = reinterpret_cast<T *>(&r);
+#pragma unroll
+          for (int i = 0; i < 4; ++i) re[i] = Elem<DT>::from_f(v[i]);
+          T *dst;
+          if constexpr (PB && MODE == kModeUp)  // tile y of the intermediate in the down GEMM's stage order
+            dst = C + y * (int64_t)BM * ldc + (col / BK) * (BM * BK) +
+                  ((rb + tr) * kCPR + swz_chunk(rb + tr, (col % BK) / 8)) * 8 + col % 8;
+          else
+            dst = C + (c_rows ? c_rows[gr] + col : (int64_t)gr * ldc + col);
+          *reinterpret_cast<uint2 *>(dst) = r;
         }
       }
-      if constexpr (PB && MODE == kModeUp)  // tile y of the intermediate in the down GEMM's stage order
-        tm_store8<DT>(C + y * (int64_t)BM * ldc + (col / BK) * (BM * BK) +
-                          (row * kCPR + swz_chunk(row, (col % BK) / 8)) * 8,
-                      v);
+    }
+  }
+}
+
+// One tile of one expert, up to BM rows x BN columns, operands as in the wave
+// kernel (A = weight rows, B = activation rows), eight waves that share both:
+// wave w owns the columns of group w % 4 (up: gate and up rows of 32 columns
+// of the 128; down: BN / 4 columns) and the row blocks of half w / 4.  Only the
+// 32-row blocks that the tile has rows in are loaded and multiplied, NB = 1 ..
+// 4 per half, and the LDS ring is cut into as many stages as fit: few rows
+// leave room for a deeper ring, which is what a tile that only streams its
+// weights needs.  One barrier per stage, between its two k-steps: it publishes
+// the next stage and frees the slot that the stage after the ring goes to.
+// Every result is the same chain of products as in the wave kernel.
+//
+// Bound by the bytes that a CU has on their way from HBM (three 32 KiB stages
+// of 4 waves before; with 8 waves and 5 to 8 stages now), by activation rows
+// that miss L2 behind the stream of weights (so weights that one workgroup
+// alone reads are loaded non-temporally: 5280 rows of 128 experts 272 -> 253
+// us; weights that several row tiles read are not: 510 against 594 us at 14.4k
+// rows of 64 experts), and, from ~150 rows per expert, by the matrix cores.  us
+// per call before (4 waves, one per SIMD, always 256 rows) -> now: hidden 2048,
+// inter 768, 128 experts: 960 rows 287 -> 205, 5280 rows 310 -> 253, 19.2k rows
+// 409 -> 366; hidden 2560, inter 1536, 64 experts: 1800 rows 358 -> 287, 14.4k
+// rows 556 -> 510.
+constexpr int kTileThreads = 512;
+constexpr int kTileLds = 163840;
+
+// Wait until at most `left` stages of kDma loads are outstanding (and LDS
+// reads are done).
+template <int kDma, int kMost>
+__device__ __forceinline__ void wait_stages(int left) {
+  if constexpr (kMost <= 0) {
+    tm_wait_vm_lgkm0_mem<0>();
+  } else {
+    if (left >= kMost) tm_wait_vm_lgkm0_mem<kMost * kDma>();
+    else wait_stages<kDma, kMost - 1>(left);
+  }
+}
+
+template <int DT, int MODE, int BN, bool PB>
+__global__ __launch_bounds__(kTileThreads, 2) void tile_gemm_kernel(
+    const typename Elem<DT>::T *__restrict__ A, int64_t lda, const int32_t *__restrict__ a_rows,
+    const typename Elem<DT>::T *__restrict__ B0, const typename Elem<DT>::T *__restrict__ B1, int64_t b_expert,
+    int K, int n_tiles, TileSrc ts, typename Elem<DT>::T *__restrict__ C, int64_t ldc,
+    const int64_t *__restrict__ c_rows, const typename Elem<DT>::T *__restrict__ addend, int64_t ld_add) {
+  using T = typename Elem<DT>::T;
+  constexpr int kMats = MODE == kModeUp ? 2 : 1;
+  constexpr int kWLoads = kMats * BN / 16;   // 1 KiB loads of a stage's weight rows
+  constexpr int kWDma = kWLoads / 8;         // ... per wave
+  constexpr int kWBytes = kWLoads * 1024;
+  constexpr int NA = MODE == kModeUp ? 2 : BN / 128;  // 32-row weight operands per wave
+  __shared__ uint4 ring[kTileLds / 16];
+
+  // Block b runs on XCD b % 8 (the dispatcher's round robin): the n_tiles
+  // column tiles of row tile y get ids 8 apart, so they share one XCD and its
+  // L2 copy of the tile's activation rows.
+  // Work items: (row tile, column tile), n_tiles per row tile.  Item b of the
+  // whole groups of 8 row tiles is row tile 8 (b / 8 / n_tiles) + b % 8, so a
+  // row tile's items run on one XCD (the dispatcher's round robin) and share
+  // its L2 copy of the activation rows; the last row tiles follow in order.
+  // The items past the last whole round of 256 are cut into 2 or 4 row
+  // ranges where that still fits the CUs (a range's parts on one XCD): 8192
+  // dense rows of hidden 2560, inter 1536 (384 items) 239 -> 214 us.
+  const int64_t row_tiles = ts.tiles != nullptr ? (ts.tiles[1] < ts.t_max ? ts.tiles[1] : ts.t_max)
+                                                : ((int64_t)ts.rows + BM - 1) / BM;
+  const int64_t total = row_tiles * n_tiles, full = row_tiles / 8 * 8 * n_tiles, rounds = total / 256 * 256;
+  int64_t b = blockIdx.x;
+  int h0 = 0, wg_rows = BM;  // this workgroup's row range of the row tile
+  if (b >= rounds) {
+    const int rem = (int)(total - rounds), id = (int)(b - rounds);
+    const int sh = rem <= 64 ? 2 : rem <= 128 ? 1 : 0;
+    wg_rows = BM >> sh;
+    h0 = ((id >> 3) & ((1 << sh) - 1)) * wg_rows;
+    b = rounds + (id >> (3 + sh)) * 8 + (id & 7);
+  }
+  if (b >= total) return;
+  int64_t y, col_tile;
+  if (b < full) {
+    y = (b >> 3) / n_tiles * 8 + (b & 7);
+    col_tile = (b >> 3) % n_tiles;
+  } else {
+    y = full / n_tiles + (b - full) / n_tiles;
+    col_tile = (b - full) % n_tiles;
+  }
+  const int n0 = (int)col_tile * BN;
+  int e, r0, r_end;
+  bool once = false;
+  if (ts.tiles != nullptr) {
+    e = ts.tiles[2 + y];
+    r0 = ts.tiles[2 + ts.t_max + y] + h0;
+    r_end = ts.expert_offsets[e + 1];
+    once = r_end - ts.expert_offsets[e] <= BM;
+  } else {
+    e = 0;
+    r0 = (int)y * BM + h0;
+    r_end = ts.rows;
+  }
+  if (r0 >= r_end) return;
+  const int rows = r_end - r0 < wg_rows ? r_end - r0 : wg_rows;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int cg = wave & 3, half = wave >> 2;
+  const int KT = K / BK;  // a multiple of 4
+  const uint32_t lds0 = (uint32_t)(uintptr_t)ring;
+  const char *const lds = reinterpret_cast<const char *>(ring);
+
+  // Weight loads wave * kWDma + j (16 rows of 64 bytes each, the slot order of
+  // the packed layout), through a buffer whose scalar offset walks K.
+  tm_rsrc_t w_rs[kMats];
+  w_rs[0] = tm_make_rsrc(B0 + (int64_t)e * b_expert + (int64_t)n0 * K, (uint64_t)BN * K * sizeof(T));
+  if constexpr (kMats > 1)
+    w_rs[1] = tm_make_rsrc(B1 + (int64_t)e * b_expert + (int64_t)n0 * K, (uint64_t)BN * K * sizeof(T));
+  const tm_rsrc_t w_mine = kMats > 1 && wave >= 4 ? w_rs[kMats - 1] : w_rs[0];  // up: waves 0-3 W1, waves 4-7 W3
+  uint32_t w_off[kWDma];
+#pragma unroll
+  for (int j = 0; j < kWDma; ++j) {
+    const int p = (((kMats > 1 ? wave & 3 : wave) * kWDma + j) * 64) + lane;  // 16-byte slot in the matrix's stage
+    const int row = p / kCPR, kc = swz_chunk(row, p % kCPR);
+    w_off[j] = PB ? (uint32_t)p * 16u : (uint32_t)row * (uint32_t)K * (uint32_t)sizeof(T) + (uint32_t)kc * 16u;
+  }
+  constexpr uint32_t kWStep = PB ? BN * 64 : BK * sizeof(T);
+  constexpr bool kTiledA = PB && MODE == kModeDown;
+  constexpr int64_t kXStep = kTiledA ? BM * BK : BK;
+
+  // operand offsets in a slot: weight rows of this wave, activation rows
+  uint32_t a_off[2], b_off[2];
+  const int ar = lane & 31;
+#pragma unroll
+  for (int ks = 0; ks < 2; ++ks) {
+    const uint32_t in_rows = (uint32_t)(ar * 64 + swz_chunk(ar, 2 * ks + (lane >> 5)) * 16);
+    a_off[ks] = in_rows + (uint32_t)cg * (MODE == kModeUp ? 2048u : NA * 2048u);
+    b_off[ks] = in_rows + kWBytes;
+    asm volatile("" : "+v"(a_off[ks]), "+v"(b_off[ks]));
+  }
+
+  tm_f32x16 acc[NA][4];
+#pragma unroll
+  for (int a = 0; a < NA; ++a)
+#pragma unroll
+    for (int q = 0; q < 4; ++q) acc[a][q] = tm_f32x16{};
+
+  auto run = [&](auto nb_c, auto once_c) {
+    constexpr int NB = decltype(nb_c)::value;
+    constexpr int kXDma = (NB + 1) / 2;  // loads of 16 activation rows per wave (4 NB in all)
+    constexpr int kDma = kWDma + kXDma;
+    constexpr int kStageBytes = kWBytes + NB * 4096;
+    constexpr int kSlots = kTileLds / kStageBytes < 8 ? kTileLds / kStageBytes : 8;
+    const uint32_t b_half = (uint32_t)(half * NB * 2048);
+    constexpr int kFrag = NA + NB, kMfma = NA * NB;
+    const T *x_src[kXDma];
+    uint32_t x_dst[kXDma];
+#pragma unroll
+    for (int j = 0; j < kXDma; ++j) {
+      const int q = (wave * kXDma + j) % (4 * NB);  // (spare waves repeat a load)
+      const int tr = q * 16 + (lane >> 2);
+      x_dst[j] = (uint32_t)(kWBytes + q * 1024);
+      if constexpr (kTiledA) {
+        x_src[j] = A + y * (int64_t)BM * lda + (int64_t)(h0 + tr) * BK + (lane & 3) * 8;
+      } else {
+        int gr = r0 + tr;
+        gr = gr < r_end ? gr : r_end - 1;  // rows past the expert re-read its last row; their results are dropped
+        const int64_t xr = a_rows ? (int64_t)a_rows[gr] : (int64_t)gr;
+        x_src[j] = A + xr * lda + swz_chunk(tr, lane & 3) * 8;
+      }
+    }
+    // load j of stage kt into the slot at byte `slot`
+    auto issue_one = [&](auto j_c, uint32_t slot, int kt) {
+      constexpr int j = decltype(j_c)::value;
+      if constexpr (j < kWDma)
+        tm_dma16_buf_so<decltype(once_c)::value>(w_mine, w_off[j], (uint32_t)kt * kWStep,
+                                                 lds0 + slot + (uint32_t)(wave * kWDma + j) * 1024u);
       else
-        tm_store8<DT>(C + (c_rows ? c_rows[gr] + col : (int64_t)gr * ldc + col), v);
+        tm_dma16_s(x_src[j - kWDma] + (int64_t)kt * kXStep, lds0 + slot + x_dst[j - kWDma]);
+    };
+    uint4 fr[2][kFrag];
+    auto read_one = [&](auto g_c, uint4 (&f)[kFrag], uint32_t slot, int ks) {
+      constexpr int g = decltype(g_c)::value;
+      if constexpr (g < NA)
+        f[g] = *reinterpret_cast<const uint4 *>(lds + slot + a_off[ks] + g * (MODE == kModeUp ? BN * 64 : 2048));
+      else
+        f[g] = *reinterpret_cast<const uint4 *>(lds + slot + b_half + b_off[ks] + (g - NA) * 2048);
+    };
+    // one k-step: its products, and spread between them the operand reads of
+    // the next one and (with DMA) the loads of a stage
+    auto kstep = [&](auto dma_c, const uint4 (&f)[kFrag], uint4 (&next)[kFrag], uint32_t rd, int ks, uint32_t dst,
+                     int st) {
+      tm_static_for<kMfma>([&](auto m_c) {
+        constexpr int m = decltype(m_c)::value;
+        constexpr int a = m / NB, q = m % NB;
+        acc[a][q] = tm_mfma32x32x16<DT>(f[a], f[NA + q], acc[a][q]);
+        constexpr int g0 = m * kFrag / kMfma, g1 = (m + 1) * kFrag / kMfma;
+        tm_static_for<g1 - g0>(
+            [&](auto g_c) { read_one(std::integral_constant<int, g0 + decltype(g_c)::value>{}, next, rd, ks); });
+        if constexpr (decltype(dma_c)::value) {
+          constexpr int d0 = m * kDma / kMfma, d1 = (m + 1) * kDma / kMfma;
+          tm_static_for<d1 - d0>(
+              [&](auto d_c) { issue_one(std::integral_constant<int, d0 + decltype(d_c)::value>{}, dst, st); });
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      });
+    };
+    const int first = KT < kSlots ? KT : kSlots;
+    for (int st = 0; st < first; ++st)
+      tm_static_for<kDma>([&](auto j_c) { issue_one(j_c, (uint32_t)(st * kStageBytes), st); });
+    wait_stages<kDma, kSlots - 1>(first - 1);  // stage 0 of this wave landed
+    __builtin_amdgcn_s_barrier();
+    tm_static_for<kFrag>([&](auto g_c) { read_one(g_c, fr[0], 0u, 0); });
+    uint32_t cur = 0;
+    int i = 0;
+    for (; i < KT - kSlots; ++i) {
+      const uint32_t nxt = cur == (kSlots - 1) * kStageBytes ? 0u : cur + kStageBytes;
+      kstep(std::false_type{}, fr[0], fr[1], cur, 1, 0u, 0);
+      tm_wait_vm_lgkm0_mem<(kSlots - 2) * kDma>();  // stage i + 1 of this wave landed; its reads are done
+      __builtin_amdgcn_s_barrier();                 // ... in every wave; no wave reads slot `cur` any more
+      kstep(std::true_type{}, fr[1], fr[0], nxt, 0, cur, i + kSlots);
+      cur = nxt;
+    }
+    for (; i < KT; ++i) {  // the last stages: nothing more to load
+      const uint32_t nxt = cur == (kSlots - 1) * kStageBytes ? 0u : cur + kStageBytes;
+      kstep(std::false_type{}, fr[0], fr[1], cur, 1, 0u, 0);
+      wait_stages<kDma, kSlots - 2>(KT - 2 - i);
+      __builtin_amdgcn_s_barrier();
+      kstep(std::false_type{}, fr[1], fr[0], nxt, 0, 0u, 0);
+      cur = nxt;
+    }
+  };
+  const int nb = (rows + 63) / 64;  // 32-row blocks per half
+  const int first_row = half * nb * 32;
+  auto run_nb = [&](auto once_c) {
+    if (nb == 1) run(std::integral_constant<int, 1>{}, once_c);
+    else if (nb == 2) run(std::integral_constant<int, 2>{}, once_c);
+    else if (nb == 3) run(std::integral_constant<int, 3>{}, once_c);
+    else run(std::integral_constant<int, 4>{}, once_c);
+  };
+  // Packed weights that no other row tile reads are loaded non-temporally.
+  if (PB && once) run_nb(std::integral_constant<bool, PB>{});
+  else run_nb(std::false_type{});
+
+  // lane: activation row lane % 32 of each block, weight rows 8 (i / 4) + 4
+  // (lane / 32) + i % 4 of each operand: runs of 4 consecutive columns
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const int tr = first_row + 32 * q + (lane & 31);
+    if (q < nb && tr < rows) {
+      const int gr = r0 + tr;
+#pragma unroll
+      for (int u = 0; u < (MODE == kModeUp ? 4 : 4 * NA); ++u) {
+        const int col = n0 + cg * (MODE == kModeUp ? 32 : NA * 32) + 8 * u + 4 * (lane >> 5);
+        float v[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          if constexpr (MODE == kModeUp) {
+            const float g = tm_round<DT>(acc[0][q][4 * u + i]);
+            v[i] = g * __builtin_amdgcn_rcpf(1.f + __expf(-g)) * acc[NA - 1][q][4 * u + i];
+          } else {
+            v[i] = acc[u / 4][q][(4 * u + i) & 15];
+          }
+        }
+        if constexpr (MODE == kModeDown) {
+          if (addend != nullptr) {  // dense rows only
+            const uint2 ad = *reinterpret_cast<const uint2 *>(addend + (int64_t)gr * ld_add + col);
+            const T *ae = reinterpret_cast<const T *>(&ad);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) v[i] += Elem<DT>::to_f(ae[i]);
+          }
+        }
+        uint2 r;
+        T *re = reinterpret_cast<T *>(&r);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) re[i] = Elem<DT>::from_f(v[i]);
+        T *dst;
+        if constexpr (PB && MODE == kModeUp)  // tile y of the intermediate in the down GEMM's stage order
+          dst = C + y * (int64_t)BM * ldc + (col / BK) * (BM * BK) +
+                ((h0 + tr) * kCPR + swz_chunk(tr, (col % BK) / 8)) * 8 + col % 8;
+        else
+          dst = C + (c_rows ? c_rows[gr] + col : (int64_t)gr * ldc + col);
+        *reinterpret_cast<uint2 *>(dst) = r;
+      }
     }
   }
 }
@@ -525,6 +823,9 @@ __global__ __launch_bounds__(kGrpThreads) void group_count_kernel(const int64_t 
   for (int e = tid; e < n_experts; e += kGrpThreads) counts[(int64_t)blockIdx.x * n_experts + e] = h[e];
 }
 
+// ONE: the batch fits one workgroup, which counts its rows itself (no
+// group_count_kernel launch before it).
+template <bool ONE>
 __global__ __launch_bounds__(kGrpThreads) void group_place_kernel(
     const int64_t *__restrict__ ids, int64_t n, int top_k, int64_t ld_ids, const uint8_t *__restrict__ mask,
     int64_t ms_b, int64_t ms_s, int n_experts, int64_t so_b, int64_t so_s, const int32_t *__restrict__ counts,
@@ -539,40 +840,50 @@ __global__ __launch_bounds__(kGrpThreads) void group_place_kernel(
   const int s0 = 2 * (tid % 4);
   int ex[2];
   grp_entries(ids, n, top_k, ld_ids, mask, ms_b, ms_s, n_experts, b, s0, ex);
-  // Thread (e, p) of ep = pow2 >= n_experts columns sums the count rows
-  // g = p, p + P, .. (P = 256 / ep) of expert e: kGrpBatch rows per round
-  // trip (clamped rows, masked by a select).
-  int ep = 1;
-  while (ep < n_experts) ep <<= 1;
-  const int P = kGrpThreads / ep;
-  const int e = tid % ep, p = tid / ep;
-  const int ec = e < n_experts ? e : n_experts - 1;
-  int32_t tot = 0, bef = 0;
-  for (int g = p; g < G; g += P * kGrpBatch) {
-    int32_t v[kGrpBatch];
-#pragma unroll
-    for (int j = 0; j < kGrpBatch; ++j) {
-      const int gj = g + P * j;
-      v[j] = counts[(int64_t)(gj < G ? gj : G - 1) * n_experts + ec];
-    }
-#pragma unroll
-    for (int j = 0; j < kGrpBatch; ++j) {
-      const int gj = g + P * j;
-      const int32_t c = (gj < G && e < n_experts) ? v[j] : 0;
-      tot += c;
-      bef += gj < g0 ? c : 0;
-    }
-  }
-  part_tot[tid] = tot;
-  part_bef[tid] = bef;
-  __syncthreads();
   // thread x owns expert x: its total and the rows of the earlier workgroups
   int32_t h = 0, hb = 0;
-  if (tid < n_experts)
-    for (int q = 0; q < P; ++q) {
-      h += part_tot[q * ep + tid];
-      hb += part_bef[q * ep + tid];
+  if constexpr (ONE) {
+    part_tot[tid] = 0;
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+      if (ex[u] >= 0) atomicAdd(&part_tot[ex[u]], 1);
+    __syncthreads();
+    h = part_tot[tid];
+  } else {
+    // Thread (e, p) of ep = pow2 >= n_experts columns sums the count rows
+    // g = p, p + P, .. (P = 256 / ep) of expert e: kGrpBatch rows per round
+    // trip (clamped rows, masked by a select).
+    int ep = 1;
+    while (ep < n_experts) ep <<= 1;
+    const int P = kGrpThreads / ep;
+    const int e = tid % ep, p = tid / ep;
+    const int ec = e < n_experts ? e : n_experts - 1;
+    int32_t tot = 0, bef = 0;
+    for (int g = p; g < G; g += P * kGrpBatch) {
+      int32_t v[kGrpBatch];
+#pragma unroll
+      for (int j = 0; j < kGrpBatch; ++j) {
+        const int gj = g + P * j;
+        v[j] = counts[(int64_t)(gj < G ? gj : G - 1) * n_experts + ec];
+      }
+#pragma unroll
+      for (int j = 0; j < kGrpBatch; ++j) {
+        const int gj = g + P * j;
+        const int32_t c = (gj < G && e < n_experts) ? v[j] : 0;
+        tot += c;
+        bef += gj < g0 ? c : 0;
+      }
     }
+    part_tot[tid] = tot;
+    part_bef[tid] = bef;
+    __syncthreads();
+    if (tid < n_experts)
+      for (int q = 0; q < P; ++q) {
+        h += part_tot[q * ep + tid];
+        hb += part_bef[q * ep + tid];
+      }
+  }
   // exclusive scans over the experts (rows and 256-row tiles): wave scans,
   // then the waves' totals in wave order
   const int32_t tc = (h + BM - 1) / BM;
@@ -621,55 +932,125 @@ __global__ __launch_bounds__(kGrpThreads) void group_place_kernel(
     }
 }
 
-template <int DT, int NB, int MODE, int BN, bool PB>
-void launch_gemm(const void *A, int64_t lda, const int32_t *a_rows, const void *B0, const void *B1, int64_t b_expert,
-                 int K, int N, const TileSrc &ts, int64_t grid_y, void *C, int64_t ldc, const int64_t *c_rows,
-                 const void *addend, int64_t ld_add, hipStream_t s) {
-  using T = typename Elem<DT>::T;
-  const int n_tiles = N / BN;
-  const int64_t blocks = tm_cdiv(grid_y, 8) * 8 * n_tiles;
-  hipLaunchKernelGGL((grouped_gemm_kernel<DT, NB, MODE, BN, PB>), dim3((unsigned)blocks), dim3(kThreads), 0, s,
-                     static_cast<const T *>(A), lda, a_rows, static_cast<const T *>(B0), static_cast<const T *>(B1),
-                     b_expert, K, n_tiles, ts, static_cast<T *>(C), ldc, c_rows, static_cast<const T *>(addend),
-                     ld_add);
-}
-
 // Column tile of the down GEMM: 256 columns when hidden allows (half the LDS
 // reads per MFMA of 128-column tiles).
 inline int down_bn(int32_t hidden) { return hidden % (2 * kMinBN) == 0 ? 2 * kMinBN : kMinBN; }
 
+// Which kernel runs the two GEMMs; every one gives the same bits.
+enum { kPlanTile = 0, kPlanWave, kPlanWave64 };
+
+// Few waves: 8 (16) columns per wave, 64-column stages and a deep ring; else
+// twice the columns and a ring that leaves room for 10 waves per CU.
+using SkUpFew = SkinnyCfg<kModeUp, 8, 2, 49152, 32>;
+using SkDownFew = SkinnyCfg<kModeDown, 16, 2, 49152, 32>;
+using SkUpMany = SkinnyCfg<kModeUp, 16, 1, 16384, 32>;
+using SkDownMany = SkinnyCfg<kModeDown, 32, 1, 16384, 32>;
+using SkUp64 = SkinnyCfg<kModeUp, 32, 1, 32768, 64>;
+using SkDown64 = SkinnyCfg<kModeDown, 64, 1, 32768, 64>;
+constexpr int kSkManyWaves = 512;
+
+template <int DT, class Cfg, bool PB>
+void launch_skinny(const void *A, int64_t lda, const int32_t *a_rows, const void *B0, const void *B1, int64_t b_expert,
+                   int K, int N, const TileSrc &ts, int64_t tiles, void *C, int64_t ldc, const int64_t *c_rows,
+                   const void *addend, int64_t ld_add, hipStream_t s) {
+  using T = typename Elem<DT>::T;
+  const int pack_bn = Cfg::MODE == kModeUp ? kMinBN : down_bn(N);
+  const bool grouped = ts.tiles != nullptr;
+  const int split = grouped ? 0 : BM / Cfg::RBMAX;
+  const int64_t blocks = grouped ? tiles : tm_cdiv(ts.rows, Cfg::RBMAX);
+  auto launch = [&](auto once_c) {
+    hipLaunchKernelGGL((skinny_gemm_kernel<DT, Cfg, PB, decltype(once_c)::value>),
+                       dim3((unsigned)(blocks * (N / Cfg::CW))), dim3(64), 0, s, static_cast<const T *>(A), lda, a_rows,
+                       static_cast<const T *>(B0), static_cast<const T *>(B1), b_expert, K, N / Cfg::CW, pack_bn, split,
+                       ts, static_cast<T *>(C), ldc, c_rows, static_cast<const T *>(addend), ld_add);
+  };
+  if (PB && grouped) launch(std::integral_constant<bool, PB>{});
+  else launch(std::false_type{});
+}
+
+template <int DT, int MODE, int BN, bool PB>
+void launch_tile(const void *A, int64_t lda, const int32_t *a_rows, const void *B0, const void *B1, int64_t b_expert,
+                 int K, int N, const TileSrc &ts, int64_t tiles, void *C, int64_t ldc, const int64_t *c_rows,
+                 const void *addend, int64_t ld_add, hipStream_t s) {
+  using T = typename Elem<DT>::T;
+  const int n_tiles = N / BN;
+  hipLaunchKernelGGL((tile_gemm_kernel<DT, MODE, BN, PB>), dim3((unsigned)(tm_cdiv(tiles * n_tiles, 256) * 256)),
+                     dim3(kTileThreads), 0, s, static_cast<const T *>(A), lda, a_rows, static_cast<const T *>(B0),
+                     static_cast<const T *>(B1), b_expert, K, n_tiles, ts, static_cast<T *>(C), ldc, c_rows,
+                     static_cast<const T *>(addend), ld_add);
+}
+
 template <int DT, bool PB>
 void swiglu_launch(const void *x, int64_t ld_x, const int32_t *row_token, int32_t hidden, int32_t inter,
-                   const void *w1, const void *w3, const void *w2, const TileSrc &ts, int64_t grid_y, void *out,
+                   const void *w1, const void *w3, const void *w2, const TileSrc &ts, int64_t tiles, void *out,
                    int64_t ld_out, const int64_t *row_out, void *fused, const void *addend, int64_t ld_add,
-                   hipStream_t s) {
-  launch_gemm<DT, 2, kModeUp, kMinBN, PB>(x, ld_x, row_token, w1, w3, (int64_t)inter * hidden, hidden, inter, ts,
-                                          grid_y, fused, inter, nullptr, nullptr, 0, s);
-  if (down_bn(hidden) == 2 * kMinBN)
-    launch_gemm<DT, 1, kModeDown, 2 * kMinBN, PB>(fused, inter, nullptr, w2, nullptr, (int64_t)hidden * inter, inter,
-                                                  hidden, ts, grid_y, out, ld_out, row_out, addend, ld_add, s);
-  else
-    launch_gemm<DT, 1, kModeDown, kMinBN, PB>(fused, inter, nullptr, w2, nullptr, (int64_t)hidden * inter, inter,
-                                              hidden, ts, grid_y, out, ld_out, row_out, addend, ld_add, s);
+                   int plan, hipStream_t s) {
+  const int64_t bw = (int64_t)inter * hidden;
+  auto up = [&](auto cfg) {
+    launch_skinny<DT, decltype(cfg), PB>(x, ld_x, row_token, w1, w3, bw, hidden, inter, ts, tiles, fused, inter,
+                                         nullptr, nullptr, 0, s);
+  };
+  auto down = [&](auto cfg) {
+    launch_skinny<DT, decltype(cfg), PB>(fused, inter, nullptr, w2, nullptr, bw, inter, hidden, ts, tiles, out, ld_out,
+                                         row_out, addend, ld_add, s);
+  };
+  if (plan == kPlanWave) {
+    const int64_t blocks = ts.tiles == nullptr ? tm_cdiv(ts.rows, 32) : tiles;
+    if (blocks * (inter / 16) >= kSkManyWaves) up(SkUpMany{});
+    else up(SkUpFew{});
+    if (blocks * (hidden / 32) >= kSkManyWaves) down(SkDownMany{});
+    else down(SkDownFew{});
+  } else if (plan == kPlanWave64) {
+    up(SkUp64{});
+    down(SkDown64{});
+  } else {
+    launch_tile<DT, kModeUp, kMinBN, PB>(x, ld_x, row_token, w1, w3, bw, hidden, inter, ts, tiles, fused, inter,
+                                         nullptr, nullptr, 0, s);
+    if (down_bn(hidden) == 2 * kMinBN)
+      launch_tile<DT, kModeDown, 2 * kMinBN, PB>(fused, inter, nullptr, w2, nullptr, bw, inter, hidden, ts, tiles, out,
+                                                 ld_out, row_out, addend, ld_add, s);
+    else
+      launch_tile<DT, kModeDown, kMinBN, PB>(fused, inter, nullptr, w2, nullptr, bw, inter, hidden, ts, tiles, out,
+                                             ld_out, row_out, addend, ld_add, s);
+  }
+}
+
+// The plan of a dense call.  One wave per column group needs no LDS exchange
+// and spreads a single expert over the chip, but re-reads its operands per 32
+// (64) rows; measured crossovers (hidden x inter 2048 x 768 | 2560 x 1536, us
+// per call): 128 rows 14 | 21 against 26 | 34 with 64-row waves and 44 | 64
+// with tiles; 512 rows 22 | 54, 27 | 37, 41 | 65; 2048 rows 81 | 192, 53 | 132,
+// 43 | 68.
+int dense_plan(int64_t rows, int32_t hidden, int32_t inter) {
+  const double work = (double)rows * hidden * inter;
+  return work <= 1.1e9 ? kPlanWave : work <= 3e9 ? kPlanWave64 : kPlanTile;
+}
+
+// The plan of a grouped call, from the most rows per expert that it can have
+// on average (the counts are on the device): measured us per call, waves |
+// tiles, at 12.5 (128 experts, 2048 x 768): 205 | 203, at 18.8 (64 experts,
+// 2560 x 1536): 292 | 264, at 9.4: 235 | 243, at 0.5: 51 | 55.
+int grouped_plan(int64_t max_rows, int32_t n_experts) {
+  return max_rows <= 12 * (int64_t)n_experts ? kPlanWave : kPlanTile;
 }
 
 // The two GEMMs of the MLP over the rows the tile source names; `addend`
 // (dense rows only, nullable) is added to the down projection before its
 // rounding; `packed`: the weights are in tm_expert_pack_weights's layout.
 int swiglu_impl(int32_t dtype, const void *x, int64_t ld_x, const int32_t *row_token, int32_t hidden,
-                int32_t inter, const void *w1, const void *w3, const void *w2, const TileSrc &ts, int64_t grid_y,
+                int32_t inter, const void *w1, const void *w3, const void *w2, const TileSrc &ts, int64_t tiles,
                 void *out, int64_t ld_out, const int64_t *row_out, void *fused, const void *addend, int64_t ld_add,
-                bool packed, hipStream_t s) {
+                bool packed, int plan, hipStream_t s) {
   return TM_DISPATCH_DTYPE(dtype, DT, [&] {
     if constexpr (DT == TM_DT_F32) {
       return tm_fail(TM_EINVAL_DTYPE, "tm_grouped_swiglu: dtype must be F16 or BF16");
     } else {
       if (packed)
-        swiglu_launch<DT, true>(x, ld_x, row_token, hidden, inter, w1, w3, w2, ts, grid_y, out, ld_out, row_out,
-                                fused, addend, ld_add, s);
+        swiglu_launch<DT, true>(x, ld_x, row_token, hidden, inter, w1, w3, w2, ts, tiles, out, ld_out, row_out,
+                                fused, addend, ld_add, plan, s);
       else
-        swiglu_launch<DT, false>(x, ld_x, row_token, hidden, inter, w1, w3, w2, ts, grid_y, out, ld_out, row_out,
-                                 fused, addend, ld_add, s);
+        swiglu_launch<DT, false>(x, ld_x, row_token, hidden, inter, w1, w3, w2, ts, tiles, out, ld_out, row_out,
+                                 fused, addend, ld_add, plan, s);
       TM_LAUNCH_CHECK("tm_grouped_swiglu");
       return TM_OK;
     }
@@ -765,10 +1146,15 @@ extern "C" int tm_group_slots_ws(const int64_t *ids, int64_t n_tokens, int32_t t
   const unsigned G = (unsigned)tm_cdiv(n_tokens, kGrpTok);
   hipStream_t s = tm_hip_stream(stream);
   int32_t *counts = static_cast<int32_t *>(workspace);
-  hipLaunchKernelGGL(group_count_kernel, dim3(G), dim3(kGrpThreads), 0, s, ids, n_tokens, top_k, ld_ids, mask, ms_b,
-                     ms_s, n_experts, counts);
-  hipLaunchKernelGGL(group_place_kernel, dim3(G), dim3(kGrpThreads), 0, s, ids, n_tokens, top_k, ld_ids, mask, ms_b,
-                     ms_s, n_experts, so_b, so_s, counts, expert_offsets, row_token, row_out, tiles, t_max);
+  if (G == 1) {  // up to kGrpTok tokens: one launch
+    hipLaunchKernelGGL(group_place_kernel<true>, dim3(1), dim3(kGrpThreads), 0, s, ids, n_tokens, top_k, ld_ids, mask,
+                       ms_b, ms_s, n_experts, so_b, so_s, counts, expert_offsets, row_token, row_out, tiles, t_max);
+  } else {
+    hipLaunchKernelGGL(group_count_kernel, dim3(G), dim3(kGrpThreads), 0, s, ids, n_tokens, top_k, ld_ids, mask, ms_b,
+                       ms_s, n_experts, counts);
+    hipLaunchKernelGGL(group_place_kernel<false>, dim3(G), dim3(kGrpThreads), 0, s, ids, n_tokens, top_k, ld_ids, mask,
+                       ms_b, ms_s, n_experts, so_b, so_s, counts, expert_offsets, row_token, row_out, tiles, t_max);
+  }
   TM_LAUNCH_CHECK("tm_group_slots_ws");
   return TM_OK;
 }
@@ -809,8 +1195,9 @@ int grouped_swiglu_impl(int32_t dtype, const void *x, int64_t ld_x, int32_t hidd
              "tm_grouped_swiglu: workspace %zu bytes < %zu", workspace_bytes, need);
   const int64_t t_max = tm_group_slots_tiles(max_rows, n_experts);
   const TileSrc ts{tiles, expert_offsets, t_max, 0};
-  return swiglu_impl(dtype, x, ld_x, row_token, hidden, inter, w1, w3, w2, ts, t_max, out, 0, row_out, workspace,
-                     nullptr, 0, packed, tm_hip_stream(stream));
+  return swiglu_impl(dtype, x, ld_x, row_token, hidden, inter, w1, w3, w2, ts, max_rows < t_max ? max_rows : t_max,
+                     out, 0, row_out, workspace, nullptr, 0, packed, grouped_plan(max_rows, n_experts),
+                     tm_hip_stream(stream));  // (a tile holds at least one row)
 }
 
 }  // namespace
@@ -893,7 +1280,8 @@ int expert_swiglu_impl(const char *name, int32_t dtype, const void *x, int64_t n
              "%s: workspace %zu bytes < %zu", name, workspace_bytes, need);
   const TileSrc ts{nullptr, nullptr, 0, (int32_t)n_rows};
   return swiglu_impl(dtype, x, ld_x, nullptr, hidden, inter, w1, w3, w2, ts, tm_cdiv(n_rows, BM), out, ld_out,
-                     nullptr, workspace, addend, ld_add, packed, tm_hip_stream(stream));
+                     nullptr, workspace, addend, ld_add, packed, dense_plan(n_rows, hidden, inter),
+                     tm_hip_stream(stream));
 }
 
 }  // namespace

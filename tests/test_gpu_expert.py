@@ -355,3 +355,59 @@ def test_shared_experts_packed_equals_plain(hip_device, m, addend, dtype):
     want = expert_swiglu(x, w1, w3, w2, addend=add)
     torch.cuda.synchronize()
     assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("h,inter,dtype,packed", [(2048, 768, torch.bfloat16, False), (2560, 1536, torch.float16, True),
+                                                  (384, 256, torch.bfloat16, True), (128, 128, torch.float16, False)])
+def test_dense_rows_do_not_depend_on_the_batch(hip_device, h, inter, dtype, packed):
+    """A row of the MLP has the same bits in a batch of any size, so whichever
+    kernel and tile cut the batch takes (one wave per column group with 16, 32
+    or 64 rows, tiles of 64 to 256 rows, the last round's tiles cut in 2 or
+    4), at the edges of each; a few rows against the oracle."""
+    from table_moe.ops import SharedExperts, expert_swiglu
+
+    dev = hip_device
+    g = torch.Generator().manual_seed(61 + h)
+    top = 4133
+    x = torch.randn(top, h, generator=g).to(dtype)
+    w = [t[0] for t in _weights(g, 1, h, inter, dtype)]
+    xd, wd = x.to(dev), [t.to(dev) for t in w]
+    sh = SharedExperts(*wd) if packed else None
+    run = lambda m: sh.forward(xd[:m]).clone() if packed else expert_swiglu(xd[:m], *wd)  # noqa: E731
+    full = run(top)
+    torch.cuda.synchronize()
+    want, _ = O.swiglu_expert(np64(x[:40]), *(np64(t) for t in w), ODT[dtype])
+    assert_mlp_close(np64(full[:40]), want, dtype)
+    for m in (1, 2, 16, 17, 32, 33, 64, 65, 127, 128, 129, 192, 193, 255, 256, 257, 500, 1025, 2049):
+        assert torch.equal(run(m), full[:m]), m
+
+
+@pytest.mark.parametrize("n,k,e,h,inter", [(1, 8, 128, 2048, 768), (64, 6, 64, 2560, 1536), (65, 8, 16, 384, 256),
+                                           (300, 8, 4, 256, 128), (900, 2, 3, 128, 384)])
+def test_grouped_rows_equal_dense_rows(hip_device, n, k, e, h, inter):
+    """Grouped rows, packed and plain, whatever the rows per expert (a row or
+    two each; experts of one and of several 256-row tiles, experts without a
+    row, ids out of range), equal the dense call of the same rows bit for
+    bit; slots that are not recomputed keep their contents."""
+    from table_moe.ops import GroupedExperts, expert_swiglu
+
+    dev = hip_device
+    g = torch.Generator().manual_seed(71 + n)
+    x = torch.randn(n, h, generator=g).to(torch.bfloat16).to(dev)
+    ws = [t.to(dev) for t in _weights(g, e, h, inter, torch.bfloat16)]
+    ids = torch.randint(0, e, (n, k), generator=g)
+    if n > 8:
+        ids[:, 0] = 0  # one expert with many rows
+        ids[3, 1], ids[4, 1] = -1, e
+    mask = torch.rand(n, k, generator=g) < 0.7
+    mask[0, 0] = True
+    for packed in (True, False):
+        slot = torch.full((n, k, h), 5.0, dtype=torch.bfloat16, device=dev)
+        GroupedExperts(*ws, packed=packed).forward(x, ids.to(dev), mask.to(dev), slot)
+        live = mask & (ids >= 0) & (ids < e)
+        assert bool((slot[~live.to(dev)] == 5.0).all())
+        for ex in range(e):
+            b, s = torch.where(live & (ids == ex))
+            if b.numel():
+                y = expert_swiglu(x[b.to(dev)].contiguous(), *(w[ex] for w in ws))
+                assert torch.equal(y, slot[b.to(dev), s.to(dev)]), (packed, ex)
