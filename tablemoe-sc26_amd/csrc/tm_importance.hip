@@ -9,115 +9,216 @@
 // keys excluded, the last query_length keys kept).  Its output feeds
 // tm_expert_keep_mask (the reference's build_prefill_keep_mask).
 //
-// Two launches.  scores_kernel: one workgroup per (512-key chunk, head,
-// batch row); 8 lanes per key (each lane a D / 8 slice, fp32 products summed
-// in lane order, then an 8-lane DPP tree), the chunk's scores to the
-// workspace and its softmax statistics (max m_c, l_c = sum exp(s - m_c)).
-// Chunk c of head h gets block id c + n_chunks * h, and the heads that share a
-// KV head are consecutive, so with 8 chunks the KV chunk they read lands on one
-// XCD.  mean_kernel: one thread per output key; per head, M = max_c m_c and
-// L = sum_c l_c exp(m_c - M), p = exp(s - M) / L, then the heads' p summed in
-// head order and divided by the head count.
+// Two launches.  scores_kernel: one workgroup per (key chunk, set of HG heads
+// that share a KV head, batch row); 8 lanes per key (each lane a D / 8 slice,
+// fp32 products summed in lane order, then an 8-lane DPP tree), every key read
+// once for the set's heads; the chunk's scores to the workspace and each
+// head's softmax statistics (max m_c, l_c = sum exp(s - m_c)).  mean_kernel: 64
+// output keys per workgroup, a quarter of the heads per thread; per head, M =
+// max_c m_c and L = sum_c l_c exp(m_c - M), p = exp(s - M) / L, then the p of
+// each quarter summed in head order, the quarters in order, and divided by the
+// head count.
+//
+// Both are chains of a few memory round trips, so what counts is how many
+// workgroups share them: chunks of 64 keys (260 workgroups at 4099 keys of 4
+// KV heads) instead of 512, and 64 keys x 4 head quarters instead of 256 keys
+// x all heads (65 workgroups instead of 17).  Chunks of 512 keys stay for long
+// prompts, whose statistics every workgroup of the mean reads.  4099 keys, 32
+// heads on 4 KV heads (us): 14.8 + 16.3 before, 5.9 + 6.0 now.
 #include "tm_internal.h"
 #include "tm_route_dev.h"
 
+#include <type_traits>
+
 namespace {
 
-constexpr int kChunk = 512;    // keys per workgroup of scores_kernel
 constexpr int kThreads = 256;  // 32 keys per pass (8 lanes each)
 constexpr int kMaxHeads = 256;
 constexpr int kMaxChunks = 1024;
+constexpr int kShortKeys = 16384;  // up to here chunks of 64 keys, then of 512
+constexpr int kMaxKeys = 512 * kMaxChunks;
+constexpr int kMeanKeys = 64;      // output keys per workgroup of mean_kernel
+constexpr int kBatch = 8;          // scores and statistics loaded per round trip
 
-template <int DT, int CH>
+inline int chunk_keys(int64_t n_keys) { return n_keys <= kShortKeys ? 64 : 512; }
+
+// Maximum / sum over the wave in every lane (DPP: row shifts, row broadcasts).
+__device__ __forceinline__ float wave_max_f(float v) {
+  auto st = [&](auto c) {
+    v = fmaxf(v, __uint_as_float(tm_dpp<decltype(c)::value>(__float_as_uint(v), __float_as_uint(v))));
+  };
+  st(std::integral_constant<int, 0x111>{});
+  st(std::integral_constant<int, 0x112>{});
+  st(std::integral_constant<int, 0x114>{});
+  st(std::integral_constant<int, 0x118>{});
+  v = fmaxf(v, __uint_as_float(tm_dpp<0x142, 0xA>(__float_as_uint(v), __float_as_uint(v))));
+  v = fmaxf(v, __uint_as_float(tm_dpp<0x143, 0xC>(__float_as_uint(v), __float_as_uint(v))));
+  return __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(v), 63));
+}
+__device__ __forceinline__ float wave_sum_f(float v) {
+  auto st = [&](auto c) { v += __uint_as_float(tm_dpp<decltype(c)::value>(0u, __float_as_uint(v))); };
+  st(std::integral_constant<int, 0x111>{});
+  st(std::integral_constant<int, 0x112>{});
+  st(std::integral_constant<int, 0x114>{});
+  st(std::integral_constant<int, 0x118>{});
+  v += __uint_as_float(tm_dpp<0x142, 0xA>(0u, __float_as_uint(v)));
+  v += __uint_as_float(tm_dpp<0x143, 0xC>(0u, __float_as_uint(v)));
+  return __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(v), 63));
+}
+
+template <int DT, int CH, int HG, int PASSES>
 __global__ __launch_bounds__(kThreads) void scores_kernel(
     const typename Elem<DT>::T *__restrict__ q, int64_t qs_b, int64_t qs_h, const typename Elem<DT>::T *__restrict__ k,
     int64_t ks_b, int64_t ks_s, int64_t ks_h, int n_heads, int groups, int64_t n_keys, float scale, int score_mode,
     const uint8_t *__restrict__ key_mask, int64_t km_b, float *__restrict__ sc, float2 *__restrict__ stats) {
   using T = typename Elem<DT>::T;
+  constexpr int kChunk = 32 * PASSES;
+  constexpr int kAhead = PASSES < 4 ? PASSES : 4;  // passes whose keys are in flight together
   // head dim 64 * CH: lane `sub` of a key's 8 lanes holds chunks sub, sub + 8, ... (8 elements each)
-  const int c = (int)blockIdx.x, h = (int)blockIdx.y;
+  const int c = (int)blockIdx.x, h0 = (int)blockIdx.y * HG;
   const int64_t b = blockIdx.z;
   const int tid = threadIdx.x, sub = tid & 7, grp = tid >> 3;
-  const int kvh = h / groups;
-  float qv[CH][8];
-#pragma unroll
-  for (int j = 0; j < CH; ++j) tm_load8<DT>(q + b * qs_b + (int64_t)h * qs_h + (j * 8 + sub) * 8, qv[j]);
-
-  __shared__ float red_m[kThreads / 64], red_l[kThreads / 64];
-  float m = -__builtin_huge_valf();
-  float sv[kChunk / 32];
-  bool ok[kChunk / 32];
+  __shared__ float tile[HG][kChunk];
   const int64_t t0 = (int64_t)c * kChunk;
+  const T *const kb = k + b * ks_b + (int64_t)(h0 / groups) * ks_h;
+  float qv[HG][CH][8];
 #pragma unroll
-  for (int it = 0; it < kChunk / 32; ++it) {
-    const int64_t t = t0 + it * 32 + grp;
-    const int64_t tc = t < n_keys ? t : n_keys - 1;
-    const T *kr = k + b * ks_b + tc * ks_s + (int64_t)kvh * ks_h;
-    float acc = 0.f;
+  for (int h = 0; h < HG; ++h)
 #pragma unroll
-    for (int j = 0; j < CH; ++j) {
-      float kv[8];
-      tm_load8<DT>(kr + (j * 8 + sub) * 8, kv);
+    for (int j = 0; j < CH; ++j) tm_load8<DT>(q + b * qs_b + (int64_t)(h0 + h) * qs_h + (j * 8 + sub) * 8, qv[h][j]);
+#pragma unroll 1
+  for (int it0 = 0; it0 < PASSES; it0 += kAhead) {
+    float kv[kAhead][CH][8];
 #pragma unroll
-      for (int i = 0; i < 8; ++i) acc = fmaf(qv[j][i], kv[i], acc);
+    for (int a = 0; a < kAhead; ++a) {
+      const int64_t t = t0 + (it0 + a) * 32 + grp;
+      const T *kr = kb + (t < n_keys ? t : n_keys - 1) * ks_s;
+#pragma unroll
+      for (int j = 0; j < CH; ++j) tm_load8<DT>(kr + (j * 8 + sub) * 8, kv[a][j]);
     }
-    acc += tm_g8f<kG8Steps[0]>(acc);
-    acc += tm_g8f<kG8Steps[1]>(acc);
-    acc += tm_g8f<kG8Steps[2]>(acc);
-    const float s = score_mode == TM_SCORE_MODEL ? tm_round<DT>(tm_round<DT>(acc) * scale) : acc * scale;
-    const bool valid = t < n_keys && (key_mask == nullptr || key_mask[b * km_b + tc] != 0);
-    sv[it] = s;
-    ok[it] = valid;
-    m = valid ? fmaxf(m, s) : m;
-    if (sub == 0 && t < n_keys) sc[(b * n_heads + h) * n_keys + t] = s;
-  }
-  // chunk max, then the sum of exp(s - max) over the valid keys
-  m = tm_wave_max(m);
-  if ((tid & 63) == 0) red_m[tid >> 6] = m;
-  __syncthreads();
-  m = fmaxf(fmaxf(red_m[0], red_m[1]), fmaxf(red_m[2], red_m[3]));
-  float l = 0.f;
-  if (sub == 0) {
 #pragma unroll
-    for (int it = 0; it < kChunk / 32; ++it) l += ok[it] ? expf(sv[it] - m) : 0.f;
+    for (int a = 0; a < kAhead; ++a)
+#pragma unroll
+      for (int h = 0; h < HG; ++h) {
+        float acc = 0.f;
+#pragma unroll
+        for (int j = 0; j < CH; ++j)
+#pragma unroll
+          for (int i = 0; i < 8; ++i) acc = fmaf(qv[h][j][i], kv[a][j][i], acc);
+        acc += tm_g8f<kG8Steps[0]>(acc);
+        acc += tm_g8f<kG8Steps[1]>(acc);
+        acc += tm_g8f<kG8Steps[2]>(acc);
+        const float s = score_mode == TM_SCORE_MODEL ? tm_round<DT>(tm_round<DT>(acc) * scale) : acc * scale;
+        if (sub == (h & 7)) tile[h][(it0 + a) * 32 + grp] = s;
+      }
   }
-  l = tm_wave_sum(l);
-  if ((tid & 63) == 0) red_l[tid >> 6] = l;
+  // which of this lane's keys count, for the statistics below
+  const int lane = tid & 63, wave = tid >> 6;
+  bool ok[kChunk / 64 > 0 ? kChunk / 64 : 1];
+#pragma unroll
+  for (int i = 0; i < kChunk / 64; ++i) {
+    const int64_t t = t0 + i * 64 + lane;
+    ok[i] = t < n_keys && (key_mask == nullptr || key_mask[b * km_b + (t < n_keys ? t : n_keys - 1)] != 0);
+  }
   __syncthreads();
-  if (tid == 0) {
-    const float lt = ((red_l[0] + red_l[1]) + red_l[2]) + red_l[3];
-    stats[(b * n_heads + h) * gridDim.x + c] = make_float2(m, lt);
+  // a wave per head: the scores out, the chunk's max, then the sum of
+  // exp(s - max) over its valid keys
+  for (int h = wave; h < HG; h += kThreads / 64) {
+    float sv[kChunk / 64];
+    float m = -__builtin_huge_valf();
+#pragma unroll
+    for (int i = 0; i < kChunk / 64; ++i) {
+      sv[i] = tile[h][i * 64 + lane];
+      m = ok[i] ? fmaxf(m, sv[i]) : m;
+      const int64_t t = t0 + i * 64 + lane;
+      if (t < n_keys) sc[(b * n_heads + h0 + h) * n_keys + t] = sv[i];
+    }
+    m = wave_max_f(m);
+    float l = 0.f;
+#pragma unroll
+    for (int i = 0; i < kChunk / 64; ++i) l += ok[i] ? expf(sv[i] - m) : 0.f;
+    l = wave_sum_f(l);
+    if (lane == 0) stats[(b * n_heads + h0 + h) * gridDim.x + c] = make_float2(m, l);
   }
 }
 
 __global__ __launch_bounds__(kThreads) void mean_kernel(const float *__restrict__ sc, const float2 *__restrict__ stats,
-                                                       int n_heads, int n_chunks, int64_t n_keys,
+                                                       int n_heads, int lanes_log2, int n_chunks, int64_t n_keys,
                                                        const uint8_t *__restrict__ key_mask, int64_t km_b,
                                                        int64_t out_len, float *__restrict__ out, int64_t ld_out) {
   __shared__ float hm[kMaxHeads], hl[kMaxHeads];
+  __shared__ float part[kThreads / kMeanKeys][kMeanKeys];
   const int64_t b = blockIdx.y;
   const int tid = threadIdx.x;
-  for (int h = tid; h < n_heads; h += kThreads) {  // combine the chunk statistics of head h
-    const float2 *st = stats + (b * n_heads + h) * n_chunks;
-    float M = -__builtin_huge_valf();
-    for (int cc = 0; cc < n_chunks; ++cc) M = fmaxf(M, st[cc].x);
-    float L = 0.f;
-    if (M != -__builtin_huge_valf())
-      for (int cc = 0; cc < n_chunks; ++cc) L += st[cc].y * expf(st[cc].x - M);
-    hm[h] = M;
-    hl[h] = L;
+  // thread: output key tid % 64, heads [ha, hb) (a quarter of them); its first
+  // scores are requested before the statistics
+  const int64_t j = (int64_t)blockIdx.x * kMeanKeys + (tid & (kMeanKeys - 1));
+  const int64_t t = n_keys - out_len + (j < out_len ? j : out_len - 1);
+  const int per = (n_heads + 3) / 4, ha = (tid / kMeanKeys) * per;
+  const int hb = ha + per < n_heads ? ha + per : n_heads;
+  const float *const col = sc + b * n_heads * n_keys + t;
+  float s0[kBatch];
+#pragma unroll
+  for (int i = 0; i < kBatch; ++i) s0[i] = col[(int64_t)(ha + i < n_heads ? ha + i : n_heads - 1) * n_keys];
+  const bool valid = key_mask == nullptr || key_mask[b * km_b + t] != 0;
+  // the chunk statistics of head h, combined by 1 << lanes_log2 lanes
+  const int lanes = 1 << lanes_log2, lane = tid & (lanes - 1);
+  for (int hbase = 0; hbase < n_heads; hbase += kThreads >> lanes_log2) {
+    const int h = hbase + (tid >> lanes_log2);
+    const float2 *st = stats + (b * n_heads + (h < n_heads ? h : n_heads - 1)) * n_chunks;
+    float M = -__builtin_huge_valf(), L = 0.f;
+    for (int c0 = lane; c0 < n_chunks; c0 += lanes * kBatch) {
+      float2 v[kBatch];
+      float m = M;
+#pragma unroll
+      for (int i = 0; i < kBatch; ++i) {
+        const int cc = c0 + i * lanes;
+        v[i] = st[cc < n_chunks ? cc : n_chunks - 1];
+        if (cc >= n_chunks) v[i] = make_float2(-__builtin_huge_valf(), 0.f);
+        m = fmaxf(m, v[i].x);
+      }
+      if (m != -__builtin_huge_valf()) {
+        L *= M == -__builtin_huge_valf() ? 0.f : expf(M - m);
+#pragma unroll
+        for (int i = 0; i < kBatch; ++i) L += v[i].y == 0.f ? 0.f : v[i].y * expf(v[i].x - m);
+        M = m;
+      }
+    }
+    for (int o = 1; o < lanes; o <<= 1) {
+      const float om = __shfl_xor(M, o, 64), ol = __shfl_xor(L, o, 64);
+      const float m = fmaxf(M, om);
+      if (m != -__builtin_huge_valf()) {
+        L = (M == -__builtin_huge_valf() ? 0.f : L * expf(M - m)) + (om == -__builtin_huge_valf() ? 0.f : ol * expf(om - m));
+        M = m;
+      }
+    }
+    if (lane == 0 && h < n_heads) {
+      hm[h] = M;
+      hl[h] = L;
+    }
   }
   __syncthreads();
-  const int64_t j = (int64_t)blockIdx.x * kThreads + tid;
-  if (j >= out_len) return;
-  const int64_t t = n_keys - out_len + j;
-  const bool valid = key_mask == nullptr || key_mask[b * km_b + t] != 0;
   float acc = 0.f;
-  for (int h = 0; h < n_heads; ++h) {
-    const float s = sc[(b * n_heads + h) * n_keys + t];
-    acc += (valid && hl[h] > 0.f) ? expf(s - hm[h]) / hl[h] : 0.f;
+  for (int hh = ha; hh < hb; hh += kBatch) {
+    float s1[kBatch];  // the next batch
+#pragma unroll
+    for (int i = 0; i < kBatch; ++i) {
+      const int hn = hh + kBatch + i;
+      s1[i] = hh + kBatch < hb ? col[(int64_t)(hn < n_heads ? hn : n_heads - 1) * n_keys] : 0.f;
+    }
+#pragma unroll
+    for (int i = 0; i < kBatch; ++i) {
+      const int h = hh + i < hb ? hh + i : hb - 1;
+      const float p = expf(s0[i] - hm[h]) / hl[h];
+      acc += (hh + i < hb && valid && hl[h] > 0.f) ? p : 0.f;
+    }
+#pragma unroll
+    for (int i = 0; i < kBatch; ++i) s0[i] = s1[i];
   }
-  out[b * ld_out + j] = acc / (float)n_heads;
+  part[tid / kMeanKeys][tid & (kMeanKeys - 1)] = acc;
+  __syncthreads();
+  if (tid < kMeanKeys && j < out_len)
+    out[b * ld_out + j] = (((part[0][tid] + part[1][tid]) + part[2][tid]) + part[3][tid]) / (float)n_heads;
 }
 
 template <int DT, int CH>
@@ -125,10 +226,23 @@ void launch_scores(const void *q, int64_t qs_b, int64_t qs_h, const void *k, int
                    int64_t batch, int n_heads, int groups, int64_t n_keys, float scale, int score_mode,
                    const uint8_t *key_mask, int64_t km_b, float *sc, float2 *stats, hipStream_t s) {
   using T = typename Elem<DT>::T;
-  const dim3 grid((unsigned)tm_cdiv(n_keys, kChunk), (unsigned)n_heads, (unsigned)batch);
-  hipLaunchKernelGGL((scores_kernel<DT, CH>), grid, dim3(kThreads), 0, s, static_cast<const T *>(q), qs_b, qs_h,
-                     static_cast<const T *>(k), ks_b, ks_s, ks_h, n_heads, groups, n_keys, scale, score_mode,
-                     key_mask, km_b, sc, stats);
+  const int chunk = chunk_keys(n_keys);
+  auto launch = [&](auto hg_c, auto passes_c) {
+    constexpr int HG = decltype(hg_c)::value, PASSES = decltype(passes_c)::value;
+    const dim3 grid((unsigned)tm_cdiv(n_keys, chunk), (unsigned)(n_heads / HG), (unsigned)batch);
+    hipLaunchKernelGGL((scores_kernel<DT, CH, HG, PASSES>), grid, dim3(kThreads), 0, s, static_cast<const T *>(q),
+                       qs_b, qs_h, static_cast<const T *>(k), ks_b, ks_s, ks_h, n_heads, groups, n_keys, scale,
+                       score_mode, key_mask, km_b, sc, stats);
+  };
+  auto heads = [&](auto hg_c) {
+    if (chunk == 64) launch(hg_c, std::integral_constant<int, 2>{});
+    else launch(hg_c, std::integral_constant<int, 16>{});
+  };
+  // heads per workgroup: as many of a KV head's as the registers hold
+  if (CH <= 2 && groups % 8 == 0) heads(std::integral_constant<int, CH <= 2 ? 8 : 4>{});
+  else if (groups % 4 == 0) heads(std::integral_constant<int, 4>{});
+  else if (groups % 2 == 0) heads(std::integral_constant<int, 2>{});
+  else heads(std::integral_constant<int, 1>{});
 }
 
 }  // namespace
@@ -136,7 +250,7 @@ void launch_scores(const void *q, int64_t qs_b, int64_t qs_h, const void *k, int
 extern "C" size_t tm_importance_workspace_size(int64_t batch, int32_t n_heads, int64_t n_keys) {
   if (batch <= 0 || n_heads <= 0 || n_keys <= 0) return 0;
   const size_t scores = (size_t)batch * n_heads * n_keys * sizeof(float);
-  const size_t stats = (size_t)batch * n_heads * tm_cdiv(n_keys, kChunk) * sizeof(float2);
+  const size_t stats = (size_t)batch * n_heads * tm_cdiv(n_keys, chunk_keys(n_keys)) * sizeof(float2);
   return (scores + 255) / 256 * 256 + stats;
 }
 
@@ -147,10 +261,10 @@ extern "C" int tm_last_query_importance(int32_t dtype, const void *q, int64_t qs
                                         float *out, int64_t ld_out, void *workspace, size_t workspace_bytes,
                                         tm_stream_t stream) {
   TM_REQUIRE(batch >= 0 && n_heads >= 1 && n_heads <= kMaxHeads && n_kv_heads >= 1 && n_heads % n_kv_heads == 0 &&
-                 n_keys >= 0 && tm_cdiv(n_keys, kChunk) <= kMaxChunks && out_len >= 0 && out_len <= n_keys &&
+                 n_keys >= 0 && n_keys <= kMaxKeys && out_len >= 0 && out_len <= n_keys &&
                  ld_out >= out_len && batch < 65536,
              TM_EINVAL_SHAPE, "tm_last_query_importance: bad sizes (heads <= %d, keys <= %d)", kMaxHeads,
-             kMaxChunks * kChunk);
+             kMaxKeys);
   TM_REQUIRE(head_dim == 64 || head_dim == 128 || head_dim == 192 || head_dim == 256, TM_EINVAL_SHAPE,
              "tm_last_query_importance: head_dim %d not in {64, 128, 192, 256}", head_dim);
   TM_REQUIRE(score_mode == TM_SCORE_MODEL || score_mode == TM_SCORE_F32, TM_EINVAL_ARG,
@@ -180,9 +294,11 @@ extern "C" int tm_last_query_importance(int32_t dtype, const void *q, int64_t qs
       default: launch_scores<DT, 4>(q, qs_b, qs_h, k, ks_b, ks_s, ks_h, batch, n_heads, groups, n_keys, scale, score_mode, key_mask, km_b, sc, stats, s); break;
     }
     TM_LAUNCH_CHECK("tm_last_query_importance(scores)");
-    hipLaunchKernelGGL(mean_kernel, dim3((unsigned)tm_cdiv(out_len, kThreads), (unsigned)batch), dim3(kThreads), 0,
-                       s, sc, stats, (int)n_heads, (int)tm_cdiv(n_keys, kChunk), n_keys, key_mask, km_b, out_len, out,
-                       ld_out);
+    int lanes_log2 = 0;  // lanes per head that combine its chunk statistics
+    while (lanes_log2 < 6 && (kThreads >> (lanes_log2 + 1)) >= n_heads) ++lanes_log2;
+    hipLaunchKernelGGL(mean_kernel, dim3((unsigned)tm_cdiv(out_len, kMeanKeys), (unsigned)batch), dim3(kThreads), 0, s,
+                       sc, stats, (int)n_heads, lanes_log2, (int)tm_cdiv(n_keys, chunk_keys(n_keys)), n_keys, key_mask,
+                       km_b, out_len, out, ld_out);
     TM_LAUNCH_CHECK("tm_last_query_importance(mean)");
     return TM_OK;
   });

@@ -76,3 +76,26 @@ def test_importance_feeds_expert_keep_mask(hip_device):
     torch.cuda.synchronize()
     want, _ = O.build_prefill_keep_mask(sel.numpy(), np64(w), np64(attn), e, 0.6)
     np.testing.assert_array_equal(mask.cpu().numpy(), want)
+
+
+@pytest.mark.parametrize("b,h,hkv,d,s,out_len", [(1, 8, 1, 128, 1, 1), (1, 3, 3, 64, 63, 63), (2, 16, 2, 128, 65, 40),
+                                                 (1, 12, 3, 192, 129, 129), (1, 40, 20, 256, 600, 577),
+                                                 (1, 16, 1, 64, 16384, 16384), (1, 8, 4, 128, 16449, 16449),
+                                                 (1, 64, 64, 64, 700, 1)])
+def test_importance_key_chunks_and_head_sets(hip_device, b, h, hkv, d, s, out_len):
+    """Chunk edges of 64 and of 512 keys (from 16385 on), 1 to 16 heads per KV
+    head, masked keys (a whole chunk of them too) and a shorter output."""
+    from table_moe.utils.importance import last_query_importance
+
+    g = torch.Generator().manual_seed(s + 7 * h)
+    q = torch.randn(b, h, d, generator=g).to(torch.bfloat16)
+    ks = torch.randn(b, s, hkv, d, generator=g).to(torch.bfloat16)
+    mask = torch.rand(b, s, generator=g) < 0.9
+    mask[:, -1] = True
+    if s > 200:
+        mask[:, 64:192] = False
+    dev = hip_device
+    got = last_query_importance(q.to(dev), ks.to(dev), hkv, d ** -0.5, True, mask.to(dev), out_len)
+    torch.cuda.synchronize()
+    want = O.last_query_importance(np64(q), np64(ks), hkv, d ** -0.5, O.F32, key_mask=mask.numpy(), out_len=out_len)
+    np.testing.assert_allclose(np64(got), want, rtol=1e-4, atol=1e-9)
