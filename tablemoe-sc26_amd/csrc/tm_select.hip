@@ -155,14 +155,188 @@ __global__ __launch_bounds__(kSelThreads) void keep_select_kernel(const float *_
 }
 
 // ---------------------------------------------------------------------------
-// (3), fast form for n <= kSelThreads * kKeepRegs: same result as
-// keep_select_kernel (tm_keep_select_fast in one 1024-thread workgroup).
+// (3) for n <= kSelThreads * 16: same result as keep_select_kernel, over many
+// workgroups that share nothing.  Every workgroup reads all n scores (thread t
+// holds scores t, t + 1024, .. as order-preserving keys, R of them, all loads
+// in flight together), counts them in a 4096-bin LDS histogram over the range
+// that they span, finds the bin the n_keep-th largest falls in with one block
+// scan, and lists that bin's keys; it decides only its own kKeepTok tokens
+// (8 threads each count the listed keys ahead of theirs: larger, or equal at a
+// lower index).  With ks.keys set the scores are decoded from packed top-1
+// search keys and a workgroup also writes its tokens' distance, centroid and
+// |q|^2.
+//
+// One workgroup for all tokens was bound by the single CU that read every key
+// and wrote every result (12301 tokens: 32.5 us, 1531: 9.2 us, in the layer
+// call); reading all scores once per 128 tokens from L2 is cheaper than a
+// second launch or a hand-off (11.4 and 4.6 us now).
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(kSelThreads) void keep_select_fast_kernel(const float *__restrict__ score, int64_t n,
-                                                                       int64_t ld, int64_t n_keep,
-                                                                       uint8_t *__restrict__ out, KeySrc ks) {
-  __shared__ KeepSmem<kSelThreads> sm;
-  tm_keep_select_fast<kSelThreads>(score, n, ld, n_keep, out, ks, sm);
+constexpr int kKeepTok = 128;
+constexpr int kKeepMost = 16;  // scores per thread
+constexpr int kKeepBins = 4096;
+static_assert(kSelThreads % kKeepTok == 0 && kSelThreads == 8 * kKeepTok && kKeepBins == 4 * kSelThreads, "shape");
+
+// Sum over the wave of `v` (one LDS read per wave when `v` comes from shared
+// memory, then DPP).
+__device__ __forceinline__ uint32_t wave_sum_u32(uint32_t v) {
+  return (uint32_t)__builtin_amdgcn_readlane((int)tm_wave_incl_scan(v), 63);
+}
+
+template <int R>
+__global__ __launch_bounds__(kSelThreads) void keep_rank_kernel(const float *__restrict__ score, int64_t n, int64_t ld,
+                                                                int64_t n_keep, uint8_t *__restrict__ out, KeySrc ks) {
+  constexpr int NW = kSelWaves;
+  __shared__ __align__(16) uint32_t hist[kKeepBins];
+  __shared__ uint32_t m_key[R * kSelThreads];
+  __shared__ uint16_t m_idx[R * kSelThreads];
+  __shared__ uint32_t own_key[kKeepTok];
+  __shared__ uint32_t wave_tot[NW], s_min[NW], s_max[NW];
+  __shared__ uint2 s_sel;  // boundary bin, keys still to keep in it
+  __shared__ uint32_t s_members;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int i0 = (int)blockIdx.x * kKeepTok;  // this workgroup's tokens
+  const int own_r = i0 / kSelThreads, own_t = i0 % kSelThreads;
+  const bool is_own = tid >= own_t && tid < own_t + kKeepTok;
+  uint32_t key[R];
+  if (ks.keys != nullptr) {  // uniform
+    constexpr int RB = R < 8 ? R : 8;  // keys per round trip (the registers of 16 would spill)
+#pragma unroll
+    for (int r0 = 0; r0 < R; r0 += RB) {
+      uint64_t kv[RB];
+      float qp[RB][4];
+#pragma unroll
+      for (int u = 0; u < RB; ++u) {
+        const int64_t j = (r0 + u) * kSelThreads + tid < n ? (r0 + u) * kSelThreads + tid : n - 1;
+        kv[u] = ks.keys[j];
+#pragma unroll
+        for (int p = 0; p < 4; ++p) qp[u][p] = ks.qn_part[(p < ks.parts ? p : 0) * n + j];
+      }
+#pragma unroll
+      for (int u = 0; u < RB; ++u) {
+        const int64_t j = (r0 + u) * kSelThreads + tid;
+        const float qn = qn_sum(qp[u][0], qp[u][1], qp[u][2], qp[u][3], ks.parts);
+        int64_t ix;
+        const float d = tm_key_to_dist(kv[u], qn, ks.l2 != 0, ix);
+        key[r0 + u] = tm_orderable(d);
+        if (r0 + u == own_r && is_own && j < n) {
+          ks.out_dist[j] = d;
+          ks.out_idx[j] = ix;
+          ks.out_qn[j] = qn;
+        }
+      }
+    }
+  } else {
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const int64_t j = r * kSelThreads + tid < n ? r * kSelThreads + tid : n - 1;
+      key[r] = tm_orderable(score[j * ld]);
+    }
+  }
+  if (n_keep <= 0 || n_keep >= n) {  // uniform
+    if (tid < kKeepTok && i0 + tid < n) out[i0 + tid] = n_keep > 0 ? 1 : 0;
+    return;
+  }
+  if (n <= 64) {  // uniform: one wave ranks the keys directly (no LDS, no barrier)
+    if (wave == 0) {
+      uint32_t rank = 0;  // keys ahead of this one: larger, or equal at a lower index
+      for (int j = 0; j < (int)n; ++j) {
+        const uint32_t kj = (uint32_t)__builtin_amdgcn_readlane((int)key[0], j);
+        rank += (kj > key[0] || (kj == key[0] && j < lane)) ? 1u : 0u;
+      }
+      if (lane < n) out[lane] = rank < (uint32_t)n_keep ? 1 : 0;
+    }
+    return;
+  }
+  *reinterpret_cast<uint4 *>(&hist[4 * tid]) = make_uint4(0, 0, 0, 0);
+  if (tid == 0) s_members = 0;
+  // scores past n repeat the last one, so they do not move the range
+  uint32_t kmin = key[0], kmax = key[0];
+#pragma unroll
+  for (int r = 1; r < R; ++r) {
+    kmin = min(kmin, key[r]);
+    kmax = max(kmax, key[r]);
+  }
+  kmin = tm_wave_min_u32(kmin);
+  kmax = tm_wave_max_u32(kmax);
+  if (lane == 0) {
+    s_min[wave] = kmin;
+    s_max[wave] = kmax;
+  }
+#pragma unroll
+  for (int r = 0; r < R; ++r)
+    if (r == own_r && is_own) own_key[tid - own_t] = key[r];
+  __syncthreads();
+  kmin = tm_wave_min_u32(lane < NW ? s_min[lane] : 0xffffffffu);
+  kmax = tm_wave_max_u32(lane < NW ? s_max[lane] : 0u);
+  const uint32_t span = kmax - kmin;
+  const int width = span ? 32 - __builtin_clz(span) : 0;
+  const int shift = width > 12 ? width - 12 : 0;
+#pragma unroll
+  for (int r = 0; r < R; ++r)
+    if (r * kSelThreads + tid < n) atomicAdd(&hist[(key[r] - kmin) >> shift], 1u);
+  __syncthreads();
+  // thread t owns the 4 bins of rank 1023 - t (descending bin order across threads)
+  const int rank4 = kSelThreads - 1 - tid;
+  const uint4 h4 = *reinterpret_cast<const uint4 *>(&hist[4 * rank4]);
+  const uint32_t hb[4] = {h4.x, h4.y, h4.z, h4.w};
+  const uint32_t tsum = hb[0] + hb[1] + hb[2] + hb[3];
+  const uint32_t inc = tm_wave_incl_scan(tsum);
+  if (lane == 63) wave_tot[wave] = inc;
+  __syncthreads();
+  uint32_t above = wave_sum_u32(lane < wave ? wave_tot[lane] : 0u) + inc - tsum;  // keys in higher bins
+  const uint32_t want = (uint32_t)n_keep;
+#pragma unroll
+  for (int b = 3; b >= 0; --b) {
+    if (above < want && want <= above + hb[b]) s_sel = make_uint2((uint32_t)(4 * rank4 + b), want - above);
+    above += hb[b];
+  }
+  __syncthreads();
+  const uint2 sel = s_sel;
+  // list the keys of the boundary bin (one LDS atomic per wave and register)
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const bool in = r * kSelThreads + tid < n && ((key[r] - kmin) >> shift) == sel.x;
+    const uint64_t who = __ballot(in);
+    if (who != 0) {  // uniform
+      uint32_t base = 0;
+      if (lane == 0) base = atomicAdd(&s_members, (uint32_t)__popcll(who));
+      base = (uint32_t)__builtin_amdgcn_readfirstlane((int)base);
+      if (in) {
+        const uint32_t at = base + (uint32_t)__popcll(who & ((1ull << lane) - 1));
+        m_key[at] = key[r];
+        m_idx[at] = (uint16_t)(r * kSelThreads + tid);
+      }
+    }
+  }
+  __syncthreads();
+  const int tok = tid >> 3, sub = tid & 7, i = i0 + tok;
+  const uint32_t mine = own_key[tok];  // (a token past n: any value, not written)
+  const uint32_t bin = (mine - kmin) >> shift;
+  uint32_t ahead = 0;
+  if (bin == sel.x) {
+    const uint32_t members = s_members;
+    for (uint32_t m = (uint32_t)sub; m < members; m += 8) {
+      const uint32_t k = m_key[m];
+      ahead += (k > mine || (k == mine && (int)m_idx[m] < i)) ? 1u : 0u;
+    }
+  }
+  ahead += (uint32_t)__shfl_xor((int)ahead, 1, 64);
+  ahead += (uint32_t)__shfl_xor((int)ahead, 2, 64);
+  ahead += (uint32_t)__shfl_xor((int)ahead, 4, 64);
+  if (sub == 0 && i < n) out[i] = bin > sel.x || (bin == sel.x && ahead < sel.y) ? 1 : 0;
+}
+
+void launch_keep_rank(const float *score, int64_t n, int64_t ld, int64_t n_keep, uint8_t *out, const KeySrc &ks,
+                      hipStream_t s) {
+  const dim3 grid((unsigned)tm_cdiv(n, kKeepTok)), block(kSelThreads);
+  if (n <= 2 * kSelThreads)
+    hipLaunchKernelGGL(keep_rank_kernel<2>, grid, block, 0, s, score, n, ld, n_keep, out, ks);
+  else if (n <= 4 * kSelThreads)
+    hipLaunchKernelGGL(keep_rank_kernel<4>, grid, block, 0, s, score, n, ld, n_keep, out, ks);
+  else if (n <= 8 * kSelThreads)
+    hipLaunchKernelGGL(keep_rank_kernel<8>, grid, block, 0, s, score, n, ld, n_keep, out, ks);
+  else
+    hipLaunchKernelGGL(keep_rank_kernel<kKeepMost>, grid, block, 0, s, score, n, ld, n_keep, out, ks);
 }
 
 // ---------------------------------------------------------------------------
@@ -405,9 +579,8 @@ extern "C" int tm_keep_select(const float *score, int64_t n, int64_t ld_score, i
              "tm_keep_select: bad sizes n=%lld", (long long)n);
   if (n == 0) return TM_OK;
   TM_REQUIRE(score && out_keep, TM_EINVAL_ARG, "tm_keep_select: null pointer");
-  if (n <= (int64_t)kSelThreads * kKeepRegs)
-    hipLaunchKernelGGL(keep_select_fast_kernel, dim3(1), dim3(kSelThreads), 0, tm_hip_stream(stream),
-                       score, n, ld_score, n_keep, out_keep, KeySrc{});
+  if (n <= (int64_t)kSelThreads * kKeepMost)
+    launch_keep_rank(score, n, ld_score, n_keep, out_keep, KeySrc{}, tm_hip_stream(stream));
   else
     hipLaunchKernelGGL(keep_select_kernel, dim3(1), dim3(kSelThreads), 0, tm_hip_stream(stream),
                        score, n, ld_score, n_keep, out_keep);
@@ -485,7 +658,7 @@ extern "C" int tm_renormalize(int32_t dtype, const void *weights, int64_t ld_w, 
   });
 }
 
-bool tm_internal_keep_keys_ok(int64_t n) { return n > 0 && n <= (int64_t)kSelThreads * kKeepRegs; }
+bool tm_internal_keep_keys_ok(int64_t n) { return n > 0 && n <= (int64_t)kSelThreads * kKeepMost; }
 
 int tm_internal_keep_keys(const uint64_t *keys, const float *qn_part, int32_t parts, int32_t metric, int64_t n,
                           int64_t n_keep, float *out_dist, int64_t *out_idx, float *out_qn, uint8_t *out_keep,
@@ -496,8 +669,7 @@ int tm_internal_keep_keys(const uint64_t *keys, const float *qn_part, int32_t pa
                  tm_aligned16(qn_part),
              TM_EINVAL_ARG, "tm_table_forward: keep select from keys: bad buffers");
   const KeySrc ks{keys, qn_part, parts, metric == TM_METRIC_L2 ? 1 : 0, out_dist, out_idx, out_qn};
-  hipLaunchKernelGGL(keep_select_fast_kernel, dim3(1), dim3(kSelThreads), 0, stream, nullptr, n, (int64_t)1,
-                     n_keep, out_keep, ks);
+  launch_keep_rank(nullptr, n, 1, n_keep, out_keep, ks, stream);
   TM_LAUNCH_CHECK("tm_table_forward(keep)");
   return TM_OK;
 }

@@ -537,3 +537,22 @@ def test_keep_select_exact(hip_device, n, pattern):
         torch.cuda.synchronize()
         want = O.keep_select(np64(s), n_keep)
         np.testing.assert_array_equal(np64(keep), want, err_msg=f"n={n} n_keep={n_keep}")
+
+
+@pytest.mark.parametrize("n", [63, 64, 65, 127, 128, 129, 2048, 2049, 4097, 8192, 8193, 12301, 16383])
+def test_keep_select_block_edges(hip_device, n):
+    """Edges of the token blocks and of the scores per thread, with a cluster
+    that falls into one histogram bin (half of the scores, repeated values
+    among them) beside a few far ones."""
+    g = _gen(77 + n)
+    s = torch.rand(n, generator=g) * 1e4
+    s[n // 4: n // 4 + n // 2] = 50.0 + torch.randint(0, 9, (n // 2,), generator=g).float() * 2.0 ** -12
+    dev = hip_device
+    sd = s.to(dev)
+    keep = torch.empty(n, dtype=torch.bool, device=dev)
+    for n_keep in sorted({1, n // 4, n // 2, n - n // 8, n - 1}):
+        if n_keep < 1:
+            continue
+        N.call("tm_keep_select", sd.data_ptr(), n, 1, n_keep, N.as_u8(keep).data_ptr(), None, 0, N.stream(dev))
+        torch.cuda.synchronize()
+        np.testing.assert_array_equal(np64(keep), O.keep_select(np64(s), n_keep), err_msg=f"n={n} n_keep={n_keep}")
