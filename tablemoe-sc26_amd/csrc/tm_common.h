@@ -238,11 +238,51 @@ __device__ __forceinline__ void tm_wave_argmax(float &v, int &i) {
     if (ov > v || (ov == v && oi < i)) { v = ov; i = oi; }
   }
 }
+// Wave minimum of a 64-bit value, in every lane: DPP exchanges inside each
+// 16-lane row (quad_perm [1,0,3,2], quad_perm [2,3,0,1], row_half_mirror,
+// row_mirror: every lane then holds its row's minimum), then the four row
+// minima read into scalars.  Every lane of the wave must call it.
+template <int CTRL>
+__device__ __forceinline__ uint64_t tm_dpp_min64(uint64_t v) {
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)v, CTRL, 0xF, 0xF, false);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(v >> 32), CTRL, 0xF, 0xF, false);
+  const uint64_t o = ((uint64_t)hi << 32) | lo;
+  return o < v ? o : v;
+}
 __device__ __forceinline__ uint64_t tm_wave_min_u64(uint64_t v) {
+  v = tm_dpp_min64<0xB1>(v);
+  v = tm_dpp_min64<0x4E>(v);
+  v = tm_dpp_min64<0x141>(v);
+  v = tm_dpp_min64<0x140>(v);
+  uint64_t m = ~0ull;
 #pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    uint64_t ov = __shfl_xor(v, o, 64);
-    v = ov < v ? ov : v;
+  for (int r = 0; r < 4; ++r) {
+    const uint64_t x = (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)v, 16 * r) |
+                       ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(v >> 32), 16 * r) << 32);
+    m = x < m ? x : m;
   }
-  return v;
+  return m;
+}
+
+// The K smallest keys of the wave, ascending, in every lane, from each lane's
+// ascending K-list: K rounds of a wave minimum over the lists' heads, the lane
+// that holds it popping its head.  Keys are unique (the centroid index is the
+// low word), so one lane pops; empty entries (~0) pop in every lane holding
+// one and stay ~0.  The same K keys as a merge of all the lists.
+template <int K>
+__device__ __forceinline__ void tm_wave_min_k(uint64_t (&l)[K]) {
+  uint64_t top[K];
+#pragma unroll
+  for (int j = 0; j < K; ++j) {
+    const uint64_t m = tm_wave_min_u64(l[0]);
+    top[j] = m;
+    if (j + 1 < K) {
+      const bool pop = l[0] == m;
+#pragma unroll
+      for (int i = 0; i + 1 < K; ++i) l[i] = pop ? l[i + 1] : l[i];
+      l[K - 1] = pop ? ~0ull : l[K - 1];
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < K; ++j) l[j] = top[j];
 }

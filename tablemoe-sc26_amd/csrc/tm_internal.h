@@ -26,6 +26,13 @@ __attribute__((visibility("hidden"))) int tm_internal_search_route(
     float *out_dist, int64_t *out_idx, void *workspace, size_t workspace_bytes, const tm_route_args *ra,
     hipStream_t stream);
 
+// tm_search_global for top_k > 1 and more than 64 tokens of 16-bit data with
+// |q|^2 as `parts` partial norms qn_part[p][i] (also summed into out_qn).
+__attribute__((visibility("hidden"))) int tm_internal_search_topk(
+    int32_t dtype, const void *q, int64_t n_tokens, int64_t ld_q, const void *cents, int64_t n_cent, int64_t ld_c,
+    const float *c_sqnorm, int32_t dim, int32_t top_k, int32_t metric, const float *qn_part, int32_t parts,
+    float *out_dist, int64_t *out_idx, float *out_qn, void *workspace, size_t workspace_bytes, hipStream_t stream);
+
 // Column-split projection of packed P (no normalisation): q rows plus the
 // partial squared norms qn_part[g][row] of column group g (dim / 64 groups,
 // added in group order by the consumer).  With `keys` set, also resets the

@@ -101,6 +101,17 @@ bool fused_top1_ok(const tm_table_layer *t, const tm_layer_io *io) {
          tm_internal_search_keys_ok(t->dtype, n, t->n_cent, t->ld_c, t->dim, 1) && tm_internal_keep_keys_ok(n);
 }
 
+// Layers of several nearest centroids and more than 64 tokens: the
+// column-split projection (with the router) also serves the top-k search,
+// whose merge adds up the partial norms.
+bool cols_topk_ok(const tm_table_layer *t, const tm_layer_io *io) {
+  return io->n_nearest > 1 && io->n_tokens > 64 && t->dtype != TM_DT_F32 &&
+         tm_internal_project_cols_parts(t->dim, io->n_tokens, t->hidden) >= 1 &&
+         tm_internal_project_cols_parts(t->dim, io->n_tokens, t->hidden) <= 4 &&
+         tm_internal_project_cols_ok(t->dtype, io->x, io->n_tokens, t->hidden, io->ld_x, t->proj_vis, t->bias_vis,
+                                     t->proj_txt, t->bias_txt, t->ps_h, t->ps_d, t->dim, io->q, t->dim);
+}
+
 int record(void *const *events, int i, hipStream_t s) {
   if (events == nullptr || events[i] == nullptr) return TM_OK;
   const hipError_t e = hipEventRecord(reinterpret_cast<hipEvent_t>(events[i]), s);
@@ -180,6 +191,21 @@ int general_stages(const tm_table_layer *t, const tm_layer_io *io, const WsLayou
     return st;
   if ((st = record(ev, 1, s)) != TM_OK) return st;
   const WsPtrs p = ptrs(w, ws);
+  if (cols_topk_ok(t, io)) {
+    float *qn_part = reinterpret_cast<float *>(p.qn_part);
+    if ((st = tm_internal_project_cols(t->dtype, io->x, n, t->hidden, io->ld_x, io->is_vision, t->proj_vis,
+                                       t->bias_vis, t->proj_txt, t->bias_txt, t->ps_h, t->ps_d, t->dim, io->q, t->dim,
+                                       qn_part, nullptr, route_fused ? &ra : nullptr, s)) != TM_OK)
+      return st;
+    if ((st = record(ev, 2, s)) != TM_OK) return st;
+    if ((st = tm_internal_search_topk(t->dtype, io->q, n, t->dim, t->cents, t->n_cent, t->ld_c, t->c_sqnorm, t->dim,
+                                      io->n_nearest, t->metric, qn_part,
+                                      (int32_t)tm_internal_project_cols_parts(t->dim, n, t->hidden), io->dist,
+                                      io->idx, io->q_sqnorm, p.search, w.search, s)) != TM_OK)
+      return st;
+    if ((st = record(ev, 3, s)) != TM_OK) return st;
+    return tm_keep_select(io->dist, n, io->n_nearest, n_keep, io->keep, w.keep ? p.keep : nullptr, w.keep, s);
+  }
   if ((st = tm_project(t->dtype, io->x, n, t->hidden, io->ld_x, io->is_vision, t->proj_vis, t->bias_vis,
                        t->proj_txt, t->bias_txt, t->ps_h, t->ps_d, t->dim, 0, 1e-6f, io->q, t->dim, io->q_sqnorm,
                        w.project ? p.project : nullptr, w.project, s)) != TM_OK)

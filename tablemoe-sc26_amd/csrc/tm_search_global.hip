@@ -138,7 +138,9 @@ SplitPlan plan_split(int64_t n, int64_t c, int dim, int top_k) {
   p.row_blocks = tm_cdiv(n, kTileRows);
   const int64_t rows = dma_rows(dim);
   const int64_t max_split = tm_cdiv(c, rows);
-  int64_t want = tm_cdiv(512, p.row_blocks);  // ~2 workgroups per CU
+  // ~2 workgroups per CU; one for top-k, whose merge reads a list per range
+  // (1531 queries x 16384 centroids: 17.6 us at two, 16.6 at one)
+  int64_t want = tm_cdiv(top_k > 1 ? 256 : 512, p.row_blocks);
   const int64_t min_split = tm_cdiv(c, 2048);  // the penalty array holds 2048 centroids
   if (want < min_split) want = min_split;
   if (want < 1) want = 1;
@@ -216,6 +218,44 @@ __device__ __forceinline__ void block_epilogue(const tm_f32x16 &acc, const float
     const float dp = (METRIC == TM_METRIC_L2) ? fmaf(-2.f, acc[i], pen[i]) : (pen[i] - acc[i]);
     best.push(dp, c);
   }
+}
+
+// The tile kernel's top-k: each lane keeps the K nearest 32-centroid BLOCKS of
+// its query, a block ranked by its nearest centroid (packed key: smallest dp
+// << 32 | first centroid).  The K nearest centroids all lie in those blocks: a
+// centroid in any other block is behind the nearest centroid of each of the K,
+// and blocks are runs of consecutive indices, so equal distances rank blocks
+// as they rank centroids (lower index first).  The merge kernel multiplies the
+// K blocks again and ranks their centroids.  A block costs one minimum over its
+// 16 values per lane, one exchange with the lane that holds the other 16 and
+// one insertion; inserting every centroid into a list costs ~40 VALU operations
+// each (1531 queries x 16384 centroids, four nearest: 40 us, 16 now; the
+// merge, which reads the blocks, 12.7 instead of 7.6).
+template <int K>
+struct BlockBest {
+  uint64_t l[K];
+  __device__ __forceinline__ void init() {
+#pragma unroll
+    for (int j = 0; j < K; ++j) l[j] = ~0ull;
+  }
+  __device__ __forceinline__ void finalize() {}
+  __device__ __forceinline__ void merge_xor(int) {}  // both lanes of a query hold the same list
+};
+
+// Epilogue of one 32x32 block for the K nearest blocks: operands as above.
+template <int K, int METRIC>
+__device__ __forceinline__ void block_epilogue(const tm_f32x16 &acc, const float (&pen)[16], int cbase, int,
+                                               BlockBest<K> &best) {
+  float m = __builtin_huge_valf();
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    const float dp = (METRIC == TM_METRIC_L2) ? fmaf(-2.f, acc[i], pen[i]) : (pen[i] - acc[i]);
+    m = i == 0 ? dp : fminf(m, dp);
+  }
+  const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(m), __float_as_uint(m), false, false);
+  m = fminf(__uint_as_float(sw[0]), __uint_as_float(sw[1]));
+  m = m != m ? __uint_as_float(0x7fc00000u) : m;  // (a block of NaNs ranks last)
+  list_insert<K>(best.l, make_key(m, cbase));
 }
 
 // ---------------------------------------------------------------------------
@@ -311,7 +351,7 @@ __global__ __launch_bounds__(kThreads, 2) void search_dma_kernel(
 #pragma unroll
   for (int u = 0; u < PEN_PER_THREAD; ++u) pen_s[tid + u * kThreads] = pen_v[u];
 
-  Best<K> best[kQS];
+  std::conditional_t<K == 1, Best<K>, BlockBest<K>> best[kQS];
 #pragma unroll
   for (int sl = 0; sl < kQS; ++sl) best[sl].init();
 
@@ -348,7 +388,8 @@ __global__ __launch_bounds__(kThreads, 2) void search_dma_kernel(
         pen[4 * g + 0] = p4.x; pen[4 * g + 1] = p4.y; pen[4 * g + 2] = p4.z; pen[4 * g + 3] = p4.w;
       }
 #pragma unroll
-      for (int sl = 0; sl < kQS; ++sl) block_epilogue<K, METRIC>(acc[sl], pen, (int)(s0 + sub * 32), lane, best[sl]);
+      for (int sl = 0; sl < kQS; ++sl)
+        block_epilogue<K, METRIC>(acc[sl], pen, (int)(s0 + sub * 32), lane, best[sl]);
     }
   };
   for (int s = 0; s < nstage; s += kDmaBufs) {
@@ -1251,6 +1292,136 @@ __global__ __launch_bounds__(kThreads) void merge_kernel(
   }
 }
 
+// Top-k merge of the tile kernel's block lists (see BlockBest): one wave per query
+// merges the sorted lists of the splits, multiplies the K blocks' 32 rows
+// against the query again (the tile kernel's products in its order, so the
+// same bits) and takes the top_k smallest keys.  D of a block has every row in
+// all of the 32 columns (each column is the query), so lane l keeps row
+// 8 (u / 4) + 4 (l / 32) + u % 4, u = l % 16, of block 2 p + (l / 16) % 2 of
+// each pair p.  |q|^2 comes from q_sqnorm, from the projection's partial norms
+// (then also written to out_qn), or is computed.
+struct QueryNorm {
+  const float *q_sqnorm;  // nullable
+  const float *part;      // nullable: [parts][n]
+  int parts;
+  float *out;
+};
+
+template <int DT, int DIM, int K, int METRIC, int RVPL>
+__global__ __launch_bounds__(kThreads) void merge_blocks_kernel(
+    const uint64_t *__restrict__ ws, int64_t n, int64_t nsplit, const typename Elem<DT>::T *__restrict__ q,
+    int64_t ld_q, const typename Elem<DT>::T *__restrict__ cents, int64_t n_cent, int64_t ld_c,
+    const float *__restrict__ c_sqnorm, QueryNorm qs, int top_k, float *__restrict__ out_dist,
+    int64_t *__restrict__ out_idx, MergeRoute mr) {
+  constexpr int KS = DIM / 16;
+  if (merge_route_role<RVPL>(mr, n)) return;
+  const int lane = threadIdx.x & 63;
+  const int64_t r = (int64_t)blockIdx.x * (kThreads / 64) + (threadIdx.x >> 6);
+  if (r >= n) return;  // whole wave exits together
+  float qn = 0.f;
+  if (qs.part != nullptr) {
+    float a[4];
+#pragma unroll
+    for (int p = 0; p < 4; ++p) a[p] = qs.part[(p < qs.parts ? p : 0) * n + r];
+    qn = qn_sum(a[0], a[1], a[2], a[3], qs.parts);
+  } else if (METRIC == TM_METRIC_L2 && qs.q_sqnorm != nullptr) {
+    qn = qs.q_sqnorm[r];
+  }
+  uint4 qf[KS];
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks)
+    qf[ks] = *reinterpret_cast<const uint4 *>(q + r * ld_q + ks * 16 + 8 * (lane >> 5));
+  uint64_t lst[K];
+#pragma unroll
+  for (int j = 0; j < K; ++j) lst[j] = ~0ull;
+  for (int64_t s = lane; s < nsplit; s += 128) {  // two lists per round trip
+    const int64_t s1 = s + 64 < nsplit ? s + 64 : s;
+    const uint64_t *src0 = ws + (s * n + r) * K, *src1 = ws + (s1 * n + r) * K;
+    uint64_t b0[K], b1[K];
+#pragma unroll
+    for (int j = 0; j < K; ++j) {
+      b0[j] = src0[j];
+      b1[j] = src1[j];
+    }
+    merge_min<K>(lst, b0);
+    if (s + 64 < nsplit) merge_min<K>(lst, b1);
+  }
+  tm_wave_min_k<K>(lst);  // block keys are unique (first centroid in the low word); in every lane
+  if (METRIC == TM_METRIC_L2 && qs.q_sqnorm == nullptr && qs.part == nullptr) {
+    for (int j = lane; j < DIM; j += 64) {
+      const float v = Elem<DT>::to_f(q[r * ld_q + j]);
+      qn = fmaf(v, v, qn);
+    }
+    qn = tm_wave_sum(qn);
+  }
+  uint64_t key[K / 2];
+  int base[K];
+  auto load = [&](int first, uint4 (&f)[KS]) __attribute__((always_inline)) {
+    const int64_t row = (int64_t)first + (lane & 31);
+    const auto *src = cents + (row < n_cent ? row : n_cent - 1) * ld_c + 8 * (lane >> 5);
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) f[ks] = *reinterpret_cast<const uint4 *>(src + ks * 16);
+  };
+  auto mul = [&](const uint4 (&f)[KS]) __attribute__((always_inline)) {
+    tm_f32x16 acc = tm_f32x16{};
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) acc = tm_mfma32x32x16<DT>(f[ks], qf[ks], acc);
+    return acc;
+  };
+#pragma unroll
+  for (int j = 0; j < K; ++j) {
+    const uint32_t c0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)lst[j]);
+    base[j] = c0 == 0xffffffffu ? 0 : (int)c0;  // (an empty entry multiplies block 0; its keys are masked)
+  }
+  const int u = lane & 15;
+  const bool odd = (lane >> 4) & 1;
+  auto rank = [&](uint64_t blk, const uint4 (&f0)[KS], const uint4 (&f1)[KS]) __attribute__((always_inline)) {
+    const bool real = (uint32_t)blk != 0xffffffffu;
+    const int64_t c = (int64_t)(real ? (uint32_t)blk : 0u) + 8 * (u >> 2) + 4 * (lane >> 5) + (u & 3);
+    const float pen = METRIC == TM_METRIC_L2 ? c_sqnorm[c < n_cent ? c : n_cent - 1] : 0.f;
+    const tm_f32x16 acc0 = mul(f0), acc1 = mul(f1);
+    float v = 0.f;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const float x = odd ? acc1[i] : acc0[i];
+      v = u == i ? x : v;
+    }
+    float dp = (METRIC == TM_METRIC_L2) ? fmaf(-2.f, v, pen) : (pen - v);
+    dp = dp != dp ? __uint_as_float(0x7fc00000u) : dp;  // NaN ranks last, whatever its sign
+    return real && c < n_cent ? make_key(dp, (int)c) : ~0ull;
+  };
+#pragma unroll
+  for (int g = 0; g < K; g += 4) {
+    uint4 a0[KS], a1[KS];
+    load(base[g], a0);
+    load(base[g + 1], a1);
+    if constexpr (KS <= 8) {  // four blocks in flight (their registers fit)
+      uint4 a2[KS], a3[KS];
+      load(base[g + 2], a2);
+      load(base[g + 3], a3);
+      key[g / 2] = rank(odd ? lst[g + 1] : lst[g], a0, a1);
+      key[g / 2 + 1] = rank(odd ? lst[g + 3] : lst[g + 2], a2, a3);
+    } else {
+      key[g / 2] = rank(odd ? lst[g + 1] : lst[g], a0, a1);
+      load(base[g + 2], a0);
+      load(base[g + 3], a1);
+      key[g / 2 + 1] = rank(odd ? lst[g + 3] : lst[g + 2], a0, a1);
+    }
+  }
+  // ascending list per lane (K entries, padded), then the wave's K smallest
+#pragma unroll
+  for (int j = 0; j < K; ++j) lst[j] = ~0ull;
+#pragma unroll
+  for (int p = 0; p < K / 2; ++p) list_insert<K>(lst, key[p]);
+  tm_wave_min_k<K>(lst);
+  if (lane == 0) {
+#pragma unroll
+    for (int j = 0; j < K; ++j)
+      if (j < top_k) write_hit<METRIC>(lst[j], qn, out_dist + r * top_k + j, out_idx + r * top_k + j);
+    if (qs.part != nullptr) qs.out[r] = qn;
+  }
+}
+
 template <int DT>
 __global__ void sqnorm_kernel(const typename Elem<DT>::T *c, int64_t n, int dim, int64_t ld, float *out) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -1261,6 +1432,23 @@ __global__ void sqnorm_kernel(const typename Elem<DT>::T *c, int64_t n, int dim,
     s = fmaf(v, v, s);
   }
   out[i] = s;
+}
+
+template <int DT, int DIM, int K, int METRIC, int RVPL>
+void launch_merge_blocks(const SplitPlan &p, int top_k, const typename Elem<DT>::T *Q, int64_t n, int64_t ld_q,
+                         const typename Elem<DT>::T *C, int64_t n_cent, int64_t ld_c, const float *c_sqnorm,
+                         const QueryNorm &qs, float *out_dist, int64_t *out_idx, const uint64_t *ws,
+                         const tm_route_args *ra, hipStream_t stream) {
+  const int64_t mblocks = tm_cdiv(n, kThreads / 64);
+  MergeRoute mr{};
+  int64_t blocks = mblocks;
+  if (RVPL > 0) {
+    mr.a = *ra;
+    mr.first = mblocks;
+    blocks += tm_cdiv(n, kThreads / 8);
+  }
+  hipLaunchKernelGGL((merge_blocks_kernel<DT, DIM, K, METRIC, RVPL>), dim3((unsigned)blocks), dim3(kThreads), 0,
+                     stream, ws, n, p.nsplit, Q, ld_q, C, n_cent, ld_c, c_sqnorm, qs, top_k, out_dist, out_idx, mr);
 }
 
 template <int DT, int K, int METRIC, int RVPL>
@@ -1286,7 +1474,8 @@ void launch_merge(const SplitPlan &p, int top_k, const typename Elem<DT>::T *Q, 
 template <int DT, int DIM, int K, int METRIC>
 int launch_search(int top_k, const void *q, int64_t n, int64_t ld_q, const float *q_sqnorm,
                   const void *cents, int64_t n_cent, int64_t ld_c, const float *c_sqnorm,
-                  float *out_dist, int64_t *out_idx, uint64_t *ws, const tm_route_args *ra, hipStream_t stream) {
+                  float *out_dist, int64_t *out_idx, uint64_t *ws, const tm_route_args *ra, const QueryNorm *part,
+                  hipStream_t stream) {
   using T = typename Elem<DT>::T;
   const SplitPlan p = plan_split(n, n_cent, DIM, top_k);
   const T *Q = static_cast<const T *>(q);
@@ -1311,12 +1500,21 @@ int launch_search(int top_k, const void *q, int64_t n, int64_t ld_q, const float
                        block, 0, stream, Q, n, ld_q, C, n_cent, ld_c, c_sqnorm, p.chunk, ws);
   }
   TM_LAUNCH_CHECK("tm_search_global");
-  if (ra == nullptr)
-    launch_merge<DT, K, METRIC, 0>(p, top_k, Q, n, ld_q, DIM, q_sqnorm, out_dist, out_idx, ws, ra, stream);
-  else if (ra->n_experts == 64)
-    launch_merge<DT, K, METRIC, 8>(p, top_k, Q, n, ld_q, DIM, q_sqnorm, out_dist, out_idx, ws, ra, stream);
-  else
-    launch_merge<DT, K, METRIC, 16>(p, top_k, Q, n, ld_q, DIM, q_sqnorm, out_dist, out_idx, ws, ra, stream);
+  auto merge = [&](auto rvpl_c) {
+    constexpr int RVPL = decltype(rvpl_c)::value;
+    if constexpr (K > 1) {
+      if (!p.stream) {
+        const QueryNorm qs = part != nullptr ? *part : QueryNorm{q_sqnorm, nullptr, 0, nullptr};
+        launch_merge_blocks<DT, DIM, K, METRIC, RVPL>(p, top_k, Q, n, ld_q, C, n_cent, ld_c, c_sqnorm, qs, out_dist,
+                                                      out_idx, ws, ra, stream);
+        return;
+      }
+    }
+    launch_merge<DT, K, METRIC, RVPL>(p, top_k, Q, n, ld_q, DIM, q_sqnorm, out_dist, out_idx, ws, ra, stream);
+  };
+  if (ra == nullptr) merge(std::integral_constant<int, 0>{});
+  else if (ra->n_experts == 64) merge(std::integral_constant<int, 8>{});
+  else merge(std::integral_constant<int, 16>{});
   TM_LAUNCH_CHECK("tm_search_global(merge)");
   return TM_OK;
 }
@@ -1324,22 +1522,24 @@ int launch_search(int top_k, const void *q, int64_t n, int64_t ld_q, const float
 template <int DT, int DIM, int METRIC>
 int dispatch_k(int top_k, const void *q, int64_t n, int64_t ld_q, const float *q_sqnorm,
                const void *cents, int64_t n_cent, int64_t ld_c, const float *c_sqnorm,
-               float *out_dist, int64_t *out_idx, uint64_t *ws, const tm_route_args *ra, hipStream_t stream) {
+               float *out_dist, int64_t *out_idx, uint64_t *ws, const tm_route_args *ra, const QueryNorm *part,
+               hipStream_t stream) {
   switch (list_len(top_k)) {
-    case 1: return launch_search<DT, DIM, 1, METRIC>(top_k, q, n, ld_q, q_sqnorm, cents, n_cent, ld_c, c_sqnorm, out_dist, out_idx, ws, ra, stream);
-    case 4: return launch_search<DT, DIM, 4, METRIC>(top_k, q, n, ld_q, q_sqnorm, cents, n_cent, ld_c, c_sqnorm, out_dist, out_idx, ws, ra, stream);
-    default: return launch_search<DT, DIM, 8, METRIC>(top_k, q, n, ld_q, q_sqnorm, cents, n_cent, ld_c, c_sqnorm, out_dist, out_idx, ws, ra, stream);
+    case 1: return launch_search<DT, DIM, 1, METRIC>(top_k, q, n, ld_q, q_sqnorm, cents, n_cent, ld_c, c_sqnorm, out_dist, out_idx, ws, ra, part, stream);
+    case 4: return launch_search<DT, DIM, 4, METRIC>(top_k, q, n, ld_q, q_sqnorm, cents, n_cent, ld_c, c_sqnorm, out_dist, out_idx, ws, ra, part, stream);
+    default: return launch_search<DT, DIM, 8, METRIC>(top_k, q, n, ld_q, q_sqnorm, cents, n_cent, ld_c, c_sqnorm, out_dist, out_idx, ws, ra, part, stream);
   }
 }
 
 template <int DT, int METRIC>
 int dispatch_dim(int dim, int top_k, const void *q, int64_t n, int64_t ld_q, const float *q_sqnorm,
                  const void *cents, int64_t n_cent, int64_t ld_c, const float *c_sqnorm,
-                 float *out_dist, int64_t *out_idx, uint64_t *ws, const tm_route_args *ra, hipStream_t stream) {
+                 float *out_dist, int64_t *out_idx, uint64_t *ws, const tm_route_args *ra, const QueryNorm *part,
+               hipStream_t stream) {
   switch (dim) {
-    case 64: return dispatch_k<DT, 64, METRIC>(top_k, q, n, ld_q, q_sqnorm, cents, n_cent, ld_c, c_sqnorm, out_dist, out_idx, ws, ra, stream);
-    case 128: return dispatch_k<DT, 128, METRIC>(top_k, q, n, ld_q, q_sqnorm, cents, n_cent, ld_c, c_sqnorm, out_dist, out_idx, ws, ra, stream);
-    case 256: return dispatch_k<DT, 256, METRIC>(top_k, q, n, ld_q, q_sqnorm, cents, n_cent, ld_c, c_sqnorm, out_dist, out_idx, ws, ra, stream);
+    case 64: return dispatch_k<DT, 64, METRIC>(top_k, q, n, ld_q, q_sqnorm, cents, n_cent, ld_c, c_sqnorm, out_dist, out_idx, ws, ra, part, stream);
+    case 128: return dispatch_k<DT, 128, METRIC>(top_k, q, n, ld_q, q_sqnorm, cents, n_cent, ld_c, c_sqnorm, out_dist, out_idx, ws, ra, part, stream);
+    case 256: return dispatch_k<DT, 256, METRIC>(top_k, q, n, ld_q, q_sqnorm, cents, n_cent, ld_c, c_sqnorm, out_dist, out_idx, ws, ra, part, stream);
     default: return tm_fail(TM_EINVAL_SHAPE, "tm_search_global: dim %d not in {64, 128, 256}", dim);
   }
 }
@@ -1528,7 +1728,7 @@ extern "C" size_t tm_search_global_workspace_size(int64_t n_tokens, int64_t n_ce
 static int search_impl(int32_t dtype, const void *q, int64_t n_tokens, int64_t ld_q, const float *q_sqnorm,
                        const void *cents, int64_t n_cent, int64_t ld_c, const float *c_sqnorm, int32_t dim,
                        int32_t top_k, int32_t metric, float *out_dist, int64_t *out_idx, void *workspace,
-                       size_t workspace_bytes, const tm_route_args *ra, hipStream_t s) {
+                       size_t workspace_bytes, const tm_route_args *ra, const QueryNorm *part, hipStream_t s) {
   TM_REQUIRE(n_tokens >= 0 && n_tokens < ((int64_t)1 << 31) && n_cent > 0 && n_cent < (int64_t)0x7fffffff, TM_EINVAL_SHAPE,
              "tm_search_global: bad sizes n=%lld C=%lld", (long long)n_tokens, (long long)n_cent);
   TM_REQUIRE(ld_q >= dim && ld_c >= dim, TM_EINVAL_SHAPE, "tm_search_global: bad row strides");
@@ -1553,12 +1753,12 @@ static int search_impl(int32_t dtype, const void *q, int64_t n_tokens, int64_t l
   }
   if (dtype == TM_DT_BF16) {
     if (metric == TM_METRIC_L2)
-      return dispatch_dim<TM_DT_BF16, TM_METRIC_L2>(dim, top_k, q, n_tokens, ld_q, q_sqnorm, cents, n_cent, ld_c, c_sqnorm, out_dist, out_idx, ws, ra, s);
-    return dispatch_dim<TM_DT_BF16, TM_METRIC_DOT>(dim, top_k, q, n_tokens, ld_q, q_sqnorm, cents, n_cent, ld_c, c_sqnorm, out_dist, out_idx, ws, ra, s);
+      return dispatch_dim<TM_DT_BF16, TM_METRIC_L2>(dim, top_k, q, n_tokens, ld_q, q_sqnorm, cents, n_cent, ld_c, c_sqnorm, out_dist, out_idx, ws, ra, part, s);
+    return dispatch_dim<TM_DT_BF16, TM_METRIC_DOT>(dim, top_k, q, n_tokens, ld_q, q_sqnorm, cents, n_cent, ld_c, c_sqnorm, out_dist, out_idx, ws, ra, part, s);
   }
   if (metric == TM_METRIC_L2)
-    return dispatch_dim<TM_DT_F16, TM_METRIC_L2>(dim, top_k, q, n_tokens, ld_q, q_sqnorm, cents, n_cent, ld_c, c_sqnorm, out_dist, out_idx, ws, ra, s);
-  return dispatch_dim<TM_DT_F16, TM_METRIC_DOT>(dim, top_k, q, n_tokens, ld_q, q_sqnorm, cents, n_cent, ld_c, c_sqnorm, out_dist, out_idx, ws, ra, s);
+    return dispatch_dim<TM_DT_F16, TM_METRIC_L2>(dim, top_k, q, n_tokens, ld_q, q_sqnorm, cents, n_cent, ld_c, c_sqnorm, out_dist, out_idx, ws, ra, part, s);
+  return dispatch_dim<TM_DT_F16, TM_METRIC_DOT>(dim, top_k, q, n_tokens, ld_q, q_sqnorm, cents, n_cent, ld_c, c_sqnorm, out_dist, out_idx, ws, ra, part, s);
 }
 
 bool tm_internal_route_fusable(const tm_route_args *ra) {
@@ -1573,7 +1773,18 @@ int tm_internal_search_route(int32_t dtype, const void *q, int64_t n_tokens, int
                              size_t workspace_bytes, const tm_route_args *ra, hipStream_t stream) {
   TM_REQUIRE(tm_internal_route_fusable(ra), TM_EINVAL_ARG, "tm_table_forward: router shape cannot be fused");
   return search_impl(dtype, q, n_tokens, ld_q, q_sqnorm, cents, n_cent, ld_c, c_sqnorm, dim, top_k, metric,
-                     out_dist, out_idx, workspace, workspace_bytes, ra, stream);
+                     out_dist, out_idx, workspace, workspace_bytes, ra, nullptr, stream);
+}
+
+int tm_internal_search_topk(int32_t dtype, const void *q, int64_t n_tokens, int64_t ld_q, const void *cents,
+                            int64_t n_cent, int64_t ld_c, const float *c_sqnorm, int32_t dim, int32_t top_k,
+                            int32_t metric, const float *qn_part, int32_t parts, float *out_dist, int64_t *out_idx,
+                            float *out_qn, void *workspace, size_t workspace_bytes, hipStream_t stream) {
+  TM_REQUIRE(n_tokens > 64 && top_k > 1 && qn_part && out_qn && parts >= 1 && parts <= 4, TM_EINVAL_ARG,
+             "tm_table_forward: search from partial norms: bad arguments");
+  const QueryNorm part{nullptr, qn_part, parts, out_qn};
+  return search_impl(dtype, q, n_tokens, ld_q, nullptr, cents, n_cent, ld_c, c_sqnorm, dim, top_k, metric, out_dist,
+                     out_idx, workspace, workspace_bytes, nullptr, &part, stream);
 }
 
 extern "C" int tm_search_global(int32_t dtype, const void *q, int64_t n_tokens, int64_t ld_q,
@@ -1582,7 +1793,7 @@ extern "C" int tm_search_global(int32_t dtype, const void *q, int64_t n_tokens, 
                                 int32_t metric, float *out_dist, int64_t *out_idx, void *workspace,
                                 size_t workspace_bytes, tm_stream_t stream) {
   return search_impl(dtype, q, n_tokens, ld_q, q_sqnorm, cents, n_cent, ld_c, c_sqnorm, dim, top_k, metric,
-                     out_dist, out_idx, workspace, workspace_bytes, nullptr, tm_hip_stream(stream));
+                     out_dist, out_idx, workspace, workspace_bytes, nullptr, nullptr, tm_hip_stream(stream));
 }
 
 namespace {

@@ -1019,3 +1019,28 @@ def test_decode_combine_update_vs_oracle(hip_device, hazard, pattern):
     np.testing.assert_array_equal(np64(mgr.online_expert_ids), st1["ids"])
     np.testing.assert_array_equal(np64(mgr.online_values), st1["values"])
     assert mgr.online_ptr == st1["ptr"]
+
+
+@pytest.mark.parametrize("n,dim,hidden,experts,nn,dt", [(65, 128, 2048, 128, 4, "bf16"), (700, 64, 2560, 64, 2, "f16"),
+                                                        (2100, 128, 2560, 64, 4, "bf16"), (300, 256, 1024, 128, 8, "bf16"),
+                                                        (333, 64, 2048, 32, 3, "f16")])
+def test_layer_of_several_nearest_equals_stage_calls(hip_device, n, dim, hidden, experts, nn, dt):
+    """Batches of more than 64 tokens with several nearest centroids
+    (column-split projection, partial norms added up by the merge) against the
+    five stage calls, bit for bit, on two calls in a row."""
+    from synth import make_workload
+    from table_moe.cache_engine import GlobalTable
+
+    dtype = {"bf16": torch.bfloat16, "f16": torch.float16}[dt]
+    top_k = 8 if experts == 128 else 6
+    w = make_workload(2, n=n, dim=dim, hidden=hidden, n_experts=experts, router_top_k=top_k, n_cent=1500, dtype=dtype,
+                      bias_scale=0.1).to(hip_device)
+    args = (w.x, w.is_vision, w.logits, w.slot_out, w.residual, top_k, nn, 0.5)
+    mk = lambda: GlobalTable(w.centroids, w.values, (w.proj_vis, w.bias_vis), (w.proj_txt, w.bias_txt))  # noqa: E731
+    a, b = mk(), mk()
+    want = {k: v.clone() for k, v in b.layer_forward_staged(*args).items()}
+    for _ in range(2):
+        got = a.layer_forward(*args)
+        torch.cuda.synchronize()
+        for k in ("weights", "ids", "q", "qn", "dist", "idx", "keep", "out"):
+            assert torch.equal(got[k], want[k]), k

@@ -556,3 +556,62 @@ def test_keep_select_block_edges(hip_device, n):
         N.call("tm_keep_select", sd.data_ptr(), n, 1, n_keep, N.as_u8(keep).data_ptr(), None, 0, N.stream(dev))
         torch.cuda.synchronize()
         np.testing.assert_array_equal(np64(keep), O.keep_select(np64(s), n_keep), err_msg=f"n={n} n_keep={n_keep}")
+
+
+@pytest.mark.parametrize("n,c,dim,top_k,metric", [(65, 3, 64, 4, "l2"), (65, 33, 128, 2, "l2"), (200, 1000, 64, 4, "l2"),
+                                                  (257, 4099, 128, 4, "dot"), (513, 2080, 256, 8, "l2"),
+                                                  (70, 16384, 128, 5, "l2"), (1531, 700, 64, 8, "dot"),
+                                                  (3000, 8192, 128, 4, "l2")])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_search_topk_blocks_exact(hip_device, n, c, dim, top_k, metric, dtype):
+    """The top-k of more than 64 queries (nearest blocks, then their
+    centroids) on small integers, whose distances are exact in fp32, so the
+    indices must be the lexicographic top-k: many equal distances (inside a
+    block, across blocks and ranges), tables that end inside a block, fewer
+    centroids than top_k (index -1, worst distance)."""
+    from table_moe.cache_engine import GlobalTable
+
+    g = _gen(91 + n + c)
+    q = torch.randint(-3, 4, (n, dim), generator=g)
+    cents = torch.randint(-3, 4, (c, dim), generator=g)
+    cents[c // 2:] = cents[torch.randint(0, c, (c - c // 2,), generator=g)]  # repeated rows
+    q[: n // 2] = cents[torch.randint(0, c, (n // 2,), generator=g)]
+    score = (q.double() @ cents.double().T)
+    if metric == "l2":
+        score = -((q.double() ** 2).sum(1, keepdim=True) - 2 * score + (cents.double() ** 2).sum(1))
+    order = torch.sort(score, dim=1, descending=True, stable=True).indices[:, :top_k]
+    want = torch.gather(score, 1, order)
+    dev = hip_device
+    p = torch.zeros(256, dim, dtype=dtype, device=dev)
+    tbl = GlobalTable(cents.to(dtype).to(dev), torch.zeros(c, 256, dtype=dtype, device=dev),
+                      (p, torch.zeros(dim, dtype=dtype, device=dev)), metric=metric)
+    dist, idx = tbl.search(q.to(dtype).to(dev), top_k)
+    torch.cuda.synchronize()
+    got = min(top_k, c)
+    np.testing.assert_array_equal(np64(idx)[:, :got], order.numpy()[:, :got])
+    np.testing.assert_array_equal(np64(dist)[:, :got], (-want if metric == "l2" else want).numpy()[:, :got])
+    if got < top_k:
+        assert (np64(idx)[:, got:] == -1).all() and np.isinf(np64(dist)[:, got:]).all()
+
+
+def test_search_topk_blocks_nan_and_inf(hip_device):
+    """A NaN query gives no finite distance to any row but its own; infinite
+    centroids rank behind finite ones."""
+    from table_moe.cache_engine import GlobalTable
+
+    dev = hip_device
+    g = _gen(5)
+    q = torch.randn(100, 64, generator=g).to(torch.bfloat16)
+    cents = torch.randn(300, 64, generator=g).to(torch.bfloat16)
+    cents[::2, 0] = float("inf")
+    tbl = GlobalTable(cents.to(dev), torch.zeros(300, 256, dtype=torch.bfloat16, device=dev),
+                      (torch.zeros(256, 64, dtype=torch.bfloat16, device=dev),
+                       torch.zeros(64, dtype=torch.bfloat16, device=dev)))
+    base_d, base_i = [t.clone() for t in tbl.search(q.to(dev), 4)]
+    assert (np64(base_i) % 2 == 1).all() and np.isfinite(np64(base_d)).all()
+    bad = q.clone()
+    bad[7] = float("nan")
+    d, i = tbl.search(bad.to(dev), 4)
+    torch.cuda.synchronize()
+    rows = np.arange(100) != 7
+    assert torch.equal(i[rows], base_i[rows]) and torch.equal(d[rows], base_d[rows])
