@@ -218,6 +218,15 @@ def mask_bytes(mask: torch.Tensor, device: torch.device) -> torch.Tensor:
     return mask.reshape(-1).to(device=device, dtype=torch.bool).contiguous()
 
 
+def flat(t: torch.Tensor, dtype: torch.dtype, device: torch.device) -> torch.Tensor:
+    """``t``'s elements in row-major order as contiguous ``dtype`` on
+    ``device``, for a call that takes a plain pointer: the tensor itself, of
+    whatever shape, when it already is that, else a converted 1-D copy."""
+    if t.dtype == dtype and t.is_contiguous() and t.get_device() == device.index:
+        return t
+    return t.reshape(-1).to(device=device, dtype=dtype).contiguous()
+
+
 def as_u8(mask: torch.Tensor) -> torch.Tensor:
     """A bool/uint8 mask viewed as bytes (no copy for torch.bool)."""
     if mask.dtype == torch.bool:

@@ -210,12 +210,13 @@ class HybridStorageManager:
         dev = N.require_hip(hidden_state, routing_weights_row, selected_experts_row, out)
         k = int(selected_experts_row.numel())
         mode = N.TM_TARGET_ORIG_SUM if target == "orig_sum" else N.TM_TARGET_ONE
-        w = routing_weights_row.reshape(-1).to(torch.float32).contiguous()
-        sel = selected_experts_row.reshape(-1).to(torch.long).contiguous()
-        u8 = lambda t: None if t is None else N.as_u8(t.reshape(-1).to(device=dev, dtype=torch.bool).contiguous())  # noqa: E731
-        cm, oh, fh = u8(compute_mask_row), u8(on_hit), u8(off_hit)
-        isv = None if is_vision is None else u8(is_vision)
-        ix = lambda t: None if t is None else t.reshape(-1).to(device=dev, dtype=torch.long).contiguous()  # noqa: E731
+        # (tensors that already are what the call takes go by pointer: this runs
+        # once per layer and token, and each torch op on them costs about 1 us)
+        w = N.flat(routing_weights_row, torch.float32, dev)
+        sel = N.flat(selected_experts_row, torch.long, dev)
+        u8 = lambda t: None if t is None else N.flat(t, torch.bool, dev)  # noqa: E731
+        cm, oh, fh, isv = u8(compute_mask_row), u8(on_hit), u8(off_hit), u8(is_vision)
+        ix = lambda t: None if t is None else N.flat(t, torch.long, dev)  # noqa: E731
         oi, osl, fi = ix(on_idx), ix(on_slot), ix(off_idx)
         x = hidden_state.reshape(-1)
         comp = None if computed is None else computed.reshape(k, -1)
@@ -256,20 +257,19 @@ class HybridStorageManager:
         dev = N.require_hip(routing_weights, selected_experts, compute_mask)
         n, k = selected_experts.shape
         mode = N.TM_TARGET_ORIG_SUM if target == "orig_sum" else N.TM_TARGET_ONE
-        w = routing_weights.to(torch.float32).contiguous()
-        sel = selected_experts.to(torch.long).contiguous()
-        u8 = lambda t: None if t is None else N.as_u8(t.to(device=dev, dtype=torch.bool).contiguous())  # noqa: E731
-        ix = lambda t: None if t is None else t.to(device=dev, dtype=torch.long).contiguous()  # noqa: E731
-        cm, fh, oh = u8(compute_mask), u8(off_hit), u8(on_hit)
-        isv = None if is_vision is None else u8(is_vision.reshape(-1))
-        fi, oi, osl = ix(off_idx), ix(None if on_idx is None else on_idx.reshape(-1)), ix(on_slot)
+        w = N.flat(routing_weights, torch.float32, dev)
+        sel = N.flat(selected_experts, torch.long, dev)
+        u8 = lambda t: None if t is None else N.flat(t, torch.bool, dev)  # noqa: E731
+        ix = lambda t: None if t is None else N.flat(t, torch.long, dev)  # noqa: E731
+        cm, fh, oh, isv = u8(compute_mask), u8(off_hit), u8(on_hit), u8(is_vision)
+        fi, oi, osl = ix(off_idx), ix(on_idx), ix(on_slot)
         if computed is not None and (computed.stride(-1) != 1 or computed.dtype != self.dtype):
             raise ValueError(f"computed must be [N, k, H] {self.dtype} with unit stride along hidden")
         if out is None:
             out = torch.empty((n, self.hidden_dim), dtype=self.dtype, device=dev)
         v = self.values_buffer
         ov = self.online_values if (oh is not None and self.enable_online) else None
-        N.call("tm_slot_combine", N.dtype_tag(self.dtype), n, k, self.hidden_dim, N.ptr(w), w.stride(0), N.ptr(cm),
+        N.call("tm_slot_combine", N.dtype_tag(self.dtype), n, k, self.hidden_dim, N.ptr(w), k, N.ptr(cm),
                N.ptr(computed), 0 if computed is None else computed.stride(0),
                0 if computed is None else computed.stride(1), N.ptr(fh), N.ptr(fi), N.ptr(sel), k, N.ptr(isv),
                N.ptr(v), v.shape[0], v.shape[2], v.stride(0), v.stride(1), v.stride(2), N.ptr(oh), N.ptr(oi),

@@ -32,6 +32,7 @@ class GroupedExperts:
         self.n_experts, self.inter, self.hidden = e, inter, h
         self.dtype, self.device = w1.dtype, dev
         self._bufs: dict = {}
+        self._sizes: dict = {}
         self.packed = None
         if packed and h % 128 == 0 and inter % 128 == 0:
             tag = N.dtype_tag(self.dtype)
@@ -49,18 +50,31 @@ class GroupedExperts:
             self._bufs[name] = t
         return t
 
+    def _call_sizes(self, n, k):
+        """(tiles, group workspace bytes, MLP workspace bytes) of a call on
+        [n, k] slots: three library queries, asked once per shape."""
+        s = self._sizes.get((n, k))
+        if s is None:
+            tag, L = N.dtype_tag(self.dtype), N.lib()
+            mlp = (L.tm_grouped_swiglu_packed_workspace_size(n * k, self.inter, self.n_experts, tag)
+                   if self.packed is not None else L.tm_swiglu_workspace_size(n * k, self.inter, tag))
+            if len(self._sizes) >= 256:
+                self._sizes.clear()
+            s = self._sizes[(n, k)] = (L.tm_group_slots_tiles(n * k, self.n_experts),
+                                       L.tm_group_slots_workspace_size(n, k, self.n_experts), mlp)
+        return s
+
     def group(self, ids: torch.Tensor, mask: torch.Tensor, slot_out: torch.Tensor):
         """Bucket the masked (token, slot) pairs by expert; ``mask`` is [N, k]
         or a per-token [N] flag."""
         n, k = ids.shape
         m = N.as_u8(mask)
         ms_b, ms_s = (m.stride(0), 0) if m.dim() == 1 else (m.stride(0), m.stride(1))
-        t_max = N.lib().tm_group_slots_tiles(n * k, self.n_experts)
+        t_max, nbytes, _ = self._call_sizes(n, k)
         offs = self._buf("offsets", self.n_experts + 1, torch.int32)
         row_token = self._buf("row_token", n * k, torch.int32)
         row_out = self._buf("row_out", n * k, torch.int64)
         tiles = self._buf("tiles", 2 + 2 * t_max, torch.int32)
-        nbytes = N.lib().tm_group_slots_workspace_size(n, k, self.n_experts)
         ws = self._buf("group_ws", max(nbytes, 1), torch.uint8)
         N.call("tm_group_slots_ws", N.ptr(ids), n, k, ids.stride(0), N.ptr(m), ms_b, ms_s, self.n_experts,
                slot_out.stride(0), slot_out.stride(1), N.ptr(offs), N.ptr(row_token), N.ptr(row_out), N.ptr(tiles),
@@ -82,10 +96,7 @@ class GroupedExperts:
             raise ValueError("slot_out rows must start on 16-byte boundaries (strides multiples of 8 elements)")
         x = hidden if hidden.stride(-1) == 1 else hidden.contiguous()
         offs, row_token, row_out, tiles = self.group(ids, mask, slot_out)
-        tag = N.dtype_tag(self.dtype)
-        nbytes = (N.lib().tm_grouped_swiglu_packed_workspace_size(n * k, self.inter, self.n_experts, tag)
-                  if self.packed is not None else N.lib().tm_swiglu_workspace_size(n * k, self.inter, tag))
-        ws = self._buf("fused", nbytes, torch.uint8)
+        ws = self._buf("fused", self._call_sizes(n, k)[2], torch.uint8)
         fn, (w1, w3, w2) = (("tm_grouped_swiglu_packed", self.packed) if self.packed is not None
                             else ("tm_grouped_swiglu", (self.w1, self.w3, self.w2)))
         N.call(fn, N.dtype_tag(self.dtype), N.ptr(x), x.stride(0), self.hidden, self.inter, self.n_experts, N.ptr(w1),
