@@ -362,3 +362,42 @@ def test_project_f32_tiled_vs_oracle(hip_device, dim, layout, n, hidden):
         bad = np.abs(np64(q) - ref) > 2 * ulp(ref, torch.float32) + 2.0**-14 * abssum
         assert not bad.any(), (normalize, bad.sum())
         np.testing.assert_allclose(np64(qn), (np64(q) ** 2).sum(1), rtol=2e-6, atol=1e-6)
+
+
+@pytest.mark.parametrize("mods", ["mixed", "vision", "text"])
+@pytest.mark.parametrize("dim,n,hidden,ld_x", [(32, 1, 32, 32), (32, 65, 96, 100), (64, 16, 2048, 2048),
+                                               (64, 257, 160, 160), (128, 33, 1056, 1060), (256, 31, 512, 512),
+                                               (64, 4097, 64, 64)])
+def test_project_f32_matrix_cores(hip_device, dim, n, hidden, ld_x, mods):
+    """k-contiguous fp32 P: row tiles of 1 to 32 rows, one to many k chunks,
+    spaced rows, tiles of one modality and of both, and an infinite row that
+    must reach no other.  Any order of ``hidden`` fp32 products and sums is
+    within (hidden + 4) 2^-24 of the sum of magnitudes."""
+    g = _gen(dim + n + hidden)
+    x = torch.randn(n, ld_x, generator=g)
+    pv, pt = (torch.randn(hidden, dim, generator=g) / hidden**0.5 for _ in range(2))
+    bv, bt = torch.randn(dim, generator=g) * 0.1, torch.randn(dim, generator=g) * 0.1
+    vis = {"mixed": torch.rand(n, generator=g) < 0.5, "vision": torch.ones(n, dtype=torch.bool),
+           "text": torch.zeros(n, dtype=torch.bool)}[mods]
+    bad_row = 5 if n > 5 else None
+    if bad_row is not None:
+        x[bad_row, 3] = float("inf")
+    dev = hip_device
+    xd, visd, bvd, btd = x.to(dev), vis.to(dev), bv.to(dev), bt.to(dev)
+    pvd, ptd = pv.t().contiguous().to(dev), pt.t().contiguous().to(dev)
+    q, qn = torch.empty(n, dim, device=dev), torch.empty(n, device=dev)
+    nbytes = N.lib().tm_project_workspace_size(n, hidden, dim)
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=dev)
+    N.call("tm_project", N.TM_DT_F32, xd.data_ptr(), n, hidden, ld_x, N.as_u8(visd).data_ptr(), pvd.data_ptr(),
+           bvd.data_ptr(), ptd.data_ptr(), btd.data_ptr(), 1, hidden, dim, 0, 1e-6, q.data_ptr(), dim,
+           qn.data_ptr(), ws.data_ptr(), nbytes, N.stream(dev))
+    torch.cuda.synchronize()
+    rows = torch.tensor([i for i in range(n) if i != bad_row])
+    xs, vs = x[rows, :hidden], vis[rows]
+    ref = O.project_queries(np64(xs), vs.numpy(), (np64(pv), np64(bv)), (np64(pt), np64(bt)), False, O.F32)
+    bound = ulp(ref, torch.float32) + (hidden + 4) * 2.0**-24 * proj_abssum(np64(xs), vs.numpy(), np64(pv), np64(pt))
+    got = np64(q)[rows.numpy()]
+    assert (np.abs(got - ref) <= bound).all()
+    np.testing.assert_allclose(np64(qn)[rows.numpy()], (got**2).sum(1), rtol=2e-6, atol=1e-6)
+    if bad_row is not None:
+        assert not torch.isfinite(q[bad_row]).any()
