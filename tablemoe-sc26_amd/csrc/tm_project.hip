@@ -54,8 +54,8 @@ ProjPlan plan_project(int64_t n, int hidden) {
   return p;
 }
 
-// Split plan of the fp32 kernel (its vector-unit k loop is slower per
-// element than the matrix cores, so small batches split hidden further):
+// Split plan of the fp32 kernels (slower per element than the 16-bit ones, so
+// small batches split hidden further):
 // up to 32 chunks of at least 64, with partials of at most 4 MiB unless the
 // 16-bit plan's are larger.
 ProjPlan plan_project_f32(int64_t n, int hidden, int dim) {
@@ -956,9 +956,10 @@ __global__ __launch_bounds__(kThreads) void project_mfma_kernel(
 constexpr int kEpiThreads = 64;
 template <int DT, int DIM>
 __global__ __launch_bounds__(kEpiThreads) void project_epilogue_kernel(
-    const float *__restrict__ partial, int nsplit, int64_t n, const uint8_t *__restrict__ is_vision,
+    const float *partial, int nsplit, int64_t n, const uint8_t *__restrict__ is_vision,
     const typename Elem<DT>::T *__restrict__ bv, const typename Elem<DT>::T *__restrict__ bt, int normalize,
-    float eps, typename Elem<DT>::T *__restrict__ q, int64_t ld_q, float *__restrict__ q_sqnorm) {
+    float eps, typename Elem<DT>::T *q, int64_t ld_q, float *__restrict__ q_sqnorm) {
+  // (partial may be q: a lane reads only the elements that it then writes)
   constexpr int TPR = DIM / 8;
   constexpr int RPB = kEpiThreads / TPR;
   constexpr int kRound = 16;  // splits whose loads are issued together
@@ -1374,10 +1375,15 @@ int launch_project(const void *x, int64_t n, int hidden, int64_t ld_x, const uin
   if constexpr (DT == TM_DT_F32) {
     const ProjPlan pl = plan_project_f32(n, hidden, dim);
     const size_t need = (size_t)pl.nsplit * (size_t)n * (size_t)dim * sizeof(float);
-    const bool tiled = (dim == 32 || dim == 64 || dim == 128 || dim == 256) && !packed && workspace != nullptr &&
-                       workspace_bytes >= need && tm_aligned16(workspace) && tm_aligned16(q) && (ld_q % 4) == 0;
+    // Unsplit, the one partial of an output is written to q itself and finished
+    // there, without a workspace (size 0): from 16384 tokens on, one thread per
+    // output took 6.3 ms where this takes 150 us (16384, 2048, 64).
+    const bool in_q = pl.nsplit == 1 && ld_q == dim;
+    const bool tiled = (dim == 32 || dim == 64 || dim == 128 || dim == 256) && !packed &&
+                       (in_q || (workspace != nullptr && workspace_bytes >= need && tm_aligned16(workspace))) &&
+                       tm_aligned16(q) && (ld_q % 4) == 0;
     if (tiled) {
-      float *partial = static_cast<float *>(workspace);
+      float *partial = in_q ? Q : static_cast<float *>(workspace);
       const dim3 grid((unsigned)pl.row_blocks, (unsigned)pl.nsplit);
       // whole 16-byte loads along k, whole 32-wide steps in every chunk.  Faster
       // at every size where both run: 14.0 -> 7.9 us at (n 1, hidden 2048, dim

@@ -367,10 +367,10 @@ def test_project_f32_tiled_vs_oracle(hip_device, dim, layout, n, hidden):
 @pytest.mark.parametrize("mods", ["mixed", "vision", "text"])
 @pytest.mark.parametrize("dim,n,hidden,ld_x", [(32, 1, 32, 32), (32, 65, 96, 100), (64, 16, 2048, 2048),
                                                (64, 257, 160, 160), (128, 33, 1056, 1060), (256, 31, 512, 512),
-                                               (64, 4097, 64, 64)])
+                                               (64, 4097, 64, 64), (128, 9000, 192, 192)])
 def test_project_f32_matrix_cores(hip_device, dim, n, hidden, ld_x, mods):
-    """k-contiguous fp32 P: row tiles of 1 to 32 rows, one to many k chunks,
-    spaced rows, tiles of one modality and of both, and an infinite row that
+    """k-contiguous fp32 P: row tiles of 1 to 32 rows, one (finished in place in
+    q, no workspace) to many k chunks, spaced rows, tiles of one modality and of both, and an infinite row that
     must reach no other.  Any order of ``hidden`` fp32 products and sums is
     within (hidden + 4) 2^-24 of the sum of magnitudes."""
     g = _gen(dim + n + hidden)
