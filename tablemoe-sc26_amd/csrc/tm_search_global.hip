@@ -112,7 +112,7 @@ static inline int64_t dma_rows(int dim) { return 16384 / (dim * 2); }
 // four-stage ring, so their chunks are a multiple of four stages.
 static inline bool top1_tile(int dim, int top_k) { return top_k <= 1 && dim <= 128; }
 
-SplitPlan plan_split(int64_t n, int64_t c, int dim, int top_k) {
+SplitPlan plan_split(int64_t n, int64_t c, int dim, int top_k, int topk_groups = 256) {
   SplitPlan p;
   p.stream = n <= 64;
   p.wide = false;
@@ -140,7 +140,7 @@ SplitPlan plan_split(int64_t n, int64_t c, int dim, int top_k) {
   const int64_t max_split = tm_cdiv(c, rows);
   // ~2 workgroups per CU; one for top-k, whose merge reads a list per range
   // (1531 queries x 16384 centroids: 17.6 us at two, 16.6 at one)
-  int64_t want = tm_cdiv(top_k > 1 ? 256 : 512, p.row_blocks);
+  int64_t want = tm_cdiv(top_k > 1 ? topk_groups : 512, p.row_blocks);
   const int64_t min_split = tm_cdiv(c, 2048);  // the penalty array holds 2048 centroids
   if (want < min_split) want = min_split;
   if (want < 1) want = 1;
@@ -1720,8 +1720,10 @@ extern "C" int tm_centroid_sqnorms(int32_t dtype, const void *cents, int64_t n_c
 extern "C" size_t tm_search_global_workspace_size(int64_t n_tokens, int64_t n_cent, int32_t dim,
                                                   int32_t top_k) {
   if (n_tokens <= 0 || n_cent <= 0 || top_k <= 0 || (dim != 64 && dim != 128 && dim != 256)) return 0;
-  const int64_t s16 = plan_split(n_tokens, n_cent, dim, top_k).nsplit;  // 16-bit tables
-  const int64_t s32 = plan_f32(n_tokens, n_cent).nsplit;                // fp32 tables
+  // 16-bit tables: lists of 512 workgroups for top-k too, though its plan uses
+  // 256 (never more ranges): callers size and limit their scratch by this value.
+  const int64_t s16 = plan_split(n_tokens, n_cent, dim, top_k, 512).nsplit;
+  const int64_t s32 = plan_f32(n_tokens, n_cent).nsplit;  // fp32 tables
   return (size_t)(s16 > s32 ? s16 : s32) * (size_t)n_tokens * (size_t)list_len(top_k) * sizeof(uint64_t);
 }
 
