@@ -448,7 +448,8 @@ int tm_group_slots(const int64_t *ids, int64_t n_tokens, int32_t top_k, int64_t 
  * launches -- per-workgroup expert counts into `workspace`
  * (tm_group_slots_workspace_size bytes, 16-byte aligned; TM_EWORKSPACE if
  * smaller), then the placement of each workgroup's rows after those of the
- * workgroups before it; other shapes run tm_group_slots (the workspace is
+ * workgroups before it (up to 64 tokens one launch does both, the workspace
+ * checked all the same); other shapes run tm_group_slots (the workspace is
  * not used, and tm_group_slots_workspace_size returns 0).  Same contract as
  * tm_group_slots: the offsets, tile list and the set of rows of each expert
  * are the same; the order of rows inside an expert is unspecified. */

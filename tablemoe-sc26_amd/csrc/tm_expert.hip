@@ -767,7 +767,8 @@ __global__ __launch_bounds__(kGroupThreads) void group_slots_kernel(
 }
 
 // Multi-workgroup grouping (tm_group_slots_ws): kGrpTok tokens per
-// workgroup, in two launches.  group_count_kernel loads its tokens' ids and
+// workgroup, in two launches (one workgroup counts for itself: up to 64 tokens
+// take one launch).  group_count_kernel loads its tokens' ids and
 // mask bytes and writes the workgroup's per-expert counts to a row of the
 // workspace; group_place_kernel loads them again, sums every workgroup's row
 // for each expert (and the rows of the workgroups before it), scans the

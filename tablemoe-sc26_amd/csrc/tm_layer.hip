@@ -18,7 +18,9 @@ constexpr size_t kAlign = 256;
 size_t align_up(size_t v) { return (v + kAlign - 1) / kAlign * kAlign; }
 
 // Three plans share one workspace layout: the general one (tm_project,
-// tm_search_global, tm_keep_select as exported), the fused top-1 one (packed
+// tm_search_global, tm_keep_select as exported; for several nearest centroids
+// of more than 64 tokens the column-split projection carrying the router, its
+// partial query norms finished by the search), the fused top-1 one (packed
 // keys and partial query norms: column-split projection carrying the router
 // and the key reset, search merging by atomic minimum, keep select decoding
 // the keys; for up to 4096 tokens the search decodes the keys and the

@@ -1,4 +1,4 @@
-// Selection kernels: keep-rate radix select (north-star kernel (3)), the
+// Selection kernels: the keep-rate select, the
 // reference's keep masks (table_moe/skip/pruning.py) and surviving-weight
 // renormalisation.
 #include "tm_internal.h"
