@@ -89,6 +89,14 @@ def test_expert_keep_mask_vs_oracle(hip_device, n, k, e, use_attn, keep_rate):
         assert len(kept_got) == len(kept_want)
 
 
+@pytest.mark.parametrize("n,k,e,use_attn", [(512, 8, 128, True), (513, 8, 128, True), (16384, 8, 128, True),
+                                            (16385, 8, 128, False), (40003, 7, 65, True)])
+def test_expert_keep_mask_group_edges(hip_device, n, k, e, use_attn):
+    """4096 mask entries per workgroup and at most 32 workgroups: the edges of
+    one workgroup and of one round, and entries left for a second and third."""
+    test_expert_keep_mask_vs_oracle(hip_device, n, k, e, use_attn, 0.6)
+
+
 @pytest.mark.parametrize("dtype,target", [(torch.float32, None), (torch.float32, "orig"), (torch.bfloat16, None),
                                           (torch.float16, "orig")])
 def test_renormalize_vs_oracle(hip_device, dtype, target):
