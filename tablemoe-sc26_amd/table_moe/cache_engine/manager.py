@@ -258,6 +258,7 @@ class HybridStorageManager:
         n, k = selected_experts.shape
         mode = N.TM_TARGET_ORIG_SUM if target == "orig_sum" else N.TM_TARGET_ONE
         w = N.flat(routing_weights, torch.float32, dev)
+        ld_w = routing_weights.shape[1:].numel()  # a row's elements; the call refuses fewer than k
         sel = N.flat(selected_experts, torch.long, dev)
         u8 = lambda t: None if t is None else N.flat(t, torch.bool, dev)  # noqa: E731
         ix = lambda t: None if t is None else N.flat(t, torch.long, dev)  # noqa: E731
@@ -269,7 +270,7 @@ class HybridStorageManager:
             out = torch.empty((n, self.hidden_dim), dtype=self.dtype, device=dev)
         v = self.values_buffer
         ov = self.online_values if (oh is not None and self.enable_online) else None
-        N.call("tm_slot_combine", N.dtype_tag(self.dtype), n, k, self.hidden_dim, N.ptr(w), k, N.ptr(cm),
+        N.call("tm_slot_combine", N.dtype_tag(self.dtype), n, k, self.hidden_dim, N.ptr(w), ld_w, N.ptr(cm),
                N.ptr(computed), 0 if computed is None else computed.stride(0),
                0 if computed is None else computed.stride(1), N.ptr(fh), N.ptr(fi), N.ptr(sel), k, N.ptr(isv),
                N.ptr(v), v.shape[0], v.shape[2], v.stride(0), v.stride(1), v.stride(2), N.ptr(oh), N.ptr(oi),

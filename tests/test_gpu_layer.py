@@ -1052,3 +1052,29 @@ def test_layer_of_several_nearest_equals_stage_calls(hip_device, n, dim, hidden,
         torch.cuda.synchronize()
         for k in ("weights", "ids", "q", "qn", "dist", "idx", "keep", "out"):
             assert torch.equal(got[k], want[k]), k
+
+
+def test_combine_slots_weight_rows(hip_device):
+    """Weights with more columns than the selection: the first top_k of each
+    row count, tokens without any source among them; with fewer, and as one
+    flat row, the call is refused before anything runs."""
+    dev = hip_device
+    mgr, g = _mode_r_manager(dev, seed=207)
+    n, k, H = 37, 6, 512
+    wide = torch.rand(n, k + 2, generator=g).to(dev)
+    sel = torch.stack([torch.randperm(16, generator=g)[:k] for _ in range(n)]).to(dev)
+    compute = torch.rand(n, k, generator=g) < 0.5
+    compute[::5] = False
+    compute = compute.to(dev)
+    computed = torch.randn(n, k, H, generator=g).to(torch.bfloat16).to(dev)
+    hit = torch.zeros(n, k, dtype=torch.bool, device=dev)
+    idx = torch.zeros(n, k, dtype=torch.long, device=dev)
+    vis = torch.zeros(n, dtype=torch.bool, device=dev)
+    want = mgr.combine_slots(wide[:, :k].contiguous(), sel, vis, compute, computed, hit, idx)
+    got = mgr.combine_slots(wide, sel, vis, compute, computed, hit, idx)
+    torch.cuda.synchronize()
+    assert torch.equal(got, want)
+    assert not want[::5].any() and want[1].any()
+    for bad in (wide[:, :k - 1].contiguous(), wide[:, 0].contiguous()):
+        with pytest.raises(ValueError):
+            mgr.combine_slots(bad, sel, vis, compute, computed, hit, idx)
