@@ -136,7 +136,8 @@ __global__ __launch_bounds__(kThreads) void scores_kernel(
     m = wave_max_f(m);
     float l = 0.f;
 #pragma unroll
-    for (int i = 0; i < kChunk / 64; ++i) l += ok[i] ? expf(sv[i] - m) : 0.f;
+    for (int i = 0; i < kChunk / 64; ++i)  // (a chunk may hold scores of -inf alone: they add nothing)
+      l += ok[i] && sv[i] != -__builtin_huge_valf() ? expf(sv[i] - m) : 0.f;
     l = wave_sum_f(l);
     if (lane == 0) stats[(b * n_heads + h0 + h) * gridDim.x + c] = make_float2(m, l);
   }
@@ -177,20 +178,17 @@ __global__ __launch_bounds__(kThreads) void mean_kernel(const float *__restrict_
         if (cc >= n_chunks) v[i] = make_float2(-__builtin_huge_valf(), 0.f);
         m = fmaxf(m, v[i].x);
       }
-      if (m != -__builtin_huge_valf()) {
-        L *= M == -__builtin_huge_valf() ? 0.f : expf(M - m);
+      // (where a maximum is -inf its sum is 0, or NaN from NaN scores, which stays)
+      L *= M == -__builtin_huge_valf() ? 0.f : expf(M - m);
 #pragma unroll
-        for (int i = 0; i < kBatch; ++i) L += v[i].y == 0.f ? 0.f : v[i].y * expf(v[i].x - m);
-        M = m;
-      }
+      for (int i = 0; i < kBatch; ++i) L += v[i].y == 0.f ? 0.f : v[i].y * expf(v[i].x - m);
+      M = m;
     }
     for (int o = 1; o < lanes; o <<= 1) {
       const float om = __shfl_xor(M, o, 64), ol = __shfl_xor(L, o, 64);
       const float m = fmaxf(M, om);
-      if (m != -__builtin_huge_valf()) {
-        L = (M == -__builtin_huge_valf() ? 0.f : L * expf(M - m)) + (om == -__builtin_huge_valf() ? 0.f : ol * expf(om - m));
-        M = m;
-      }
+      L = L * (M == -__builtin_huge_valf() ? 0.f : expf(M - m)) + ol * (om == -__builtin_huge_valf() ? 0.f : expf(om - m));
+      M = m;
     }
     if (lane == 0 && h < n_heads) {
       hm[h] = M;

@@ -99,3 +99,24 @@ def test_importance_key_chunks_and_head_sets(hip_device, b, h, hkv, d, s, out_le
     torch.cuda.synchronize()
     want = O.last_query_importance(np64(q), np64(ks), hkv, d ** -0.5, O.F32, key_mask=mask.numpy(), out_len=out_len)
     np.testing.assert_allclose(np64(got), want, rtol=1e-4, atol=1e-9)
+
+
+@pytest.mark.parametrize("s,lo,hi", [(300, 64, 192), (4099, 128, 2700), (16500, 16384, 16500)])
+def test_importance_scores_of_minus_infinity(hip_device, s, lo, hi):
+    """Keys that score -inf, whole chunks of them, take no weight and leave the
+    others' as if they were masked."""
+    from table_moe.utils.importance import last_query_importance
+
+    g = torch.Generator().manual_seed(s)
+    h, hkv, d = 8, 2, 128
+    q = torch.randn(1, h, d, generator=g).to(torch.bfloat16)
+    q[:, :, 0] = 1.0
+    ks = torch.randn(1, s, hkv, d, generator=g).to(torch.bfloat16)
+    mask = torch.ones(1, s, dtype=torch.bool)
+    mask[:, lo:hi] = False
+    want = O.last_query_importance(np64(q), np64(ks), hkv, d ** -0.5, O.F32, key_mask=mask.numpy(), out_len=s)
+    ks[:, lo:hi, :, 0] = -float("inf")
+    dev = hip_device
+    got = last_query_importance(q.to(dev), ks.to(dev), hkv, d ** -0.5, True, None, s)
+    torch.cuda.synchronize()
+    np.testing.assert_allclose(np64(got), want, rtol=1e-4, atol=1e-9)
