@@ -159,21 +159,30 @@ __global__ __launch_bounds__(kSelThreads) void keep_select_kernel(const float *_
 // workgroups that share nothing.  Every workgroup reads all n scores (thread t
 // holds scores t, t + 1024, .. as order-preserving keys, R of them, all loads
 // in flight together), counts them in a 4096-bin LDS histogram over the range
-// that they span, finds the bin the n_keep-th largest falls in with one block
-// scan, and lists that bin's keys; it decides only its own kKeepTok tokens
-// (8 threads each count the listed keys ahead of theirs: larger, or equal at a
-// lower index).  With ks.keys set the scores are decoded from packed top-1
-// search keys and a workgroup also writes its tokens' distance, centroid and
-// |q|^2.
+// that they span and finds the bin the n_keep-th largest falls in with one block
+// scan.  A bin of more than kKeepList keys is counted again over its own range
+// (12 bits of the key a time, so at most three counts), until it holds few keys
+// or a single key value; then the workgroup decides only its own kKeepTok
+// tokens: it lists the bin's keys and 8 threads count those ahead of theirs
+// (larger, or equal at a lower index), or, where the bin is a single value,
+// it counts the copies before its tokens.  With ks.keys set the scores are
+// decoded from packed top-1 search keys and a workgroup also writes its
+// tokens' distance, centroid and |q|^2.
 //
 // One workgroup for all tokens was bound by the single CU that read every key
 // and wrote every result (12301 tokens: 32.5 us, 1531: 9.2 us, in the layer
 // call); reading all scores once per 128 tokens from L2 is cheaper than a
-// second launch or a hand-off (11.4 and 4.6 us now).
+// second launch or a hand-off (11.4 and 4.6 us now).  The bins split the range
+// of the key's bits, so one score of 0 or infinity beside a cluster, or many
+// equal scores, put most keys in one bin: us at 12301 scores with one 0 beside
+// a cluster | half of them 0 | all equal: 84 | 106 | 204 when a bin of any size
+// was listed, 17 | 25 | 8 with a radix select in one workgroup, 14 | 23 | 5.5 now
+// (distinct random scores 9-10).
 // ---------------------------------------------------------------------------
 constexpr int kKeepTok = 128;
 constexpr int kKeepMost = 16;  // scores per thread
 constexpr int kKeepBins = 4096;
+constexpr int kKeepList = 128;  // most keys that are ranked pair by pair
 static_assert(kSelThreads % kKeepTok == 0 && kSelThreads == 8 * kKeepTok && kKeepBins == 4 * kSelThreads, "shape");
 
 // Sum over the wave of `v` (one LDS read per wave when `v` comes from shared
@@ -187,11 +196,11 @@ __global__ __launch_bounds__(kSelThreads) void keep_rank_kernel(const float *__r
                                                                 int64_t n_keep, uint8_t *__restrict__ out, KeySrc ks) {
   constexpr int NW = kSelWaves;
   __shared__ __align__(16) uint32_t hist[kKeepBins];
-  __shared__ uint32_t m_key[R * kSelThreads];
-  __shared__ uint16_t m_idx[R * kSelThreads];
+  __shared__ uint32_t m_key[kKeepList];
+  __shared__ uint16_t m_idx[kKeepList];
   __shared__ uint32_t own_key[kKeepTok];
   __shared__ uint32_t wave_tot[NW], s_min[NW], s_max[NW];
-  __shared__ uint2 s_sel;  // boundary bin, keys still to keep in it
+  __shared__ uint4 s_sel;  // boundary bin, keys still to keep in it, keys in it
   __shared__ uint32_t s_members;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int i0 = (int)blockIdx.x * kKeepTok;  // this workgroup's tokens
@@ -268,41 +277,76 @@ __global__ __launch_bounds__(kSelThreads) void keep_rank_kernel(const float *__r
   __syncthreads();
   kmin = tm_wave_min_u32(lane < NW ? s_min[lane] : 0xffffffffu);
   kmax = tm_wave_max_u32(lane < NW ? s_max[lane] : 0u);
-  const uint32_t span = kmax - kmin;
-  const int width = span ? 32 - __builtin_clz(span) : 0;
-  const int shift = width > 12 ? width - 12 : 0;
+  // [base, base + lim]: the keys that the n_keep-th largest is one of, `want`
+  // of which are kept; every key above them is kept, every key below is not
+  uint32_t base = kmin, lim = kmax - kmin, want = (uint32_t)n_keep, members = 0;
+  int shift = lim > 0xfffu ? 20 - __builtin_clz(lim) : 0;
+  auto narrow = [&]() __attribute__((always_inline)) {  // to the bin of the n_keep-th largest, once all keys are counted
+    __syncthreads();
+    // thread t owns the 4 bins of rank 1023 - t (descending bin order across threads)
+    const int rank4 = kSelThreads - 1 - tid;
+    const uint4 h4 = *reinterpret_cast<const uint4 *>(&hist[4 * rank4]);
+    const uint32_t hb[4] = {h4.x, h4.y, h4.z, h4.w};
+    const uint32_t tsum = hb[0] + hb[1] + hb[2] + hb[3];
+    const uint32_t inc = tm_wave_incl_scan(tsum);
+    if (lane == 63) wave_tot[wave] = inc;
+    __syncthreads();
+    uint32_t above = wave_sum_u32(lane < wave ? wave_tot[lane] : 0u) + inc - tsum;  // keys in higher bins
 #pragma unroll
-  for (int r = 0; r < R; ++r)
-    if (r * kSelThreads + tid < n) atomicAdd(&hist[(key[r] - kmin) >> shift], 1u);
-  __syncthreads();
-  // thread t owns the 4 bins of rank 1023 - t (descending bin order across threads)
-  const int rank4 = kSelThreads - 1 - tid;
-  const uint4 h4 = *reinterpret_cast<const uint4 *>(&hist[4 * rank4]);
-  const uint32_t hb[4] = {h4.x, h4.y, h4.z, h4.w};
-  const uint32_t tsum = hb[0] + hb[1] + hb[2] + hb[3];
-  const uint32_t inc = tm_wave_incl_scan(tsum);
-  if (lane == 63) wave_tot[wave] = inc;
-  __syncthreads();
-  uint32_t above = wave_sum_u32(lane < wave ? wave_tot[lane] : 0u) + inc - tsum;  // keys in higher bins
-  const uint32_t want = (uint32_t)n_keep;
+    for (int b = 3; b >= 0; --b) {
+      if (above < want && want <= above + hb[b]) s_sel = make_uint4((uint32_t)(4 * rank4 + b), want - above, hb[b], 0u);
+      above += hb[b];
+    }
+    __syncthreads();
+    const uint4 sel = s_sel;
+    base += sel.x << shift;
+    lim = (1u << shift) - 1u;
+    want = sel.y;
+    members = sel.z;
+  };
+  if (lim != 0) {  // uniform
 #pragma unroll
-  for (int b = 3; b >= 0; --b) {
-    if (above < want && want <= above + hb[b]) s_sel = make_uint2((uint32_t)(4 * rank4 + b), want - above);
-    above += hb[b];
+    for (int r = 0; r < R; ++r)
+      if (r * kSelThreads + tid < n) atomicAdd(&hist[(key[r] - base) >> shift], 1u);
+    narrow();
+    while (lim != 0 && members > (uint32_t)kKeepList) {  // uniform
+      *reinterpret_cast<uint4 *>(&hist[4 * tid]) = make_uint4(0, 0, 0, 0);
+      __syncthreads();  // (also: every thread has read s_sel)
+      shift = shift > 12 ? shift - 12 : 0;
+#pragma unroll
+      for (int r = 0; r < R; ++r)
+        if (r * kSelThreads + tid < n && key[r] - base <= lim) atomicAdd(&hist[(key[r] - base) >> shift], 1u);
+      narrow();
+    }
   }
-  __syncthreads();
-  const uint2 sel = s_sel;
-  // list the keys of the boundary bin (one LDS atomic per wave and register)
+  if (lim == 0) {  // uniform: copies of one value, base
+    uint32_t eq = 0;  // those before this workgroup's tokens
+#pragma unroll
+    for (int r = 0; r < R; ++r) eq += (r * kSelThreads + tid < i0 && key[r] == base) ? 1u : 0u;
+    eq = wave_sum_u32(eq);
+    if (lane == 0) wave_tot[wave] = eq;  // (its last readers are a barrier behind)
+    __syncthreads();
+    if (wave < kKeepTok / 64) {  // uniform: a lane per token
+      uint32_t before = wave_sum_u32(lane < NW ? wave_tot[lane] : 0u);
+      for (int w = 0; w < wave; ++w) before += (uint32_t)__popcll(__ballot(own_key[64 * w + lane] == base));
+      const uint32_t mine = own_key[tid];  // (a token past n: any value, not written)
+      const uint64_t same = __ballot(mine == base);
+      const uint32_t rank = before + (uint32_t)__popcll(same & ((1ull << lane) - 1));
+      if (i0 + tid < n) out[i0 + tid] = mine > base || (mine == base && rank < want) ? 1 : 0;
+    }
+    return;
+  }
+  // list the keys of the range (one LDS atomic per wave and register)
 #pragma unroll
   for (int r = 0; r < R; ++r) {
-    const bool in = r * kSelThreads + tid < n && ((key[r] - kmin) >> shift) == sel.x;
+    const bool in = r * kSelThreads + tid < n && key[r] - base <= lim;
     const uint64_t who = __ballot(in);
     if (who != 0) {  // uniform
-      uint32_t base = 0;
-      if (lane == 0) base = atomicAdd(&s_members, (uint32_t)__popcll(who));
-      base = (uint32_t)__builtin_amdgcn_readfirstlane((int)base);
+      uint32_t at0 = 0;
+      if (lane == 0) at0 = atomicAdd(&s_members, (uint32_t)__popcll(who));
+      at0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)at0);
       if (in) {
-        const uint32_t at = base + (uint32_t)__popcll(who & ((1ull << lane) - 1));
+        const uint32_t at = at0 + (uint32_t)__popcll(who & ((1ull << lane) - 1));
         m_key[at] = key[r];
         m_idx[at] = (uint16_t)(r * kSelThreads + tid);
       }
@@ -311,19 +355,17 @@ __global__ __launch_bounds__(kSelThreads) void keep_rank_kernel(const float *__r
   __syncthreads();
   const int tok = tid >> 3, sub = tid & 7, i = i0 + tok;
   const uint32_t mine = own_key[tok];  // (a token past n: any value, not written)
-  const uint32_t bin = (mine - kmin) >> shift;
+  const bool in = mine - base <= lim;
   uint32_t ahead = 0;
-  if (bin == sel.x) {
-    const uint32_t members = s_members;
+  if (in)
     for (uint32_t m = (uint32_t)sub; m < members; m += 8) {
       const uint32_t k = m_key[m];
       ahead += (k > mine || (k == mine && (int)m_idx[m] < i)) ? 1u : 0u;
     }
-  }
   ahead += (uint32_t)__shfl_xor((int)ahead, 1, 64);
   ahead += (uint32_t)__shfl_xor((int)ahead, 2, 64);
   ahead += (uint32_t)__shfl_xor((int)ahead, 4, 64);
-  if (sub == 0 && i < n) out[i] = bin > sel.x || (bin == sel.x && ahead < sel.y) ? 1 : 0;
+  if (sub == 0 && i < n) out[i] = (in ? ahead < want : mine > base) ? 1 : 0;
 }
 
 void launch_keep_rank(const float *score, int64_t n, int64_t ld, int64_t n_keep, uint8_t *out, const KeySrc &ks,

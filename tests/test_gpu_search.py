@@ -558,6 +558,85 @@ def test_keep_select_block_edges(hip_device, n):
         np.testing.assert_array_equal(np64(keep), O.keep_select(np64(s), n_keep), err_msg=f"n={n} n_keep={n_keep}")
 
 
+def _clustered_scores(g, n, how):
+    """Scores whose keep boundary lies among many close or equal ones."""
+    s = 100.0 + 0.5 * torch.randn(n, generator=g)
+    if how == "equal":
+        s.fill_(2.0)
+    elif how == "one zero":
+        s[n // 3] = 0.0
+    elif how == "half zero":
+        s[::2] = 0.0
+    elif how == "inf and nan":
+        s[n // 3], s[n // 5] = float("inf"), float("nan")
+    elif how == "two values":
+        s = torch.where(s > 100.0, 3.0, 3.0 + 2.0 ** -22)
+    elif how == "signs":
+        s = torch.where(s > 100.0, s * 1e-30, -s)
+    elif how == "runs":  # equal values in a band one bin wide beside a far one
+        s = 50.0 + torch.randint(0, 5, (n,), generator=g).float() * 2.0 ** -18
+        s[n - 1] = -1e30
+    return s
+
+
+@pytest.mark.parametrize("how", ["equal", "one zero", "half zero", "inf and nan", "two values", "signs", "runs"])
+@pytest.mark.parametrize("n", [65, 128, 129, 1000, 1024, 2049, 12301, 16384])
+def test_keep_select_clusters(hip_device, n, how):
+    """Scores that share one histogram bin, so that the bin is counted again
+    (up to the last bit of the key) or is a single value: the answer is the
+    stable order's (larger first, then the lower index; NaN above infinity)."""
+    s = _clustered_scores(_gen(7 + n), n, how)
+    key = np64(torch.nan_to_num(s.double(), nan=1e300, posinf=1e299))
+    order = np.argsort(-key, kind="stable")
+    dev = hip_device
+    sd = s.to(dev)
+    keep = torch.empty(n, dtype=torch.bool, device=dev)
+    for n_keep in sorted({1, 2, n // 2, O.keep_count(n, 0.6), n - 2, n - 1}):
+        want = np.zeros(n, dtype=bool)
+        want[order[:n_keep]] = True
+        N.call("tm_keep_select", sd.data_ptr(), n, 1, n_keep, N.as_u8(keep).data_ptr(), None, 0, N.stream(dev))
+        torch.cuda.synchronize()
+        np.testing.assert_array_equal(np64(keep).astype(bool), want, err_msg=f"n_keep={n_keep}")
+
+
+def _device_us(call, passes=20, reps=9):
+    """Median device time of one `call`, from a captured graph of `passes`."""
+    call()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        for _ in range(passes):
+            call()
+    graph.replay()
+    torch.cuda.synchronize()
+    us = []
+    for _ in range(reps):
+        a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        a.record()
+        graph.replay()
+        b.record()
+        torch.cuda.synchronize()
+        us.append(a.elapsed_time(b) * 1e3 / passes)
+    return sorted(us)[reps // 2]
+
+
+@pytest.mark.parametrize("how", ["equal", "one zero", "half zero"])
+def test_keep_select_clusters_cost(hip_device, how):
+    """Close and equal scores are counted again and not ranked pair by pair,
+    which took 8 to 20 times as long as distinct scores at 12301 (the three
+    counts that the key's bits can need: at most 2.4 times)."""
+    n, n_keep = 12301, 7381
+    dev = hip_device
+    keep = torch.empty(n, dtype=torch.bool, device=dev)
+
+    def us(s):
+        return _device_us(lambda: N.call("tm_keep_select", s.data_ptr(), n, 1, n_keep, N.as_u8(keep).data_ptr(), None,
+                                         0, N.stream(dev)))
+
+    plain = us(torch.randn(n, generator=_gen(3)).to(dev))
+    assert us(_clustered_scores(_gen(4), n, how).to(dev)) < 4 * plain
+
+
 @pytest.mark.parametrize("n,c,dim,top_k,metric", [(65, 3, 64, 4, "l2"), (65, 33, 128, 2, "l2"), (200, 1000, 64, 4, "l2"),
                                                   (257, 4099, 128, 4, "dot"), (513, 2080, 256, 8, "l2"),
                                                   (70, 16384, 128, 5, "l2"), (1531, 700, 64, 8, "dot"),
