@@ -43,6 +43,7 @@ constexpr int kStreamChunk = 128;  // centroids per split of the stream kernel (
 struct SplitPlan {
   bool stream;  // small-n shape
   bool wide;    // top-1 wide tile kernel (8-wave workgroups)
+  bool blocks;  // top-k tile kernel: lists of the nearest blocks (BlockBest), not of centroids
   int qs;       // query slabs per wave
   int64_t row_blocks;
   int64_t nsplit;
@@ -112,10 +113,38 @@ static inline int64_t dma_rows(int dim) { return 16384 / (dim * 2); }
 // four-stage ring, so their chunks are a multiple of four stages.
 static inline bool top1_tile(int dim, int top_k) { return top_k <= 1 && dim <= 128; }
 
-SplitPlan plan_split(int64_t n, int64_t c, int dim, int top_k, int topk_groups = 256) {
+// Whether a top-k search of more than 64 queries lists each query's nearest
+// blocks (BlockBest) or its nearest centroids (CentBest).  Blocks save the
+// insertion of every centroid and cost a merge that reads 32 centroid rows per
+// list entry (n * K * 64 * dim bytes), so they win on large tables, and where
+// the queries are so few that the merge's reads don't fill the chip.  The lines
+// lie where the two cross (either time moves in steps, as the workgroups fill
+// whole rounds of CUs).  us per search, K = 4 | 8, centroids against blocks:
+// d 64, 12000 queries: 1279 centroids 34 | 61 against 38 | 78, 2048: 47 | 86 against
+// 40 | 80; 4000 queries of 256: 21 | 37 against 18 | 36.  d 128: 12000 of 3072: 59 |
+// 106 against 80 | 142, of 4096: 85 | 152 against 83 | 145; 1531 of 2048: 18 | 28
+// against 19 | 32, of 3072: 23 | 36 against 20 | 33; 768 of 256: 16 | 25 against
+// 15 | 23.  d 256: 4000 of 1024: 24 | 40 against 55 | 80, of 14000 (3000): 70 | 133
+// against 76 | 122, of 16384 (10000): 244 | 503 against 220 | 351, (8000): 142 | 289
+// against 169 | 296; 768 of 8192: 27 | 46 against 28 | 47, of 12000: 33 | 57 against
+// 28 | 49; 65 of 12000: 19 | 30 against 20 | 33.
+inline bool topk_blocks(int64_t n, int64_t c, int dim, int top_k) {
+  if (dim == 64) return n <= 5120 || c >= (top_k > 4 ? 1408 : 1344);
+  if (dim == 128) {
+    if (n <= 1024) return true;
+    if (n <= 2048) return tm_cdiv(n, kTileRows) * tm_cdiv(c, dma_rows(128)) > 256;  // past one round of CUs
+    return c >= (n > 4096 ? 4096 : 3072);
+  }
+  if (n <= 256) return c >= 16384;
+  if (n <= 2048 || top_k > 4) return c >= 12000;
+  return c >= (n > 5120 && n <= 8192 ? 24576 : 16384);
+}
+
+SplitPlan plan_split(int64_t n, int64_t c, int dim, int top_k, int block_groups = 256) {
   SplitPlan p;
   p.stream = n <= 64;
   p.wide = false;
+  p.blocks = false;
   if (p.stream) {
     p.qs = n <= 32 ? 1 : 2;
     p.row_blocks = 1;
@@ -135,12 +164,13 @@ SplitPlan plan_split(int64_t n, int64_t c, int dim, int top_k, int topk_groups =
       return p;
     }
   }
+  p.blocks = top_k > 1 && topk_blocks(n, c, dim, top_k);
   p.row_blocks = tm_cdiv(n, kTileRows);
   const int64_t rows = dma_rows(dim);
   const int64_t max_split = tm_cdiv(c, rows);
-  // ~2 workgroups per CU; one for top-k, whose merge reads a list per range
-  // (1531 queries x 16384 centroids: 17.6 us at two, 16.6 at one)
-  int64_t want = tm_cdiv(top_k > 1 ? topk_groups : 512, p.row_blocks);
+  // ~2 workgroups per CU; one for lists of blocks, whose merge costs more per
+  // range (1531 queries x 16384 centroids: 17.6 us at two, 16.6 at one)
+  int64_t want = tm_cdiv(p.blocks ? block_groups : 512, p.row_blocks);
   const int64_t min_split = tm_cdiv(c, 2048);  // the penalty array holds 2048 centroids
   if (want < min_split) want = min_split;
   if (want < 1) want = 1;
@@ -209,9 +239,9 @@ struct Best {
 // Epilogue of one 32x32 block: lane owns query (l%32) and the 16 centroids
 // m = 8*(i/4) + 4*(l/32) + (i%4) of the block.  pen[i] = ||c||^2 (L2) or
 // 0 (dot) for valid centroids, +inf past the end.
-template <int K, int METRIC>
-__device__ __forceinline__ void block_epilogue(const tm_f32x16 &acc, const float (&pen)[16], int cbase,
-                                               int lane, Best<K> &best) {
+template <int K, int METRIC, typename B>
+__device__ __forceinline__ void block_epilogue(const tm_f32x16 &acc, const float (&pen)[16], int cbase, int lane,
+                                               B &best) {
 #pragma unroll
   for (int i = 0; i < 16; ++i) {
     const int c = cbase + 8 * (i >> 2) + 4 * (lane >> 5) + (i & 3);
@@ -220,8 +250,47 @@ __device__ __forceinline__ void block_epilogue(const tm_f32x16 &acc, const float
   }
 }
 
-// The tile kernel's top-k: each lane keeps the K nearest 32-centroid BLOCKS of
-// its query, a block ranked by its nearest centroid (packed key: smallest dp
+// The tile kernel's top-k over small tables (see topk_blocks): each lane keeps
+// the K nearest of its centroids (half of each block).  Its keys hold the
+// distance's order-preserving bits less those of -inf: the NaNs with a sign,
+// which lie below -inf, wrap round and rank last as the others do (xor and
+// subtraction are one instruction).  The tile's padding (+inf, an index past
+// the table) is dropped at the end.
+template <int K>
+struct CentBest {
+  static constexpr uint32_t kLow = 0x007fffffu;  // tm_orderable(-inf)
+  uint64_t l[K];
+  __device__ __forceinline__ void init() {
+#pragma unroll
+    for (int j = 0; j < K; ++j) l[j] = ~0ull;
+  }
+  __device__ __forceinline__ void push(float dp, int c) {
+    const uint64_t key = ((uint64_t)(tm_orderable(dp) - kLow) << 32) | (uint32_t)c;
+    if (key < l[K - 1]) list_insert<K>(l, key);
+  }
+  // to the keys of the lists in memory
+  __device__ __forceinline__ void finalize(int n_cent) {
+#pragma unroll
+    for (int j = 0; j < K; ++j) {
+      const uint32_t hi = (uint32_t)(l[j] >> 32), c = (uint32_t)l[j];
+      const bool nan = hi > tm_orderable(__builtin_huge_valf()) - kLow;
+      const uint64_t key = make_key(nan ? __uint_as_float(0x7fc00000u) : tm_from_orderable(hi + kLow), (int)c);
+      l[j] = c < (uint32_t)n_cent ? key : ~0ull;
+    }
+  }
+  // merge with the lane `o` lanes away (same query, other centroids)
+  __device__ __forceinline__ void merge_xor(int o) {
+    uint64_t other[K];
+#pragma unroll
+    for (int j = 0; j < K; ++j) other[j] = __shfl_xor(l[j], o, 64);
+#pragma unroll
+    for (int j = 0; j < K; ++j)
+      if (other[j] < l[K - 1]) list_insert<K>(l, other[j]);
+  }
+};
+
+// The tile kernel's top-k over large tables: each lane keeps the K nearest
+// 32-centroid BLOCKS of its query, a block ranked by its nearest centroid (packed key: smallest dp
 // << 32 | first centroid).  The K nearest centroids all lie in those blocks: a
 // centroid in any other block is behind the nearest centroid of each of the K,
 // and blocks are runs of consecutive indices, so equal distances rank blocks
@@ -238,7 +307,7 @@ struct BlockBest {
 #pragma unroll
     for (int j = 0; j < K; ++j) l[j] = ~0ull;
   }
-  __device__ __forceinline__ void finalize() {}
+  __device__ __forceinline__ void finalize(int) {}
   __device__ __forceinline__ void merge_xor(int) {}  // both lanes of a query hold the same list
 };
 
@@ -280,7 +349,7 @@ constexpr int kDmaStageBytes = 16384;
 
 
 
-template <int DT, int DIM, int K, int METRIC>
+template <int DT, int DIM, int K, int METRIC, bool BLOCKS>
 __global__ __launch_bounds__(kThreads, 2) void search_dma_kernel(
     const typename Elem<DT>::T *__restrict__ q, int64_t n, int64_t ld_q,
     const typename Elem<DT>::T *__restrict__ cents, int64_t n_cent, int64_t ld_c,
@@ -351,7 +420,7 @@ __global__ __launch_bounds__(kThreads, 2) void search_dma_kernel(
 #pragma unroll
   for (int u = 0; u < PEN_PER_THREAD; ++u) pen_s[tid + u * kThreads] = pen_v[u];
 
-  std::conditional_t<K == 1, Best<K>, BlockBest<K>> best[kQS];
+  std::conditional_t<K == 1, Best<K>, std::conditional_t<BLOCKS, BlockBest<K>, CentBest<K>>> best[kQS];
 #pragma unroll
   for (int sl = 0; sl < kQS; ++sl) best[sl].init();
 
@@ -402,7 +471,8 @@ __global__ __launch_bounds__(kThreads, 2) void search_dma_kernel(
 
 #pragma unroll
   for (int sl = 0; sl < kQS; ++sl) {
-    best[sl].finalize();
+    if constexpr (K == 1) best[sl].finalize();
+    else best[sl].finalize((int)n_cent);
     best[sl].merge_xor(32);  // the two half-waves saw disjoint centroids of the same query
     const int64_t r = row_base + sl * 32 + (lane & 31);
     if (lane < 32 && r < n) {
@@ -1247,19 +1317,36 @@ __global__ __launch_bounds__(kThreads) void merge_top1_kernel(
   if (r < n && j == 0) write_hit<METRIC>(best, qn, out_dist + r, out_idx + r);
 }
 
+// |q|^2 of a search's queries: given, the projection's partial norms (the merge
+// then also writes their sum to `out`), or, with neither, computed by the merge.
+struct QueryNorm {
+  const float *q_sqnorm;  // nullable
+  const float *part;      // nullable: [parts][n]
+  int parts;
+  float *out;
+};
+
+__device__ __forceinline__ float part_norm(const QueryNorm &qs, int64_t n, int64_t r) {
+  float a[4];
+#pragma unroll
+  for (int p = 0; p < 4; ++p) a[p] = qs.part[(p < qs.parts ? p : 0) * n + r];
+  return qn_sum(a[0], a[1], a[2], a[3], qs.parts);
+}
+
 // Top-k merge (k = 4 or 8): one wave per query; lane l merges the sorted lists
 // of splits l, l+64, ...; then six xor-shuffle steps merge the lanes' lists.
 template <int DT, int K, int METRIC, int RVPL>
 __global__ __launch_bounds__(kThreads) void merge_kernel(
     const uint64_t *__restrict__ ws, int64_t n, int64_t nsplit, const typename Elem<DT>::T *__restrict__ q,
-    int64_t ld_q, int dim, const float *__restrict__ q_sqnorm, int top_k, float *__restrict__ out_dist,
-    int64_t *__restrict__ out_idx, MergeRoute mr) {
+    int64_t ld_q, int dim, QueryNorm qs, int top_k, float *__restrict__ out_dist, int64_t *__restrict__ out_idx,
+    MergeRoute mr) {
   if (merge_route_role<RVPL>(mr, n)) return;
   const int lane = threadIdx.x & 63;
   const int64_t r = (int64_t)blockIdx.x * (kThreads / 64) + (threadIdx.x >> 6);
   if (r >= n) return;  // whole wave exits together
   float qn = 0.f;
-  if (METRIC == TM_METRIC_L2 && q_sqnorm != nullptr) qn = q_sqnorm[r];
+  if (qs.part != nullptr) qn = part_norm(qs, n, r);
+  else if (METRIC == TM_METRIC_L2 && qs.q_sqnorm != nullptr) qn = qs.q_sqnorm[r];
   uint64_t lst[K];
 #pragma unroll
   for (int j = 0; j < K; ++j) lst[j] = ~0ull;
@@ -1278,7 +1365,7 @@ __global__ __launch_bounds__(kThreads) void merge_kernel(
     for (int j = 0; j < K; ++j) other[j] = __shfl_xor(lst[j], o, 64);
     merge_min<K>(lst, other);
   }
-  if (METRIC == TM_METRIC_L2 && q_sqnorm == nullptr) {
+  if (METRIC == TM_METRIC_L2 && qs.q_sqnorm == nullptr && qs.part == nullptr) {
     for (int j = lane; j < dim; j += 64) {
       const float v = Elem<DT>::to_f(q[r * ld_q + j]);
       qn = fmaf(v, v, qn);
@@ -1289,6 +1376,7 @@ __global__ __launch_bounds__(kThreads) void merge_kernel(
 #pragma unroll
     for (int j = 0; j < K; ++j)
       if (j < top_k) write_hit<METRIC>(lst[j], qn, out_dist + r * top_k + j, out_idx + r * top_k + j);
+    if (qs.part != nullptr) qs.out[r] = qn;
   }
 }
 
@@ -1298,15 +1386,7 @@ __global__ __launch_bounds__(kThreads) void merge_kernel(
 // same bits) and takes the top_k smallest keys.  D of a block has every row in
 // all of the 32 columns (each column is the query), so lane l keeps row
 // 8 (u / 4) + 4 (l / 32) + u % 4, u = l % 16, of block 2 p + (l / 16) % 2 of
-// each pair p.  |q|^2 comes from q_sqnorm, from the projection's partial norms
-// (then also written to out_qn), or is computed.
-struct QueryNorm {
-  const float *q_sqnorm;  // nullable
-  const float *part;      // nullable: [parts][n]
-  int parts;
-  float *out;
-};
-
+// each pair p. 
 template <int DT, int DIM, int K, int METRIC, int RVPL>
 __global__ __launch_bounds__(kThreads) void merge_blocks_kernel(
     const uint64_t *__restrict__ ws, int64_t n, int64_t nsplit, const typename Elem<DT>::T *__restrict__ q,
@@ -1319,14 +1399,8 @@ __global__ __launch_bounds__(kThreads) void merge_blocks_kernel(
   const int64_t r = (int64_t)blockIdx.x * (kThreads / 64) + (threadIdx.x >> 6);
   if (r >= n) return;  // whole wave exits together
   float qn = 0.f;
-  if (qs.part != nullptr) {
-    float a[4];
-#pragma unroll
-    for (int p = 0; p < 4; ++p) a[p] = qs.part[(p < qs.parts ? p : 0) * n + r];
-    qn = qn_sum(a[0], a[1], a[2], a[3], qs.parts);
-  } else if (METRIC == TM_METRIC_L2 && qs.q_sqnorm != nullptr) {
-    qn = qs.q_sqnorm[r];
-  }
+  if (qs.part != nullptr) qn = part_norm(qs, n, r);
+  else if (METRIC == TM_METRIC_L2 && qs.q_sqnorm != nullptr) qn = qs.q_sqnorm[r];
   uint4 qf[KS];
 #pragma unroll
   for (int ks = 0; ks < KS; ++ks)
@@ -1453,7 +1527,7 @@ void launch_merge_blocks(const SplitPlan &p, int top_k, const typename Elem<DT>:
 
 template <int DT, int K, int METRIC, int RVPL>
 void launch_merge(const SplitPlan &p, int top_k, const typename Elem<DT>::T *Q, int64_t n, int64_t ld_q, int dim,
-                  const float *q_sqnorm, float *out_dist, int64_t *out_idx, const uint64_t *ws,
+                  const QueryNorm &qs, float *out_dist, int64_t *out_idx, const uint64_t *ws,
                   const tm_route_args *ra, hipStream_t stream) {
   const int64_t mblocks = K == 1 ? tm_cdiv(n, kThreads / 4) : tm_cdiv(n, kThreads / 64);
   MergeRoute mr{};
@@ -1465,10 +1539,10 @@ void launch_merge(const SplitPlan &p, int top_k, const typename Elem<DT>::T *Q, 
   }
   if constexpr (K == 1)
     hipLaunchKernelGGL((merge_top1_kernel<DT, METRIC, RVPL>), dim3((unsigned)blocks), dim3(kThreads), 0, stream, ws,
-                       n, p.nsplit, Q, ld_q, dim, q_sqnorm, out_dist, out_idx, mr);
+                       n, p.nsplit, Q, ld_q, dim, qs.q_sqnorm, out_dist, out_idx, mr);
   else
     hipLaunchKernelGGL((merge_kernel<DT, K, METRIC, RVPL>), dim3((unsigned)blocks), dim3(kThreads), 0, stream, ws,
-                       n, p.nsplit, Q, ld_q, dim, q_sqnorm, top_k, out_dist, out_idx, mr);
+                       n, p.nsplit, Q, ld_q, dim, qs, top_k, out_dist, out_idx, mr);
 }
 
 template <int DT, int DIM, int K, int METRIC>
@@ -1495,22 +1569,27 @@ int launch_search(int top_k, const void *q, int64_t n, int64_t ld_q, const float
     // (d = 256 would not fit two waves per SIMD; the stage byte offsets must fit 31 bits)
     hipLaunchKernelGGL((search_top1_kernel<DT, DIM < 256 ? DIM : 128, METRIC>), dim3((unsigned)p.row_blocks, (unsigned)p.nsplit),
                        block, 0, stream, Q, n, ld_q, C, n_cent, ld_c, c_sqnorm, p.chunk, ws, nullptr);
+  } else if (p.blocks) {
+    hipLaunchKernelGGL((search_dma_kernel<DT, DIM, K, METRIC, (K > 1)>),
+                       dim3((unsigned)p.row_blocks, (unsigned)p.nsplit), block, 0, stream, Q, n, ld_q, C, n_cent, ld_c,
+                       c_sqnorm, p.chunk, ws);
   } else {
-    hipLaunchKernelGGL((search_dma_kernel<DT, DIM, K, METRIC>), dim3((unsigned)p.row_blocks, (unsigned)p.nsplit),
-                       block, 0, stream, Q, n, ld_q, C, n_cent, ld_c, c_sqnorm, p.chunk, ws);
+    hipLaunchKernelGGL((search_dma_kernel<DT, DIM, K, METRIC, false>),
+                       dim3((unsigned)p.row_blocks, (unsigned)p.nsplit), block, 0, stream, Q, n, ld_q, C, n_cent, ld_c,
+                       c_sqnorm, p.chunk, ws);
   }
   TM_LAUNCH_CHECK("tm_search_global");
   auto merge = [&](auto rvpl_c) {
     constexpr int RVPL = decltype(rvpl_c)::value;
+    const QueryNorm qs = part != nullptr ? *part : QueryNorm{q_sqnorm, nullptr, 0, nullptr};
     if constexpr (K > 1) {
-      if (!p.stream) {
-        const QueryNorm qs = part != nullptr ? *part : QueryNorm{q_sqnorm, nullptr, 0, nullptr};
+      if (p.blocks) {
         launch_merge_blocks<DT, DIM, K, METRIC, RVPL>(p, top_k, Q, n, ld_q, C, n_cent, ld_c, c_sqnorm, qs, out_dist,
                                                       out_idx, ws, ra, stream);
         return;
       }
     }
-    launch_merge<DT, K, METRIC, RVPL>(p, top_k, Q, n, ld_q, DIM, q_sqnorm, out_dist, out_idx, ws, ra, stream);
+    launch_merge<DT, K, METRIC, RVPL>(p, top_k, Q, n, ld_q, DIM, qs, out_dist, out_idx, ws, ra, stream);
   };
   if (ra == nullptr) merge(std::integral_constant<int, 0>{});
   else if (ra->n_experts == 64) merge(std::integral_constant<int, 8>{});
@@ -1674,7 +1753,8 @@ int launch_search_f32(int top_k, const void *q, int64_t n, int64_t ld_q, const f
   else
     go(std::integral_constant<int, 16>{});
   TM_LAUNCH_CHECK("tm_search_global(f32)");
-  launch_merge<TM_DT_F32, K, METRIC, 0>(p, top_k, Q, n, ld_q, DIM, q_sqnorm, out_dist, out_idx, ws, nullptr, stream);
+  launch_merge<TM_DT_F32, K, METRIC, 0>(p, top_k, Q, n, ld_q, DIM, QueryNorm{q_sqnorm, nullptr, 0, nullptr}, out_dist,
+                                        out_idx, ws, nullptr, stream);
   TM_LAUNCH_CHECK("tm_search_global(merge)");
   return TM_OK;
 }
@@ -1720,8 +1800,9 @@ extern "C" int tm_centroid_sqnorms(int32_t dtype, const void *cents, int64_t n_c
 extern "C" size_t tm_search_global_workspace_size(int64_t n_tokens, int64_t n_cent, int32_t dim,
                                                   int32_t top_k) {
   if (n_tokens <= 0 || n_cent <= 0 || top_k <= 0 || (dim != 64 && dim != 128 && dim != 256)) return 0;
-  // 16-bit tables: lists of 512 workgroups for top-k too, though its plan uses
-  // 256 (never more ranges): callers size and limit their scratch by this value.
+  // 16-bit tables: lists of 512 workgroups for every plan, though that of block
+  // lists uses 256 (never more ranges): callers size and limit their scratch by
+  // this value.
   const int64_t s16 = plan_split(n_tokens, n_cent, dim, top_k, 512).nsplit;
   const int64_t s32 = plan_f32(n_tokens, n_cent).nsplit;  // fp32 tables
   return (size_t)(s16 > s32 ? s16 : s32) * (size_t)n_tokens * (size_t)list_len(top_k) * sizeof(uint64_t);
