@@ -185,38 +185,71 @@ __device__ __forceinline__ void skinny_block(const typename Elem<DT>::T *const (
   tm_wait_vm_lgkm0_mem<0>();  // every read is done before the next block's loads
 }
 
-// split > 0 (dense rows): a workgroup takes one RBMAX-row block of a tile
-// (split blocks per tile); split == 0: all of the tile's, one after the other.
-// ONCE: no other workgroup reads these weights (grouped rows), so they are
-// loaded non-temporally and leave the L2 to the activation rows.
-template <int DT, class Cfg, bool PB, bool ONCE>
+// A workgroup takes one RBMAX-row block of a tile.  Grouped rows: the first
+// `slots` blocks of workgroups take the tiles' first row blocks, so a call whose
+// experts have few rows each runs as if there were no others; the blocks past
+// them look for the tile of their further row block (a scan of the tile list)
+// and find none where routing is even.  One workgroup for all rows of a tile,
+// one block after the other, made uneven routing slow (us, 2048 x 768: 192 rows
+// on each of 8 experts 124, 63 now and 74 with tiles of four waves before; 1536
+// rows on one expert 135, 61 now and 76).
+// Packed weights of an expert of one row block are read by no other workgroup:
+// they are loaded non-temporally and leave the L2 to the activation rows.
+template <int DT, class Cfg, bool PB>
 __global__ __launch_bounds__(64) void skinny_gemm_kernel(
     const typename Elem<DT>::T *__restrict__ A, int64_t lda, const int32_t *__restrict__ a_rows,
     const typename Elem<DT>::T *__restrict__ B0, const typename Elem<DT>::T *__restrict__ B1, int64_t b_expert,
-    int K, int n_groups, int pack_bn, int split, TileSrc ts, typename Elem<DT>::T *__restrict__ C, int64_t ldc,
+    int K, int n_groups, int pack_bn, int slots, TileSrc ts, typename Elem<DT>::T *__restrict__ C, int64_t ldc,
     const int64_t *__restrict__ c_rows, const typename Elem<DT>::T *__restrict__ addend, int64_t ld_add) {
   using T = typename Elem<DT>::T;
   constexpr int MODE = Cfg::MODE, CW = Cfg::CW, SUB = Cfg::SUB;
   __shared__ uint4 ring[Cfg::LDS / 16];
+  const int lane = threadIdx.x & 63;
   const int64_t blk = blockIdx.x / n_groups;
-  const int64_t y = split > 0 ? blk / split : blk;
   const int n0 = (int)(blockIdx.x % n_groups) * CW;
-  int e, r0, r_end;
+  int64_t y = blk;
+  int e, r0, r_end, rb = 0;  // expert, the tile's rows [r0, r_end), this block's first row in it
+  bool once = false;
   if (ts.tiles != nullptr) {
-    if (y >= ts.t_max || y >= ts.tiles[1]) return;  // uniform: past the last tile
+    const int64_t nt = ts.tiles[1] < ts.t_max ? ts.tiles[1] : ts.t_max;
+    if (blk >= slots) {
+      int u = (int)(blk - slots);  // this is further row block u
+      for (int64_t t0 = 0;; t0 += 64) {
+        if (t0 >= nt) return;  // uniform: there are fewer
+        const int64_t t = t0 + lane;
+        int more = 0;
+        if (t < nt) {
+          const int rows = ts.expert_offsets[ts.tiles[2 + t] + 1] - ts.tiles[2 + ts.t_max + t];
+          more = ((rows < BM ? rows : BM) - 1) / Cfg::RBMAX;
+        }
+        const int upto = (int)tm_wave_incl_scan((uint32_t)more);
+        const int total = __builtin_amdgcn_readlane(upto, 63);
+        if (u < total) {  // uniform
+          const int l = __builtin_ctzll(__ballot(u < upto));
+          y = t0 + l;
+          rb = (u - __builtin_amdgcn_readlane(upto - more, l) + 1) * Cfg::RBMAX;
+          break;
+        }
+        u -= total;
+      }
+    }
+    if (y >= nt) return;  // uniform: past the last tile
     e = ts.tiles[2 + y];
     r0 = ts.tiles[2 + ts.t_max + y];
     r_end = ts.expert_offsets[e + 1];
+    once = r_end - ts.expert_offsets[e] <= Cfg::RBMAX;
   } else {
+    constexpr int kBlocks = BM / Cfg::RBMAX;
+    y = blk / kBlocks;
+    rb = (int)(blk % kBlocks) * Cfg::RBMAX;
     e = 0;
     r0 = (int)y * BM;
     if (r0 >= ts.rows) return;
     r_end = ts.rows;
   }
   r_end = r_end < r0 + BM ? r_end : r0 + BM;  // this tile's rows
-  const int rb0 = split > 0 ? (int)(blk % split) * Cfg::RBMAX : 0;
-  const int rb1 = split > 0 && rb0 + Cfg::RBMAX < r_end - r0 ? rb0 + Cfg::RBMAX : r_end - r0;
-  const int lane = threadIdx.x & 63;
+  const int rows = r_end - r0 - rb < Cfg::RBMAX ? r_end - r0 - rb : Cfg::RBMAX;
+  if (rows <= 0) return;  // uniform
   const int KT = K / BK;
   const uint32_t lds0 = (uint32_t)(uintptr_t)ring;
   const char *const lds = reinterpret_cast<const char *>(ring);
@@ -267,78 +300,80 @@ __global__ __launch_bounds__(64) void skinny_gemm_kernel(
   constexpr bool kTiledA = PB && MODE == kModeDown;
   constexpr int kNBMax = Cfg::RBMAX > 32 ? Cfg::RBMAX / 32 : 1;
   const int64_t x_step = kTiledA ? (int64_t)BM * BK : BK;
-  for (int rb = rb0; rb < rb1; rb += Cfg::RBMAX) {
-    const int rows = rb1 - rb;
-    const T *x_src[4] = {};
+  const T *x_src[4] = {};
 #pragma unroll
-    for (int j = 0; j < Cfg::RBMAX / 16; ++j) {
-      const int tr = 16 * j + lr;
-      if constexpr (kTiledA) {
-        x_src[j] = A + y * (int64_t)BM * lda + (int64_t)(rb + tr) * BK + (lane & 3) * 8;
-      } else {
-        int gr = r0 + rb + tr;
-        gr = gr < r_end ? gr : r_end - 1;  // rows past the expert re-read its last row; their results are dropped
-        const int64_t xr = a_rows ? (int64_t)a_rows[gr] : (int64_t)gr;
-        x_src[j] = A + xr * lda + swz_chunk(tr, lane & 3) * 8;
-      }
+  for (int j = 0; j < Cfg::RBMAX / 16; ++j) {
+    const int tr = 16 * j + lr;
+    if constexpr (kTiledA) {
+      x_src[j] = A + y * (int64_t)BM * lda + (int64_t)(rb + tr) * BK + (lane & 3) * 8;
+    } else {
+      int gr = r0 + rb + tr;
+      gr = gr < r_end ? gr : r_end - 1;  // rows past the expert re-read its last row; their results are dropped
+      const int64_t xr = a_rows ? (int64_t)a_rows[gr] : (int64_t)gr;
+      x_src[j] = A + xr * lda + swz_chunk(tr, lane & 3) * 8;
     }
-    tm_f32x16 acc[Cfg::kNA][kNBMax];
+  }
+  tm_f32x16 acc[Cfg::kNA][kNBMax];
 #pragma unroll
-    for (int a = 0; a < Cfg::kNA; ++a)
+  for (int a = 0; a < Cfg::kNA; ++a)
 #pragma unroll
-      for (int b = 0; b < kNBMax; ++b) acc[a][b] = tm_f32x16{};
-    auto run = [&](auto rb_c) {
-      constexpr int RB = decltype(rb_c)::value;
-      using S = SkinnyShape<Cfg, RB>;
+    for (int b = 0; b < kNBMax; ++b) acc[a][b] = tm_f32x16{};
+  auto run = [&](auto rb_c) {
+    constexpr int RB = decltype(rb_c)::value;
+    using S = SkinnyShape<Cfg, RB>;
+    auto stream = [&](auto once_c) {
+      constexpr bool kOnce = decltype(once_c)::value;
       if (KT / SUB >= S::kDeep)
-        skinny_block<DT, Cfg, RB, S::kDeep, ONCE>(w_src, w_step, x_src, x_step, KT, a_off, lds0, lds, acc);
+        skinny_block<DT, Cfg, RB, S::kDeep, kOnce>(w_src, w_step, x_src, x_step, KT, a_off, lds0, lds, acc);
       else
-        skinny_block<DT, Cfg, RB, S::kShallow, ONCE>(w_src, w_step, x_src, x_step, KT, a_off, lds0, lds, acc);
+        skinny_block<DT, Cfg, RB, S::kShallow, kOnce>(w_src, w_step, x_src, x_step, KT, a_off, lds0, lds, acc);
     };
-    if (rows <= 16) run(std::integral_constant<int, 16>{});
-    else if (Cfg::RBMAX == 32 || rows <= 32) run(std::integral_constant<int, 32>{});
-    else run(std::integral_constant<int, Cfg::RBMAX>{});
-    // lane: activation row lane % 32 of each B operand, weight rows 8 (i / 4)
-    // + 4 (lane / 32) + i % 4 of each A operand: runs of 4 consecutive columns
+    if (PB && once) stream(std::integral_constant<bool, PB>{});
+    else stream(std::false_type{});
+  };
+  if (rows <= 16) run(std::integral_constant<int, 16>{});
+  else if (Cfg::RBMAX == 32 || rows <= 32) run(std::integral_constant<int, 32>{});
+  else run(std::integral_constant<int, Cfg::RBMAX>{});
+  // lane: activation row lane % 32 of each B operand, weight rows 8 (i / 4)
+  // + 4 (lane / 32) + i % 4 of each A operand: runs of 4 consecutive columns
 #pragma unroll
-    for (int b = 0; b < kNBMax; ++b) {
-      const int tr = 32 * b + (lane & 31);
-      if (tr < rows && (rows > 16 || tr < 16)) {
-        const int gr = r0 + rb + tr;
+  for (int b = 0; b < kNBMax; ++b) {
+    const int tr = 32 * b + (lane & 31);
+    if (tr < rows && (rows > 16 || tr < 16)) {
+      const int gr = r0 + rb + tr;
 #pragma unroll
-        for (int u = 0; u < CW / 8; ++u) {
-          const int col = n0 + 8 * u + 4 * (lane >> 5);
-          float v[4];
+      for (int u = 0; u < CW / 8; ++u) {
+        const int col = n0 + 8 * u + 4 * (lane >> 5);
+        float v[4];
 #pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            if constexpr (MODE == kModeUp) {
-              const float g = tm_round<DT>(acc[0][b][4 * u + i]);
-              const float up = CW == 32 ? acc[Cfg::kNA - 1][b][4 * u + i] : acc[0][b][(CW / 2 + 4 * u + i) & 15];
-              v[i] = g * __builtin_amdgcn_rcpf(1.f + __expf(-g)) * up;
-            } else {
-              v[i] = acc[u / 4][b][(4 * u + i) & 15];
-            }
+        for (int i = 0; i < 4; ++i) {
+          if constexpr (MODE == kModeUp) {
+            const float g = tm_round<DT>(acc[0][b][4 * u + i]);
+            const float up = CW == 32 ? acc[Cfg::kNA - 1][b][4 * u + i] : acc[0][b][(CW / 2 + 4 * u + i) & 15];
+            v[i] = g * __builtin_amdgcn_rcpf(1.f + __expf(-g)) * up;
+          } else {
+            v[i] = acc[u / 4][b][(4 * u + i) & 15];
           }
-          if constexpr (MODE == kModeDown) {
-            if (addend != nullptr) {  // dense rows only
-              const uint2 a = *reinterpret_cast<const uint2 *>(addend + (int64_t)gr * ld_add + col);
-              const T *ae = reinterpret_cast<const T *>(&a);
-#pragma unroll
-              for (int i = 0; i < 4; ++i) v[i] += Elem<DT>::to_f(ae[i]);
-            }
-          }
-          uint2 r;
-          T *re = reinterpret_cast<T *>(&r);
-#pragma unroll
-          for (int i = 0; i < 4; ++i) re[i] = Elem<DT>::from_f(v[i]);
-          T *dst;
-          if constexpr (PB && MODE == kModeUp)  // tile y of the intermediate in the down GEMM's stage order
-            dst = C + y * (int64_t)BM * ldc + (col / BK) * (BM * BK) +
-                  ((rb + tr) * kCPR + swz_chunk(rb + tr, (col % BK) / 8)) * 8 + col % 8;
-          else
-            dst = C + (c_rows ? c_rows[gr] + col : (int64_t)gr * ldc + col);
-          *reinterpret_cast<uint2 *>(dst) = r;
         }
+        if constexpr (MODE == kModeDown) {
+          if (addend != nullptr) {  // dense rows only
+            const uint2 a = *reinterpret_cast<const uint2 *>(addend + (int64_t)gr * ld_add + col);
+            const T *ae = reinterpret_cast<const T *>(&a);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) v[i] += Elem<DT>::to_f(ae[i]);
+          }
+        }
+        uint2 r;
+        T *re = reinterpret_cast<T *>(&r);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) re[i] = Elem<DT>::from_f(v[i]);
+        T *dst;
+        if constexpr (PB && MODE == kModeUp)  // tile y of the intermediate in the down GEMM's stage order
+          dst = C + y * (int64_t)BM * ldc + (col / BK) * (BM * BK) +
+                ((rb + tr) * kCPR + swz_chunk(rb + tr, (col % BK) / 8)) * 8 + col % 8;
+        else
+          dst = C + (c_rows ? c_rows[gr] + col : (int64_t)gr * ldc + col);
+        *reinterpret_cast<uint2 *>(dst) = r;
       }
     }
   }
@@ -957,16 +992,12 @@ void launch_skinny(const void *A, int64_t lda, const int32_t *a_rows, const void
   using T = typename Elem<DT>::T;
   const int pack_bn = Cfg::MODE == kModeUp ? kMinBN : down_bn(N);
   const bool grouped = ts.tiles != nullptr;
-  const int split = grouped ? 0 : BM / Cfg::RBMAX;
-  const int64_t blocks = grouped ? tiles : tm_cdiv(ts.rows, Cfg::RBMAX);
-  auto launch = [&](auto once_c) {
-    hipLaunchKernelGGL((skinny_gemm_kernel<DT, Cfg, PB, decltype(once_c)::value>),
-                       dim3((unsigned)(blocks * (N / Cfg::CW))), dim3(64), 0, s, static_cast<const T *>(A), lda, a_rows,
-                       static_cast<const T *>(B0), static_cast<const T *>(B1), b_expert, K, N / Cfg::CW, pack_bn, split,
-                       ts, static_cast<T *>(C), ldc, c_rows, static_cast<const T *>(addend), ld_add);
-  };
-  if (PB && grouped) launch(std::integral_constant<bool, PB>{});
-  else launch(std::false_type{});
+  // grouped: a row block per tile, and as many more as the rows can have past them
+  const int64_t blocks = grouped ? tiles + (ts.rows - 1) / Cfg::RBMAX : tm_cdiv(ts.rows, Cfg::RBMAX);
+  hipLaunchKernelGGL((skinny_gemm_kernel<DT, Cfg, PB>), dim3((unsigned)(blocks * (N / Cfg::CW))), dim3(64), 0, s,
+                     static_cast<const T *>(A), lda, a_rows, static_cast<const T *>(B0), static_cast<const T *>(B1),
+                     b_expert, K, N / Cfg::CW, pack_bn, (int)tiles, ts, static_cast<T *>(C), ldc, c_rows,
+                     static_cast<const T *>(addend), ld_add);
 }
 
 template <int DT, int MODE, int BN, bool PB>
@@ -1030,7 +1061,8 @@ int dense_plan(int64_t rows, int32_t hidden, int32_t inter) {
 // The plan of a grouped call, from the most rows per expert that it can have
 // on average (the counts are on the device): measured us per call, waves |
 // tiles, at 12.5 (128 experts, 2048 x 768): 205 | 203, at 18.8 (64 experts,
-// 2560 x 1536): 292 | 264, at 9.4: 235 | 243, at 0.5: 51 | 55.
+// 2560 x 1536): 292 | 264, at 9.4: 235 | 243, at 0.5: 51 | 55.  Rows need not be
+// even for it: the wave kernel spreads an expert's rows in blocks of 32.
 int grouped_plan(int64_t max_rows, int32_t n_experts) {
   return max_rows <= 12 * (int64_t)n_experts ? kPlanWave : kPlanTile;
 }
@@ -1195,7 +1227,7 @@ int grouped_swiglu_impl(int32_t dtype, const void *x, int64_t ld_x, int32_t hidd
   TM_REQUIRE(workspace != nullptr && workspace_bytes >= need && tm_aligned16(workspace), TM_EWORKSPACE,
              "tm_grouped_swiglu: workspace %zu bytes < %zu", workspace_bytes, need);
   const int64_t t_max = tm_group_slots_tiles(max_rows, n_experts);
-  const TileSrc ts{tiles, expert_offsets, t_max, 0};
+  const TileSrc ts{tiles, expert_offsets, t_max, (int32_t)max_rows};
   return swiglu_impl(dtype, x, ld_x, row_token, hidden, inter, w1, w3, w2, ts, max_rows < t_max ? max_rows : t_max,
                      out, 0, row_out, workspace, nullptr, 0, packed, grouped_plan(max_rows, n_experts),
                      tm_hip_stream(stream));  // (a tile holds at least one row)

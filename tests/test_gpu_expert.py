@@ -411,3 +411,39 @@ def test_grouped_rows_equal_dense_rows(hip_device, n, k, e, h, inter):
             if b.numel():
                 y = expert_swiglu(x[b.to(dev)].contiguous(), *(w[ex] for w in ws))
                 assert torch.equal(y, slot[b.to(dev), s.to(dev)]), (packed, ex)
+
+
+@pytest.mark.parametrize("n,k,e,h,inter,how", [(300, 4, 128, 384, 256, "one popular"), (300, 1, 64, 2560, 1536, "one"),
+                                               (192, 8, 128, 256, 128, "eight"), (1000, 1, 128, 128, 384, "one"),
+                                               (33, 4, 16, 256, 256, "one popular"), (70, 9, 90, 256, 256, "steps")])
+@pytest.mark.parametrize("packed", [True, False])
+def test_grouped_few_rows_on_average_uneven(hip_device, n, k, e, h, inter, how, packed):
+    """At most 12 rows per expert on average, but many on some: several
+    32-row blocks of a tile, several 256-row tiles of an expert, whichever
+    block of workgroups takes them; the dense call's rows bit for bit."""
+    from table_moe.ops import GroupedExperts, expert_swiglu
+
+    assert n * k <= 12 * e
+    dev = hip_device
+    g = torch.Generator().manual_seed(5 + n)
+    x = torch.randn(n, h, generator=g).to(torch.bfloat16).to(dev)
+    ws = [t.to(dev) for t in _weights(g, e, h, inter, torch.bfloat16)]
+    ids = torch.randint(0, e, (n, k), generator=g)
+    if how == "one popular":
+        ids[:, 0] = e - 1
+    elif how == "one":
+        ids[:] = 3
+    elif how == "eight":
+        ids[:] = torch.arange(8) * 5
+    else:  # 0, 1, 2, .. rows on successive experts
+        ids[:] = torch.repeat_interleave(torch.arange(e), torch.arange(e))[: n * k].view(n, k)
+    mask = torch.ones(n, k, dtype=torch.bool)
+    mask[n // 2, 0] = False
+    slot = torch.full((n, k, h), 5.0, dtype=torch.bfloat16, device=dev)
+    GroupedExperts(*ws, packed=packed).forward(x, ids.to(dev), mask.to(dev), slot)
+    assert bool((slot[~mask.to(dev)] == 5.0).all())
+    for ex in ids.unique().tolist():
+        b, s = torch.where(mask & (ids == ex))
+        if b.numel():
+            y = expert_swiglu(x[b.to(dev)].contiguous(), *(w[ex] for w in ws))
+            assert torch.equal(y, slot[b.to(dev), s.to(dev)]), ex
