@@ -214,20 +214,32 @@ __global__ __launch_bounds__(64) void skinny_gemm_kernel(
     const int64_t nt = ts.tiles[1] < ts.t_max ? ts.tiles[1] : ts.t_max;
     if (blk >= slots) {
       int u = (int)(blk - slots);  // this is further row block u
-      for (int64_t t0 = 0;; t0 += 64) {
+      if (u >= (ts.tiles[0] - nt) / Cfg::RBMAX) return;  // uniform: more than the rows can have past their tiles' first
+      const int32_t *const row0 = ts.tiles + 2 + ts.t_max;  // tiles' rows follow each other
+      for (int64_t t0 = 0;; t0 += 256) {  // four tiles per lane
         if (t0 >= nt) return;  // uniform: there are fewer
-        const int64_t t = t0 + lane;
-        int more = 0;
-        if (t < nt) {
-          const int rows = ts.expert_offsets[ts.tiles[2 + t] + 1] - ts.tiles[2 + ts.t_max + t];
-          more = ((rows < BM ? rows : BM) - 1) / Cfg::RBMAX;
+        const int64_t t = t0 + 4 * lane;
+        int at[5], more[4], sum = 0;
+#pragma unroll
+        for (int j = 0; j < 5; ++j) at[j] = row0[t + j < nt ? t + j : nt - 1];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          more[j] = t + j < nt ? ((t + j + 1 < nt ? at[j + 1] : ts.tiles[0]) - at[j] - 1) / Cfg::RBMAX : 0;
+          sum += more[j];
         }
-        const int upto = (int)tm_wave_incl_scan((uint32_t)more);
+        const int upto = (int)tm_wave_incl_scan((uint32_t)sum);
         const int total = __builtin_amdgcn_readlane(upto, 63);
         if (u < total) {  // uniform
           const int l = __builtin_ctzll(__ballot(u < upto));
-          y = t0 + l;
-          rb = (u - __builtin_amdgcn_readlane(upto - more, l) + 1) * Cfg::RBMAX;
+          u -= __builtin_amdgcn_readlane(upto - sum, l);
+          int j = 0;
+          for (int m = __builtin_amdgcn_readlane(more[0], l); j < 3 && u >= m;) {
+            u -= m;
+            ++j;
+            m = __builtin_amdgcn_readlane(j == 1 ? more[1] : j == 2 ? more[2] : more[3], l);
+          }
+          y = t0 + 4 * l + j;
+          rb = (u + 1) * Cfg::RBMAX;
           break;
         }
         u -= total;
@@ -1062,9 +1074,13 @@ int dense_plan(int64_t rows, int32_t hidden, int32_t inter) {
 // on average (the counts are on the device): measured us per call, waves |
 // tiles, at 12.5 (128 experts, 2048 x 768): 205 | 203, at 18.8 (64 experts,
 // 2560 x 1536): 292 | 264, at 9.4: 235 | 243, at 0.5: 51 | 55.  Rows need not be
-// even for it: the wave kernel spreads an expert's rows in blocks of 32.
-int grouped_plan(int64_t max_rows, int32_t n_experts) {
-  return max_rows <= 12 * (int64_t)n_experts ? kPlanWave : kPlanTile;
+// even for it: the wave kernel spreads an expert's rows in blocks of 32, up to
+// the work of one expert with all of them that the dense waves are good for: even
+// routing | all rows on one expert, waves against tiles, 768 rows of 64 experts,
+// 2560 x 1536: 262 | 70 against 260 | 53; 1536 rows of 128, 2560 x 1536: 543 | 124
+// against 502 | 62; 3072 rows of 1024, 1024 x 256: 280 | 49 against 302 | 40.
+int grouped_plan(int64_t max_rows, int32_t n_experts, int32_t hidden, int32_t inter) {
+  return max_rows <= 12 * (int64_t)n_experts && (double)max_rows * hidden * inter <= 3.1e9 ? kPlanWave : kPlanTile;
 }
 
 // The two GEMMs of the MLP over the rows the tile source names; `addend`
@@ -1229,7 +1245,7 @@ int grouped_swiglu_impl(int32_t dtype, const void *x, int64_t ld_x, int32_t hidd
   const int64_t t_max = tm_group_slots_tiles(max_rows, n_experts);
   const TileSrc ts{tiles, expert_offsets, t_max, (int32_t)max_rows};
   return swiglu_impl(dtype, x, ld_x, row_token, hidden, inter, w1, w3, w2, ts, max_rows < t_max ? max_rows : t_max,
-                     out, 0, row_out, workspace, nullptr, 0, packed, grouped_plan(max_rows, n_experts),
+                     out, 0, row_out, workspace, nullptr, 0, packed, grouped_plan(max_rows, n_experts, hidden, inter),
                      tm_hip_stream(stream));  // (a tile holds at least one row)
 }
 
