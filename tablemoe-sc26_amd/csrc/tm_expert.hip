@@ -1064,8 +1064,12 @@ void swiglu_launch(const void *x, int64_t ld_x, const int32_t *row_token, int32_
 // (64) rows; measured crossovers (hidden x inter 2048 x 768 | 2560 x 1536, us
 // per call): 128 rows 14 | 21 against 26 | 34 with 64-row waves and 44 | 64
 // with tiles; 512 rows 22 | 54, 27 | 37, 41 | 65; 2048 rows 81 | 192, 53 | 132,
-// 43 | 68.
+// 43 | 68.  Small weights: from 32 tiles of many rows on, tiles fill the chip and
+// read the weights less often: 128 x 128 4096 rows 8.9 | 12.4 | 11.5, 16384 17.7 |
+// 16.3 | 13.0, 65536 44 | 41 | 26; 256 x 512 2048 rows 14.7 | 17.2 | 17.3, 4096 22 | 21 |
+// 18.6, 16384 61 | 47 | 32.
 int dense_plan(int64_t rows, int32_t hidden, int32_t inter) {
+  if (rows > 2048 && tm_cdiv(rows, BM) * (inter / kMinBN) >= 32) return kPlanTile;
   const double work = (double)rows * hidden * inter;
   return work <= 1.1e9 ? kPlanWave : work <= 3e9 ? kPlanWave64 : kPlanTile;
 }

@@ -447,3 +447,46 @@ def test_grouped_few_rows_on_average_uneven(hip_device, n, k, e, h, inter, how, 
         if b.numel():
             y = expert_swiglu(x[b.to(dev)].contiguous(), *(w[ex] for w in ws))
             assert torch.equal(y, slot[b.to(dev), s.to(dev)]), ex
+
+
+@pytest.mark.parametrize("rows,h,inter", [(65536, 128, 128), (16384, 512, 256)])
+def test_dense_many_rows_small_weights_cost(hip_device, rows, h, inter):
+    """A dense call takes about as long as the grouped GEMMs of one expert with
+    the same rows, which run as tiles: one wave per 32 or 64 rows and column
+    group, which re-read the weights for each, took 1.6 times as long."""
+    from table_moe import _native as N
+    from table_moe.ops import GroupedExperts, expert_swiglu
+
+    dev = hip_device
+    g = torch.Generator().manual_seed(3)
+    x = torch.randn(rows, h, generator=g).to(torch.bfloat16).to(dev)
+    w = [t.to(dev) for t in _weights(g, 1, h, inter, torch.bfloat16)]
+    ge = GroupedExperts(*w, packed=False)
+    ids = torch.zeros(rows, 1, dtype=torch.long, device=dev)
+    mask = torch.ones(rows, 1, dtype=torch.bool, device=dev)
+    slot = torch.empty(rows, 1, h, dtype=torch.bfloat16, device=dev)
+    ge.forward(x, ids, mask, slot)
+    offs, row_token, row_out, tiles = ge.group(ids, mask, slot)
+    ws = torch.empty(rows * inter, dtype=torch.bfloat16, device=dev)
+    out = torch.empty_like(x)
+    dense = [t[0] for t in w]
+
+    def us(call):
+        for _ in range(3):
+            call()
+        times = []
+        for _ in range(15):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            for _ in range(20):
+                call()
+            b.record()
+            torch.cuda.synchronize()
+            times.append(a.elapsed_time(b) * 50)
+        return sorted(times)[7]
+
+    grouped = us(lambda: N.call("tm_grouped_swiglu", N.dtype_tag(x.dtype), N.ptr(x), h, h, inter, 1, N.ptr(w[0]),
+                                N.ptr(w[1]), N.ptr(w[2]), rows, N.ptr(offs), N.ptr(row_token), N.ptr(row_out),
+                                N.ptr(tiles), N.ptr(slot), N.ptr(ws), 2 * ws.numel(), N.stream(dev)))
+    assert us(lambda: expert_swiglu(x, *dense, out=out)) < 1.3 * grouped
+    assert torch.equal(out, slot.view(rows, h))
