@@ -380,7 +380,11 @@ int tm_decode_combine_update(int32_t dtype, int32_t top_k, int32_t hidden, const
  * 0 and leave the normalisation.  p = softmax over t in fp32;
  * out[b*ld_out + j] = mean over heads of p at key n_keys - out_len + j.
  * head_dim in {64, 128, 192, 256}; n_heads <= 256; n_keys <= 524288.
- * Workspace: tm_importance_workspace_size (scores and chunk statistics).
+ * Workspace: tm_importance_workspace_size (scores and chunk statistics),
+ * never less for more keys; down to the scores and one statistic per head and
+ * 512 keys is taken as well (4 * batch * n_heads * n_keys bytes rounded up to
+ * 256, and 8 * batch * n_heads * ceil(n_keys / 512)), short prompts then run in
+ * longer chunks.
  * ====================================================================== */
 #define TM_SCORE_MODEL 0
 #define TM_SCORE_F32 1

@@ -23,8 +23,10 @@
 // workgroups share them: chunks of 64 keys (260 workgroups at 4099 keys of 4
 // KV heads) instead of 512, and 64 keys x 4 head quarters instead of 256 keys
 // x all heads (65 workgroups instead of 17).  Chunks of 512 keys stay for long
-// prompts, whose statistics every workgroup of the mean reads.  4099 keys, 32
-// heads on 4 KV heads (us): 14.8 + 16.3 before, 5.9 + 6.0 now.
+// prompts, whose statistics every workgroup of the mean reads, and for calls
+// whose workspace holds no more.  32 heads on 4 KV heads, us before (one head per
+// workgroup, 256 keys x all heads) and now: 4099 keys 14.8 + 16.3, 5.9 + 6.0; both
+// together 16384 keys 39, 22; 16385 51, 24; 131072 141, 65; 524288 893, 355.
 #include "tm_internal.h"
 #include "tm_route_dev.h"
 
@@ -40,7 +42,13 @@ constexpr int kMaxKeys = 512 * kMaxChunks;
 constexpr int kMeanKeys = 64;      // output keys per workgroup of mean_kernel
 constexpr int kBatch = 8;          // scores and statistics loaded per round trip
 
-inline int chunk_keys(int64_t n_keys) { return n_keys <= kShortKeys ? 64 : 512; }
+// Workspace of a call with chunks of `chunk` keys: scores, then statistics.
+inline size_t score_bytes(int64_t batch, int n_heads, int64_t n_keys) {
+  return ((size_t)batch * n_heads * n_keys * sizeof(float) + 255) / 256 * 256;
+}
+inline size_t ws_bytes(int64_t batch, int n_heads, int64_t n_keys, int chunk) {
+  return score_bytes(batch, n_heads, n_keys) + (size_t)batch * n_heads * tm_cdiv(n_keys, chunk) * sizeof(float2);
+}
 
 // Maximum / sum over the wave in every lane (DPP: row shifts, row broadcasts).
 __device__ __forceinline__ float wave_max_f(float v) {
@@ -220,11 +228,10 @@ __global__ __launch_bounds__(kThreads) void mean_kernel(const float *__restrict_
 }
 
 template <int DT, int CH>
-void launch_scores(const void *q, int64_t qs_b, int64_t qs_h, const void *k, int64_t ks_b, int64_t ks_s, int64_t ks_h,
+void launch_scores(int chunk, const void *q, int64_t qs_b, int64_t qs_h, const void *k, int64_t ks_b, int64_t ks_s, int64_t ks_h,
                    int64_t batch, int n_heads, int groups, int64_t n_keys, float scale, int score_mode,
                    const uint8_t *key_mask, int64_t km_b, float *sc, float2 *stats, hipStream_t s) {
   using T = typename Elem<DT>::T;
-  const int chunk = chunk_keys(n_keys);
   auto launch = [&](auto hg_c, auto passes_c) {
     constexpr int HG = decltype(hg_c)::value, PASSES = decltype(passes_c)::value;
     const dim3 grid((unsigned)tm_cdiv(n_keys, chunk), (unsigned)(n_heads / HG), (unsigned)batch);
@@ -247,9 +254,10 @@ void launch_scores(const void *q, int64_t qs_b, int64_t qs_h, const void *k, int
 
 extern "C" size_t tm_importance_workspace_size(int64_t batch, int32_t n_heads, int64_t n_keys) {
   if (batch <= 0 || n_heads <= 0 || n_keys <= 0) return 0;
-  const size_t scores = (size_t)batch * n_heads * n_keys * sizeof(float);
-  const size_t stats = (size_t)batch * n_heads * tm_cdiv(n_keys, chunk_keys(n_keys)) * sizeof(float2);
-  return (scores + 255) / 256 * 256 + stats;
+  // never less than that of a shorter prompt, so one buffer serves every prompt up to the one it was sized for
+  const size_t chunks64 = ws_bytes(batch, n_heads, n_keys < kShortKeys ? n_keys : kShortKeys, 64);
+  const size_t chunks512 = ws_bytes(batch, n_heads, n_keys, 512);
+  return chunks64 > chunks512 ? chunks64 : chunks512;
 }
 
 extern "C" int tm_last_query_importance(int32_t dtype, const void *q, int64_t qs_b, int64_t qs_h, const void *k,
@@ -269,13 +277,14 @@ extern "C" int tm_last_query_importance(int32_t dtype, const void *q, int64_t qs
              "tm_last_query_importance: bad score mode");
   if (batch == 0 || n_keys == 0 || out_len == 0) return TM_OK;
   TM_REQUIRE(q && k && out, TM_EINVAL_ARG, "tm_last_query_importance: null pointer");
-  const size_t need = tm_importance_workspace_size(batch, n_heads, n_keys);
+  const size_t need = ws_bytes(batch, n_heads, n_keys, 512);
   TM_REQUIRE(workspace != nullptr && workspace_bytes >= need && tm_aligned16(workspace), TM_EWORKSPACE,
              "tm_last_query_importance: workspace %zu bytes < %zu", workspace_bytes, need);
   hipStream_t s = tm_hip_stream(stream);
+  // short prompts run in chunks of 64 keys where their statistics fit
+  const int chunk = n_keys <= kShortKeys && workspace_bytes >= ws_bytes(batch, n_heads, n_keys, 64) ? 64 : 512;
   float *sc = static_cast<float *>(workspace);
-  const size_t sc_bytes = ((size_t)batch * n_heads * n_keys * sizeof(float) + 255) / 256 * 256;
-  float2 *stats = reinterpret_cast<float2 *>(static_cast<char *>(workspace) + sc_bytes);
+  float2 *stats = reinterpret_cast<float2 *>(static_cast<char *>(workspace) + score_bytes(batch, n_heads, n_keys));
   const int groups = n_heads / n_kv_heads;
   return TM_DISPATCH_DTYPE(dtype, DT, [&] {
     const int E = Elem<DT>::kBytes;
@@ -286,16 +295,16 @@ extern "C" int tm_last_query_importance(int32_t dtype, const void *q, int64_t qs
       TM_REQUIRE(score_mode == TM_SCORE_F32, TM_EINVAL_ARG, "tm_last_query_importance: fp32 inputs score in fp32");
     }
     switch (head_dim) {
-      case 64: launch_scores<DT, 1>(q, qs_b, qs_h, k, ks_b, ks_s, ks_h, batch, n_heads, groups, n_keys, scale, score_mode, key_mask, km_b, sc, stats, s); break;
-      case 128: launch_scores<DT, 2>(q, qs_b, qs_h, k, ks_b, ks_s, ks_h, batch, n_heads, groups, n_keys, scale, score_mode, key_mask, km_b, sc, stats, s); break;
-      case 192: launch_scores<DT, 3>(q, qs_b, qs_h, k, ks_b, ks_s, ks_h, batch, n_heads, groups, n_keys, scale, score_mode, key_mask, km_b, sc, stats, s); break;
-      default: launch_scores<DT, 4>(q, qs_b, qs_h, k, ks_b, ks_s, ks_h, batch, n_heads, groups, n_keys, scale, score_mode, key_mask, km_b, sc, stats, s); break;
+      case 64: launch_scores<DT, 1>(chunk, q, qs_b, qs_h, k, ks_b, ks_s, ks_h, batch, n_heads, groups, n_keys, scale, score_mode, key_mask, km_b, sc, stats, s); break;
+      case 128: launch_scores<DT, 2>(chunk, q, qs_b, qs_h, k, ks_b, ks_s, ks_h, batch, n_heads, groups, n_keys, scale, score_mode, key_mask, km_b, sc, stats, s); break;
+      case 192: launch_scores<DT, 3>(chunk, q, qs_b, qs_h, k, ks_b, ks_s, ks_h, batch, n_heads, groups, n_keys, scale, score_mode, key_mask, km_b, sc, stats, s); break;
+      default: launch_scores<DT, 4>(chunk, q, qs_b, qs_h, k, ks_b, ks_s, ks_h, batch, n_heads, groups, n_keys, scale, score_mode, key_mask, km_b, sc, stats, s); break;
     }
     TM_LAUNCH_CHECK("tm_last_query_importance(scores)");
     int lanes_log2 = 0;  // lanes per head that combine its chunk statistics
     while (lanes_log2 < 6 && (kThreads >> (lanes_log2 + 1)) >= n_heads) ++lanes_log2;
     hipLaunchKernelGGL(mean_kernel, dim3((unsigned)tm_cdiv(out_len, kMeanKeys), (unsigned)batch), dim3(kThreads), 0, s,
-                       sc, stats, (int)n_heads, lanes_log2, (int)tm_cdiv(n_keys, chunk_keys(n_keys)), n_keys, key_mask,
+                       sc, stats, (int)n_heads, lanes_log2, (int)tm_cdiv(n_keys, chunk), n_keys, key_mask,
                        km_b, out_len, out, ld_out);
     TM_LAUNCH_CHECK("tm_last_query_importance(mean)");
     return TM_OK;

@@ -159,3 +159,18 @@ def test_noalloc_limit_without_device(lib):
     io.n_tokens = 0
     assert lib.tm_table_forward_noalloc(C.byref(t), C.byref(io), None) == N.TM_OK
     assert lib.tm_table_forward_noalloc(None, C.byref(io), None) == N.TM_EINVAL_ARG
+
+
+def test_importance_workspace_grows_with_the_prompt(lib):
+    """A buffer for the longest prompt serves every shorter one: the size never
+    falls from one length to the next, across the change of the chunk length
+    too, and covers the scores and a statistic per 64 keys up to 16384."""
+    for b, h in ((1, 32), (3, 5)):
+        size = [lib.tm_importance_workspace_size(b, h, n) for n in list(range(1, 1200)) + list(range(16000, 18500, 7))
+                + [16383, 16384, 16385, 17000, 32768, 524288]]
+        assert all(x <= y for x, y in zip(size[:1198], size[1:1199]))
+        tail = sorted(zip(list(range(16000, 18500, 7)) + [16383, 16384, 16385, 17000, 32768, 524288], size[1199:]))
+        assert all(x[1] <= y[1] for x, y in zip(tail, tail[1:]))
+        at = dict(tail)
+        assert at[16384] == (4 * b * h * 16384 + 255) // 256 * 256 + 8 * b * h * 256
+        assert at[16385] >= at[16384]

@@ -120,3 +120,35 @@ def test_importance_scores_of_minus_infinity(hip_device, s, lo, hi):
     got = last_query_importance(q.to(dev), ks.to(dev), hkv, d ** -0.5, True, None, s)
     torch.cuda.synchronize()
     np.testing.assert_allclose(np64(got), want, rtol=1e-4, atol=1e-9)
+
+
+@pytest.mark.parametrize("s", [65, 4099, 16384])
+def test_importance_in_the_least_workspace(hip_device, s):
+    """The scores and a statistic per 512 keys are enough (one byte less is
+    refused): the same importance up to the order of the sums, and nothing past
+    the workspace is written."""
+    from table_moe import _native as N
+    from table_moe.utils.importance import last_query_importance
+
+    g = torch.Generator().manual_seed(s)
+    h, hkv, d = 8, 2, 128
+    dev = hip_device
+    q = torch.randn(1, h, d, generator=g).to(torch.bfloat16).to(dev)
+    ks = torch.randn(1, s, hkv, d, generator=g).to(torch.bfloat16).to(dev)
+    want = last_query_importance(q, ks, hkv, d ** -0.5, True)
+    need = (4 * h * s + 255) // 256 * 256 + 8 * h * ((s + 511) // 512)
+    assert need < N.lib().tm_importance_workspace_size(1, h, s)
+    ws = torch.full((need + 4096,), 77, dtype=torch.uint8, device=dev)
+    out = torch.empty(1, s, device=dev)
+
+    def call(nbytes):
+        N.call("tm_last_query_importance", N.dtype_tag(q.dtype), q.data_ptr(), q.stride(0), q.stride(1), ks.data_ptr(),
+               ks.stride(0), ks.stride(1), ks.stride(2), 1, h, hkv, d, s, d ** -0.5, N.TM_SCORE_F32, None, 0, s,
+               out.data_ptr(), s, ws.data_ptr(), nbytes, N.stream(dev))
+
+    with pytest.raises(ValueError):
+        call(need - 1)
+    call(need)
+    torch.cuda.synchronize()
+    np.testing.assert_allclose(np64(out), np64(want), rtol=1e-5, atol=0)
+    assert bool((ws[need:] == 77).all())
