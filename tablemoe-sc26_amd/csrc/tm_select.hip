@@ -36,8 +36,9 @@ __device__ __forceinline__ uint32_t block_exclusive_scan(uint32_t v, uint32_t *w
 
 // ---------------------------------------------------------------------------
 // (3) keep the n_keep largest scores; ties -> lower token index.
-// One workgroup; thread t owns the contiguous token range [t*per, (t+1)*per)
-// and caches its order-preserving uint32 keys in registers (n <= 16384).
+// For n > 16384 (keep_rank_kernel below takes the others).  One workgroup;
+// thread t owns the contiguous token range [t*per, (t+1)*per) and reads its
+// scores again in each pass, as order-preserving uint32 keys.
 // Four 8-bit radix passes find the boundary key T and how many copies of T
 // are kept: each pass builds a 256-bin histogram of the keys still matching
 // the known high bits (one private histogram per wave, so nearby distances
@@ -48,7 +49,6 @@ __device__ __forceinline__ uint32_t block_exclusive_scan(uint32_t v, uint32_t *w
 // ---------------------------------------------------------------------------
 constexpr int kSelThreads = 1024;
 constexpr int kSelWaves = kSelThreads / 64;
-constexpr int kSelRegs = 16;
 
 __global__ __launch_bounds__(kSelThreads) void keep_select_kernel(const float *__restrict__ score,
                                                                   int64_t n, int64_t ld,
@@ -70,37 +70,16 @@ __global__ __launch_bounds__(kSelThreads) void keep_select_kernel(const float *_
     for (int64_t i = lo; i < hi; ++i) out[i] = v;
     return;
   }
-  const bool cached = per <= kSelRegs;  // uniform
-  uint32_t keys[kSelRegs];
-  if (cached) {
-#pragma unroll
-    for (int j = 0; j < kSelRegs; ++j) keys[j] = (j < cnt) ? tm_orderable(score[(lo + j) * ld]) : 0u;
-  }
-  auto key_at = [&](int j) -> uint32_t {
-    if (cached) {
-      uint32_t k = 0;
-#pragma unroll
-      for (int u = 0; u < kSelRegs; ++u)
-        if (u == j) k = keys[u];
-      return k;
-    }
-    return tm_orderable(score[(lo + j) * ld]);
-  };
+  auto key_at = [&](int j) -> uint32_t { return tm_orderable(score[(lo + j) * ld]); };
 
   if (tid == 0) { s_prefix = 0; s_mask = 0; s_remaining = n_keep; }
   for (int shift = 24; shift >= 0; shift -= 8) {
     for (int b = lane; b < 256; b += 64) whist[wave][b] = 0;
     __syncthreads();
     const uint32_t prefix = s_prefix, mask = s_mask;
-    if (cached) {
-#pragma unroll
-      for (int j = 0; j < kSelRegs; ++j)
-        if (j < cnt && (keys[j] & mask) == prefix) atomicAdd(&whist[wave][(keys[j] >> shift) & 255u], 1u);
-    } else {
-      for (int j = 0; j < cnt; ++j) {
-        const uint32_t k = key_at(j);
-        if ((k & mask) == prefix) atomicAdd(&whist[wave][(k >> shift) & 255u], 1u);
-      }
+    for (int j = 0; j < cnt; ++j) {
+      const uint32_t k = key_at(j);
+      if ((k & mask) == prefix) atomicAdd(&whist[wave][(k >> shift) & 255u], 1u);
     }
     __syncthreads();
     if (tid < 256) {  // thread t sums bin t over the waves
