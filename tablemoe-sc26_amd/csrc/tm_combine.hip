@@ -197,7 +197,7 @@ __global__ __launch_bounds__(kThreads) void gather_combine_fast_kernel(
 // from the residual, sources added in order with fmaf, one rounding.
 // Keep decisions when the keep set is ranked in the combine: token b is
 // kept when fewer than n_keep tokens are ahead of it (a larger distance, or
-// the same at a lower index), the set the radix select gives.  One pass over
+// the same at a lower index), the set tm_keep_select gives.  One pass over
 // the n distances (contiguous, 16-byte aligned) serves the TPB tokens of the
 // workgroup (token b0 + g for g < TPB; TPB * 256 threads).
 struct RankKeep {
@@ -633,8 +633,8 @@ __global__ __launch_bounds__(kThreads) void gather_combine_kernel(
 // ---------------------------------------------------------------------------
 // combine_row for at most kSlotSrc sources (16-byte rows): every source load
 // of a chunk is issued before the first is used (the sources past nsrc read
-// the output row itself and are not added), so a token's rows stream in one
-// round trip instead of one per source.
+// the first source's row again, without any the output row, and are not
+// added), so a token's rows stream in one round trip instead of one per source.
 constexpr int kSlotSrc = 8;
 
 template <int DT>

@@ -441,9 +441,6 @@ __global__ __launch_bounds__(kTileThreads, 2) void tile_gemm_kernel(
   constexpr int NA = MODE == kModeUp ? 2 : BN / 128;  // 32-row weight operands per wave
   __shared__ uint4 ring[kTileLds / 16];
 
-  // Block b runs on XCD b % 8 (the dispatcher's round robin): the n_tiles
-  // column tiles of row tile y get ids 8 apart, so they share one XCD and its
-  // L2 copy of the tile's activation rows.
   // Work items: (row tile, column tile), n_tiles per row tile.  Item b of the
   // whole groups of 8 row tiles is row tile 8 (b / 8 / n_tiles) + b % 8, so a
   // row tile's items run on one XCD (the dispatcher's round robin) and share
@@ -622,7 +619,8 @@ __global__ __launch_bounds__(kTileThreads, 2) void tile_gemm_kernel(
     else if (nb == 3) run(std::integral_constant<int, 3>{}, once_c);
     else run(std::integral_constant<int, 4>{}, once_c);
   };
-  // Packed weights that no other row tile reads are loaded non-temporally.
+  // Packed weights that no other row tile reads are loaded non-temporally (the
+  // row ranges of a tile that is cut do read the same ones, at the same time).
   if (PB && once) run_nb(std::integral_constant<bool, PB>{});
   else run_nb(std::false_type{});
 
@@ -1134,7 +1132,7 @@ __global__ __launch_bounds__(kThreads) void pack_weights_kernel(const T *__restr
 }
 
 bool shapes_ok(int32_t hidden, int32_t inter) {
-  // multiples of 128: whole column tiles, and K in whole rounds of the 4-slot ring (4 stages of BK)
+  // multiples of 128: whole column tiles, and K an even number of two-stage steps (the wave kernel's rings)
   return hidden > 0 && inter > 0 && hidden % kMinBN == 0 && inter % kMinBN == 0 && (int64_t)inter * hidden <
          ((int64_t)1 << 30);
 }
@@ -1155,7 +1153,7 @@ extern "C" int tm_group_slots(const int64_t *ids, int64_t n_tokens, int32_t top_
   TM_REQUIRE(n_tokens * top_k < ((int64_t)1 << 31), TM_EINVAL_SHAPE, "tm_group_slots: too many slots");
   TM_REQUIRE(expert_offsets && tiles && (n_tokens == 0 || (ids && mask && row_token && row_out)), TM_EINVAL_ARG,
              "tm_group_slots: null pointer");
-  // tm_grouped_swiglu writes each row in 16-byte pieces from row_out
+  // tm_grouped_swiglu's contract: rows at 16-byte offsets of row_out (it writes them in 8-byte pieces)
   TM_REQUIRE(so_b % 8 == 0 && so_s % 8 == 0, TM_EINVAL_SHAPE,
              "tm_group_slots: output strides (%lld, %lld) must be multiples of 8 elements", (long long)so_b,
              (long long)so_s);

@@ -385,10 +385,12 @@ def test_dense_rows_do_not_depend_on_the_batch(hip_device, h, inter, dtype, pack
 @pytest.mark.parametrize("n,k,e,h,inter", [(1, 8, 128, 2048, 768), (64, 6, 64, 2560, 1536), (65, 8, 16, 384, 256),
                                            (300, 8, 4, 256, 128), (900, 2, 3, 128, 384)])
 def test_grouped_rows_equal_dense_rows(hip_device, n, k, e, h, inter):
-    """Grouped rows, packed and plain, whatever the rows per expert (a row or
-    two each; experts of one and of several 256-row tiles, experts without a
-    row, ids out of range), equal the dense call of the same rows bit for
-    bit; slots that are not recomputed keep their contents."""
+    """Grouped rows, packed and plain, equal the dense call of the same rows bit
+    for bit: in the wave kernel a row or two per expert and up to three 32-row
+    blocks (the first two shapes; more in
+    test_grouped_few_rows_on_average_uneven), in the tile kernel experts of
+    one and of several 256-row tiles; experts without a row, ids out of range.
+    Slots that are not recomputed keep their contents."""
     from table_moe.ops import GroupedExperts, expert_swiglu
 
     dev = hip_device

@@ -744,24 +744,34 @@ def test_search_topk_small_table_cost(hip_device, n, dim, k, small, large):
     assert us[0] < 0.6 * us[1], us
 
 
-def test_search_topk_blocks_nan_and_inf(hip_device):
-    """A NaN query gives no finite distance to any row but its own; infinite
-    centroids rank behind finite ones."""
+@pytest.mark.parametrize("n,c,dim,top_k", [(100, 300, 64, 4), (1100, 300, 128, 4), (100, 300, 256, 8)])
+@pytest.mark.parametrize("metric", ["l2", "dot"])
+def test_search_topk_blocks_nan_and_inf(hip_device, n, c, dim, top_k, metric):
+    """Lists of blocks and of centroids.  Infinite centroids rank behind finite
+    ones (l2).  A NaN query changes no row but its own, whose entries are the
+    first indices of the table and whose distances are no ranking: 0 (l2,
+    clamped) or NaN (dot)."""
     from table_moe.cache_engine import GlobalTable
 
     dev = hip_device
     g = _gen(5)
-    q = torch.randn(100, 64, generator=g).to(torch.bfloat16)
-    cents = torch.randn(300, 64, generator=g).to(torch.bfloat16)
-    cents[::2, 0] = float("inf")
-    tbl = GlobalTable(cents.to(dev), torch.zeros(300, 256, dtype=torch.bfloat16, device=dev),
-                      (torch.zeros(256, 64, dtype=torch.bfloat16, device=dev),
-                       torch.zeros(64, dtype=torch.bfloat16, device=dev)))
-    base_d, base_i = [t.clone() for t in tbl.search(q.to(dev), 4)]
-    assert (np64(base_i) % 2 == 1).all() and np.isfinite(np64(base_d)).all()
+    q = torch.randn(n, dim, generator=g).to(torch.bfloat16)
+    cents = torch.randn(c, dim, generator=g).to(torch.bfloat16)
+    if metric == "l2":
+        cents[::2, 0] = float("inf")
+    tbl = GlobalTable(cents.to(dev), torch.zeros(c, 256, dtype=torch.bfloat16, device=dev),
+                      (torch.zeros(256, dim, dtype=torch.bfloat16, device=dev),
+                       torch.zeros(dim, dtype=torch.bfloat16, device=dev)), metric=metric)
+    base_d, base_i = [t.clone() for t in tbl.search(q.to(dev), top_k)]
+    assert np.isfinite(np64(base_d)).all()
+    if metric == "l2":
+        assert (np64(base_i) % 2 == 1).all()
     bad = q.clone()
     bad[7] = float("nan")
-    d, i = tbl.search(bad.to(dev), 4)
+    d, i = tbl.search(bad.to(dev), top_k)
     torch.cuda.synchronize()
-    rows = np.arange(100) != 7
+    rows = np.arange(n) != 7
     assert torch.equal(i[rows], base_i[rows]) and torch.equal(d[rows], base_d[rows])
+    np.testing.assert_array_equal(np64(i[7]), np.arange(top_k))
+    nan_d = np64(d[7])
+    assert (nan_d == 0.0).all() if metric == "l2" else np.isnan(nan_d).all()
