@@ -127,7 +127,8 @@ static inline bool top1_tile(int dim, int top_k) { return top_k <= 1 && dim <= 1
 // 15 | 23.  d 256: 4000 of 1024: 24 | 40 against 55 | 80, of 14000 (3000): 70 | 133
 // against 76 | 122, of 16384 (10000): 244 | 503 against 220 | 351, (8000): 142 | 289
 // against 169 | 296; 768 of 8192: 27 | 46 against 28 | 47, of 12000: 33 | 57 against
-// 28 | 49; 65 of 12000: 19 | 30 against 20 | 33.
+// 28 | 49; 65 of 12000: 19 | 30 against 20 | 33, 200 of 16384: 24 | 38 against 23 | 42,
+// of 20480: 26 | 44 against 24 | 44.
 inline bool topk_blocks(int64_t n, int64_t c, int dim, int top_k) {
   if (dim == 64) return n <= 5120 || c >= (top_k > 4 ? 1408 : 1344);
   if (dim == 128) {
@@ -135,7 +136,7 @@ inline bool topk_blocks(int64_t n, int64_t c, int dim, int top_k) {
     if (n <= 2048) return tm_cdiv(n, kTileRows) * tm_cdiv(c, dma_rows(128)) > 256;  // past one round of CUs
     return c >= (n > 4096 ? 4096 : 3072);
   }
-  if (n <= 256) return c >= 16384;
+  if (n <= 256) return c >= (top_k > 4 ? 20480 : 16384);
   if (n <= 2048 || top_k > 4) return c >= 12000;
   return c >= (n > 5120 && n <= 8192 ? 24576 : 16384);
 }
