@@ -407,8 +407,11 @@ __global__ __launch_bounds__(64) void skinny_gemm_kernel(
 // that miss L2 behind the stream of weights (so weights that one workgroup
 // alone reads are loaded non-temporally: 5280 rows of 128 experts 272 -> 253
 // us; weights that several row tiles read are not: 510 against 594 us at 14.4k
-// rows of 64 experts), and, from ~150 rows per expert, by the matrix cores.  us
-// per call before (4 waves, one per SIMD, always 256 rows) -> now: hidden 2048,
+// rows of 64 experts).  With many rows per expert neither HBM nor the matrix
+// cores are at their limit (230 rows of 64 experts, hidden 2560, inter 1536: up
+// 797 TFLOP/s, weights at 3.5 TB/s, waves waiting half of the time, no bank
+// conflicts; 4096 dense rows 982 TFLOP/s): 6 operand reads per 8 products and a
+// barrier per stage on one workgroup per CU.  us per call before (4 waves, one per SIMD, always 256 rows) -> now: hidden 2048,
 // inter 768, 128 experts: 960 rows 287 -> 205, 5280 rows 310 -> 253, 19.2k rows
 // 409 -> 366; hidden 2560, inter 1536, 64 experts: 1800 rows 358 -> 287, 14.4k
 // rows 556 -> 510.
@@ -1080,9 +1083,14 @@ int dense_plan(int64_t rows, int32_t hidden, int32_t inter) {
 // the work of one expert with all of them that the dense waves are good for: even
 // routing | all rows on one expert, waves against tiles, 768 rows of 64 experts,
 // 2560 x 1536: 262 | 70 against 260 | 53; 1536 rows of 128, 2560 x 1536: 543 | 124
-// against 502 | 62; 3072 rows of 1024, 1024 x 256: 280 | 49 against 302 | 40.
-int grouped_plan(int64_t max_rows, int32_t n_experts, int32_t hidden, int32_t inter) {
-  return max_rows <= 12 * (int64_t)n_experts && (double)max_rows * hidden * inter <= 3.1e9 ? kPlanWave : kPlanTile;
+// against 502 | 62; 3072 rows of 1024, 1024 x 256: 271 | 49 against 302 | 40.  Plain
+// weights, which a wave reads in rows of 64 bytes, up to half of that: 512 rows of
+// 128, 2048 x 768: 233 | 37 (on eight) against 248 | 50; 1536 rows: 281 | 77 against
+// 262 | 53; 512 rows of 64, 2560 x 1536: 351 | 81 against 317 | 68.
+int grouped_plan(int64_t max_rows, int32_t n_experts, int32_t hidden, int32_t inter, bool packed) {
+  return max_rows <= 12 * (int64_t)n_experts && (double)max_rows * hidden * inter <= (packed ? 3.1e9 : 1.6e9)
+             ? kPlanWave
+             : kPlanTile;
 }
 
 // The two GEMMs of the MLP over the rows the tile source names; `addend`
@@ -1247,7 +1255,7 @@ int grouped_swiglu_impl(int32_t dtype, const void *x, int64_t ld_x, int32_t hidd
   const int64_t t_max = tm_group_slots_tiles(max_rows, n_experts);
   const TileSrc ts{tiles, expert_offsets, t_max, (int32_t)max_rows};
   return swiglu_impl(dtype, x, ld_x, row_token, hidden, inter, w1, w3, w2, ts, max_rows < t_max ? max_rows : t_max,
-                     out, 0, row_out, workspace, nullptr, 0, packed, grouped_plan(max_rows, n_experts, hidden, inter),
+                     out, 0, row_out, workspace, nullptr, 0, packed, grouped_plan(max_rows, n_experts, hidden, inter, packed),
                      tm_hip_stream(stream));  // (a tile holds at least one row)
 }
 
