@@ -451,6 +451,47 @@ def test_grouped_few_rows_on_average_uneven(hip_device, n, k, e, h, inter, how, 
             assert torch.equal(y, slot[b.to(dev), s.to(dev)]), ex
 
 
+def test_grouped_one_expert_cost(hip_device):
+    """1536 rows that all meet on one of 128 experts take less than twice the
+    dense call of that expert (with its grouping launches; 3 times as long when
+    one workgroup took all rows of a tile)."""
+    from table_moe.ops import GroupedExperts, SharedExperts
+
+    dev = hip_device
+    g = torch.Generator().manual_seed(6)
+    n, e, h, inter = 1536, 128, 2048, 768
+    x = torch.randn(n, h, generator=g).to(torch.bfloat16).to(dev)
+    w1, w3 = (torch.randn(e, inter, h, device=dev, dtype=torch.bfloat16) * 0.02 for _ in range(2))
+    w2 = torch.randn(e, h, inter, device=dev, dtype=torch.bfloat16) * 0.02
+    ge, one = GroupedExperts(w1, w3, w2), SharedExperts(w1[7], w3[7], w2[7])
+    ids = torch.full((n, 1), 7, dtype=torch.long, device=dev)
+    mask = torch.ones(n, 1, dtype=torch.bool, device=dev)
+    slot = torch.empty(n, 1, h, dtype=torch.bfloat16, device=dev)
+
+    def us(call):
+        call()
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            for _ in range(10):
+                call()
+        graph.replay()
+        torch.cuda.synchronize()
+        times = []
+        for _ in range(9):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            graph.replay()
+            b.record()
+            torch.cuda.synchronize()
+            times.append(a.elapsed_time(b) * 100)
+        return sorted(times)[4]
+
+    dense = us(lambda: one.forward(x))
+    assert us(lambda: ge.forward(x, ids, mask, slot)) < 2 * dense
+    assert torch.equal(slot.view(n, h), one.forward(x))
+
+
 @pytest.mark.parametrize("rows,h,inter", [(65536, 128, 128), (16384, 512, 256)])
 def test_dense_many_rows_small_weights_cost(hip_device, rows, h, inter):
     """A dense call takes about as long as the grouped GEMMs of one expert with

@@ -644,7 +644,8 @@ def test_keep_select_clusters_cost(hip_device, how):
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_search_topk_blocks_exact(hip_device, n, c, dim, top_k, metric, dtype):
     """The top-k of more than 64 queries (nearest blocks, then their
-    centroids) on small integers, whose distances are exact in fp32, so the
+    centroids; lists of centroids at d = 256 here) on small integers, whose
+    distances are exact in fp32, so the
     indices must be the lexicographic top-k: many equal distances (inside a
     block, across blocks and ranges), tables that end inside a block, fewer
     centroids than top_k (index -1, worst distance)."""
@@ -683,6 +684,14 @@ def test_search_topk_centroids_exact(hip_device, n, c, dim, top_k, metric, dtype
     """The shapes of test_search_topk_blocks_exact whose lists hold centroids
     (small tables): the same lexicographic top-k."""
     test_search_topk_blocks_exact(hip_device, n, c, dim, top_k, metric, dtype)
+
+
+@pytest.mark.parametrize("n,c,dim,top_k,metric", [(5121, 1408, 64, 8, "l2"), (1025, 3300, 128, 4, "dot"),
+                                                  (2049, 3072, 128, 8, "l2"), (70, 16411, 256, 4, "l2"),
+                                                  (300, 12001, 256, 8, "dot")])
+def test_search_topk_blocks_from_the_line_on(hip_device, n, c, dim, top_k, metric):
+    """Lists of blocks at the smallest tables that take them, and at d = 256."""
+    test_search_topk_blocks_exact(hip_device, n, c, dim, top_k, metric, torch.bfloat16)
 
 
 @pytest.mark.parametrize("n,c,dim,top_k", [(100, 300, 64, 4), (70, 4096, 128, 8), (1100, 300, 128, 8),
