@@ -215,16 +215,21 @@ __global__ __launch_bounds__(64) void skinny_gemm_kernel(
     if (blk >= slots) {
       int u = (int)(blk - slots);  // this is further row block u
       if (u >= (ts.tiles[0] - nt) / Cfg::RBMAX) return;  // uniform: more than the rows can have past their tiles' first
-      const int32_t *const row0 = ts.tiles + 2 + ts.t_max;  // tiles' rows follow each other
       for (int64_t t0 = 0;; t0 += 256) {  // four tiles per lane
         if (t0 >= nt) return;  // uniform: there are fewer
         const int64_t t = t0 + 4 * lane;
-        int at[5], more[4], sum = 0;
-#pragma unroll
-        for (int j = 0; j < 5; ++j) at[j] = row0[t + j < nt ? t + j : nt - 1];
+        int ex[4], at[4], more[4], sum = 0;
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-          more[j] = t + j < nt ? ((t + j + 1 < nt ? at[j + 1] : ts.tiles[0]) - at[j] - 1) / Cfg::RBMAX : 0;
+          const int64_t tj = t + j < nt ? t + j : nt - 1;
+          ex[j] = ts.tiles[2 + tj];
+          at[j] = ts.tiles[2 + ts.t_max + tj];
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j) ex[j] = ts.expert_offsets[ex[j] + 1] - at[j];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          more[j] = t + j < nt ? ((ex[j] < BM ? ex[j] : BM) - 1) / Cfg::RBMAX : 0;
           sum += more[j];
         }
         const int upto = (int)tm_wave_incl_scan((uint32_t)sum);
@@ -1083,7 +1088,7 @@ int dense_plan(int64_t rows, int32_t hidden, int32_t inter) {
 // the work of one expert with all of them that the dense waves are good for: even
 // routing | all rows on one expert, waves against tiles, 768 rows of 64 experts,
 // 2560 x 1536: 262 | 70 against 260 | 53; 1536 rows of 128, 2560 x 1536: 543 | 124
-// against 502 | 62; 3072 rows of 1024, 1024 x 256: 271 | 49 against 302 | 40.  Plain
+// against 502 | 62; 3072 rows of 1024, 1024 x 256: 275 | 50 against 302 | 40.  Plain
 // weights, which a wave reads in rows of 64 bytes, up to half of that: 512 rows of
 // 128, 2048 x 768: 233 | 37 (on eight) against 248 | 50; 1536 rows: 281 | 77 against
 // 262 | 53; 512 rows of 64, 2560 x 1536: 351 | 81 against 317 | 68.
